@@ -86,7 +86,8 @@ def build_hip_lib(jobs: int = 8) -> str:
 
 def build_oracle(with_reference: bool | None = None) -> str:
     if with_reference is None:
-        with_reference = os.path.isdir(REFERENCE_DIR)
+        # an empty mount point holds no sources to build from
+        with_reference = os.path.isdir(os.path.join(REFERENCE_DIR, "codes"))
     targets = ["all"] + (["ref"] if with_reference else [])
     _run(["make", "-s", "-j8", "-C", ORACLE_DIR, *targets])
     return ORACLE_LIB
