@@ -36,4 +36,5 @@ def gpu():
 
 
 def reference_present():
-    return os.path.isdir(REFERENCE_DIR)
+    # an empty mount point is no reference tree
+    return os.path.isdir(os.path.join(REFERENCE_DIR, "include"))
