@@ -291,16 +291,35 @@ constexpr int kAlpha = 14;
 constexpr int kBeta = 24;
 constexpr long long kQueueEdges = 1 << 16;
 
-__global__ void __launch_bounds__(kBlock) bfs_do_init(int src, const int* __restrict__ nindex, int m,
-                                                       Entry* __restrict__ q0, unsigned* __restrict__ bm, int words,
-                                                       Ctl* ctl)
+// Narrow levels.  A level costs two dependent launches, about 12 us on this
+// chip however few vertices it has, and a mesh has thousands of levels of a
+// few hundred.  So the workgroup that ends a level goes on by itself while the
+// frontier has at most kNarrowEdges edges: the frontier's edges are a list in
+// LDS (no owner search), a level is one pass over it by 1024 threads, and
+// nothing is written to memory but the levels themselves.  What bounds such a
+// level is the chain nlist -> dist -> compare-and-swap -> nindex, about 4 us
+// (grid 512 x 512 without long edges: 1018 levels in 3.9 ms).  At 4096 edges
+// it takes about as long as the two launches (a limit of 8192 measured the
+// same), since one CU takes in about one cache line a cycle.  A launch ends
+// after kNarrowLevels levels, so that the host can look at its time limit.
+// Levels from a queue above the limit run on few workgroups, one per
+// kLevelEdges edges.  Grid 1024 x 1024, whole run: 21.3 -> 11.0 ms.
+constexpr int kNarrowEdges = 4096;
+constexpr int kNarrowLevels = 512;
+constexpr long long kLevelEdges = 256;  // frontier edges per workgroup of a level from a queue
+constexpr int kNarrowShift = 21;  // a wave's edges, cut off: 256 * (kNarrowEdges + 1) < 2^21; its vertices above
+typedef int NarrowRow __attribute__((ext_vector_type(2), aligned(4)));  // a row's two offsets in one load
+
+// Clears the control block and prepares the run: dist, bitmaps 0 and 1 (2 is
+// cleared during level 0) with src in 0, and src's chunks in queue segment 0.
+__global__ void __launch_bounds__(kBlock) bfs_do_init(int src, const int* __restrict__ nindex, int n, int m,
+                                                       int* __restrict__ dist, Entry* __restrict__ q0,
+                                                       unsigned* __restrict__ bm, int words, Ctl* ctl)
 {
-  // bitmaps 0 and 1 start empty (2 is cleared during level 0); src is in 0;
-  // src's chunks go to queue segment 0
   const int stride = gridDim.x * kBlock;
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < 2 * words; i += stride) {
-    bm[i] = (i == (src >> 5)) ? (1u << (src & 31)) : 0u;
-  }
+  const int t = blockIdx.x * kBlock + threadIdx.x;
+  for (int v = t; v < n; v += stride) dist[v] = (v == src) ? 0 : kInf;
+  for (int i = t; i < 2 * words; i += stride) bm[i] = (i == (src >> 5)) ? (1u << (src & 31)) : 0u;
   if (blockIdx.x != 0) return;
   const int beg = nindex[src], end = nindex[src + 1];
   const int c = chunks_of(end - beg);
@@ -308,13 +327,18 @@ __global__ void __launch_bounds__(kBlock) bfs_do_init(int src, const int* __rest
     const int b = beg + k * kChunk;
     q0[k] = Entry{src, b, (b + kChunk < end) ? b + kChunk : end, 0};
   }
+  if ((int)threadIdx.x < kGroups) {
+    GroupSlot* gs = ctl_groups(ctl) + threadIdx.x;
+    gs->qcount[0] = (threadIdx.x == 0) ? c : 0;
+    gs->qcount[1] = 0;
+    gs->tiles = 0;
+  }
   if (threadIdx.x == 0) {
-    ctl_groups(ctl)[0].qcount[0] = c;
-    ctl->mode = 0;
-    ctl->level = 0;
-    ctl->in_bits = 0;
-    ctl->edges_next = end - beg;  // edges of the current frontier
-    ctl->edges_unvisited = (long long)m - (end - beg);
+    Ctl z = {};
+    z.n = n;
+    z.edges_next = end - beg;  // edges of the current frontier
+    z.edges_unvisited = (long long)m - (end - beg);
+    *ctl = z;
   }
 }
 
@@ -334,6 +358,9 @@ __global__ void __launch_bounds__(kBlock) bfs_do_level(const int* __restrict__ n
   __shared__ Entry s_ent[kWavesPerBlock][kWave];
   __shared__ long long s_red[kWavesPerBlock * kStats];
   if (round_done(ctl)) return;
+  // a level from a small queue runs on the first `active` workgroups only
+  const int active = (ctl->active > 0) ? ctl->active : (int)gridDim.x;
+  if ((int)blockIdx.x >= active) return;
   const int level = ctl->level;
   const int mode = ctl->mode;
   const int in_b = ctl->in_bits;
@@ -343,16 +370,17 @@ __global__ void __launch_bounds__(kBlock) bfs_do_level(const int* __restrict__ n
   const SegQ q_out = p ? q0 : q1;
   Entry* q_mine = segq_mine(q_out);
   int* out_count = segq_counter(ctl, p ^ 1, my_group());
-  const unsigned* cur = bm + (size_t)(level % 3) * words;
-  unsigned* next = bm + (size_t)((level + 1) % 3) * words;
-  unsigned* stale = bm + (size_t)((level + 2) % 3) * words;
+  const int turn = level + ctl->bm_phase;
+  const unsigned* cur = bm + (size_t)(turn % 3) * words;
+  unsigned* next = bm + (size_t)((turn + 1) % 3) * words;
+  unsigned* stale = bm + (size_t)((turn + 2) % 3) * words;
   const int nd = level + 1;
   const int w = threadIdx.x / kWave;
   const int lane = lane_id();
   const int gw = blockIdx.x * kWavesPerBlock + w;
-  const int nwaves = gridDim.x * kWavesPerBlock;
+  const int nwaves = active * kWavesPerBlock;
   {
-    const int stride = gridDim.x * kBlock;
+    const int stride = active * kBlock;
     for (int i = blockIdx.x * kBlock + threadIdx.x; i < words; i += stride) stale[i] = 0u;
   }
   long long found_v = 0, found_e = 0;
@@ -491,8 +519,8 @@ __global__ void __launch_bounds__(kBlock) bfs_do_level(const int* __restrict__ n
   round_partials(ctl, found_v, found_e, 0, 0, s_red);
 }
 
-// Level decision (run by round_finalize after each bfs_do_level): totals s[0]
-// = vertices found, s[1] = their edges.
+// Level decision (thread 0 of bfs_do_finish after each bfs_do_level): totals
+// s[0] = vertices found, s[1] = their edges.
 struct FinBfsDo {
   __device__ void operator()(Ctl* ctl, const RoundTotals& t) const
   {
@@ -516,6 +544,171 @@ struct FinBfsDo {
     ctl->iter += 1;
   }
 };
+
+// Ends a level (after_level; the first launch of a run has none to end) and
+// runs the narrow levels that follow it, see kNarrowEdges.  One workgroup.
+//
+// The frontier comes from the queue and, when the narrow levels end with one
+// left, goes back to it (segment 0) and to its bitmap, in the state that
+// bfs_do_level expects.  In between the bitmaps are not kept: the entry
+// frontier's bits are cleared, which leaves the bitmap of the frontier before
+// it the only one with bits, and bm_phase is set so that at the end this one
+// is the stale bitmap again.
+__global__ void __launch_bounds__(kFinBlock) bfs_do_finish(const int* __restrict__ nindex,
+                                                            const int* __restrict__ nlist, int* __restrict__ dist,
+                                                            SegQ q0, SegQ q1, unsigned* __restrict__ bm, int words,
+                                                            int nparts, bool after_level, Ctl* ctl)
+{
+  __shared__ int s_edge[2][kNarrowEdges];  // edges of the current and of the next frontier
+  __shared__ int s_vert[kNarrowEdges];     // vertices of the next frontier (at most one per edge walked)
+  __shared__ unsigned long long s_found;   // vertices (high half) and edges of the next frontier
+  __shared__ int s_edges, s_over, s_chunks;
+  __shared__ int s_go;
+  if (round_done(ctl)) return;
+  const int tid = threadIdx.x;
+  if (after_level) {
+    const RoundTotals tot = round_totals(ctl, nparts, 0x3);
+    if (tid == 0) FinBfsDo{}(ctl, tot);
+  }
+  // workgroups of the next level: a queue level takes one per kLevelEdges edges, at least 64
+  auto set_active = [&]() {
+    const long long want = (ctl->edges_next + kLevelEdges - 1) / kLevelEdges;
+    const bool few = ctl->mode == 0 && ctl->in_bits == 0 && want < nparts;
+    ctl->active = few ? (int)max(want, 64LL) : 0;
+  };
+  if (tid == 0) {
+    s_go = !ctl->done && ctl->in_bits == 0 && ctl->edges_next <= kNarrowEdges;
+    s_edges = 0;
+    s_chunks = 0;
+    if (!s_go) set_active();
+  }
+  __syncthreads();
+  if (!s_go) return;
+  const int level0 = ctl->level;
+  const int phase0 = ctl->bm_phase;
+  long long unvisited = ctl->edges_unvisited;
+  {
+    const int p = level0 & 1;
+    const SegQ q_in = p ? q1 : q0;
+    unsigned* cur = bm + (size_t)((level0 + phase0) % 3) * words;
+    const SegPrefix pre = segq_prefix(ctl, p);
+    for (int i = tid; i < pre.pre[kGroups]; i += kFinBlock) {
+      const Entry en = segq_at(q_in, pre, i);
+      cur[en.v >> 5] = 0u;
+      const int len = en.end - en.beg;
+      const int at = atomicAdd(&s_edges, len);
+      for (int k = 0; k < len; k++) s_edge[0][at + k] = en.beg + k;
+    }
+  }
+  int level = level0;
+  int count = 0;
+  int found = 1;
+  __syncthreads();
+  count = s_edges;
+  __syncthreads();
+  if (tid < kGroups) ctl_groups(ctl)[tid].qcount[level0 & 1] = 0;
+  for (;;) {  // uniform
+    if (tid == 0) {
+      s_found = 0;
+      s_over = 0;
+    }
+    __syncthreads();
+    const int* in = s_edge[(level - level0) & 1];
+    int* out = s_edge[((level - level0) & 1) ^ 1];
+    const int nd = level + 1;
+    constexpr int kPer = kNarrowEdges / kFinBlock;
+    int u[kPer], d[kPer];
+    #pragma unroll
+    for (int k = 0; k < kPer; k++) {
+      const int i = k * kFinBlock + tid;
+      u[k] = (i < count) ? nlist[in[i]] : -1;
+    }
+    #pragma unroll
+    for (int k = 0; k < kPer; k++) d[k] = (u[k] >= 0) ? dist[u[k]] : 0;
+    bool won[kPer];
+    #pragma unroll
+    for (int k = 0; k < kPer; k++) {
+      won[k] = false;
+      if (d[k] == kInf) {
+        int expected = kInf;
+        won[k] = __hip_atomic_compare_exchange_strong(&dist[u[k]], &expected, nd, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    // the rows of the winners only: one CU takes in about one cache line a
+    // cycle, and with thousands of scattered edges that rate is the level's time
+    NarrowRow row[kPer];
+    #pragma unroll
+    for (int k = 0; k < kPer; k++) row[k] = won[k] ? *(const NarrowRow*)(nindex + u[k]) : NarrowRow{0, 0};
+    // places for the thread's winners and their edges: one scan and one LDS
+    // atomic per wave, of (winners, edges) in one number; lengths enter it cut
+    // off just above kNarrowEdges, what is cut goes to s_over
+    unsigned mine = 0;
+    #pragma unroll
+    for (int k = 0; k < kPer; k++) {
+      const int len = row[k][1] - row[k][0];
+      if (won[k]) mine += (1u << kNarrowShift) + (unsigned)min(len, kNarrowEdges + 1);
+      if (len > kNarrowEdges + 1) atomicAdd(&s_over, len - (kNarrowEdges + 1));
+    }
+    if (ballot(mine != 0) != 0) {
+      const unsigned incl = (unsigned)wave_incl_scan((int)mine);
+      unsigned long long base = 0;
+      if (lane_id() == kWave - 1) {
+        base = atomicAdd(&s_found, ((unsigned long long)(incl >> kNarrowShift) << 32) |
+                                       (incl & ((1u << kNarrowShift) - 1u)));
+      }
+      base = __shfl(base, kWave - 1, kWave);
+      const unsigned excl = incl - mine;
+      int vat = (int)(base >> 32) + (int)(excl >> kNarrowShift);
+      int eat = (int)(base & 0xffffffffull) + (int)(excl & ((1u << kNarrowShift) - 1u));
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) {
+        if (!won[k]) continue;
+        s_vert[vat++] = u[k];
+        const int len = min(row[k][1] - row[k][0], kNarrowEdges + 1);
+        if (eat <= kNarrowEdges - len) {  // else the frontier is not narrow: the list is not used
+          for (int j = 0; j < len; j++) out[eat + j] = row[k][0] + j;
+        }
+        eat += len;
+      }
+    }
+    __syncthreads();
+    count = (int)(s_found & 0xffffffffull) + s_over;
+    found = (int)(s_found >> 32);
+    __syncthreads();
+    level++;
+    unvisited -= count;
+    if (found == 0 || count > kNarrowEdges || level - level0 >= kNarrowLevels) break;
+  }
+  if (found != 0) {
+    const int p = level & 1;
+    const SegQ q = p ? q1 : q0;
+    unsigned* cur = bm + (size_t)((level0 + phase0) % 3) * words;  // empty since the entry
+    for (int i = tid; i < found; i += kFinBlock) {
+      const int v = s_vert[i];
+      const int vb = nindex[v], ve = nindex[v + 1];
+      atomicOr(&cur[v >> 5], 1u << (v & 31));
+      const int c = chunks_of(ve - vb);
+      const int at = atomicAdd(&s_chunks, c);
+      for (int k = 0; k < c; k++) {
+        const int x = vb + k * kChunk;
+        q.base[at + k] = Entry{v, x, (x + kChunk < ve) ? x + kChunk : ve, 0};
+      }
+    }
+  }
+  __syncthreads();
+  if (tid == 0) {
+    ctl->iter += level - level0;
+    ctl->level = level;
+    ctl->bm_phase = (phase0 + 2 * (level - level0)) % 3;  // level + bm_phase stays the same modulo 3
+    ctl->edges_unvisited = unvisited;
+    ctl->edges_next = count;
+    ctl->done = (found == 0) ? 1 : 0;
+    ctl->mode = (count > kNarrowEdges && count > unvisited / kAlpha) ? 1 : 0;
+    ctl_groups(ctl)[0].qcount[level & 1] = s_chunks;
+    set_active();
+  }
+}
 
 // ------------------------------------------------------------ host side ----
 struct Bufs {
@@ -670,11 +863,14 @@ int style_do_hybrid(const igx_graph* g, int src, void* out, const void*, igx_run
   IGX_TRY(ws_get(WS_H, sizeof(int) * 64, &pc));
   const SegQ q0{(Entry*)p0, cap}, q1{(Entry*)p1, cap};
   IGX_TRY(timer_start());
-  IGX_TRY(ctl_reset(g->nodes));
+  hipLaunchKernelGGL(bfs_do_init, dim3(blocks_for(g->nodes, kBlock)), dim3(kBlock), 0, R.stream, src, g->nindex,
+                     g->nodes, g->edges, dist, (Entry*)p0, (unsigned*)pb, words, R.d_ctl);
   IGX_TRY(big_rows(g, pq, (int*)pc));
-  hipLaunchKernelGGL(bfs_init, dim3(blocks_for(g->nodes, kBlock)), dim3(kBlock), 0, R.stream, src, dist, g->nodes);
-  hipLaunchKernelGGL(bfs_do_init, dim3(blocks_for(2 * (long long)words, kBlock)), dim3(kBlock), 0, R.stream, src,
-                     g->nindex, g->edges, (Entry*)p0, (unsigned*)pb, words, R.d_ctl);
+  auto finish = [&](bool after_level) {
+    hipLaunchKernelGGL(bfs_do_finish, dim3(1), dim3(kFinBlock), 0, R.stream, g->nindex, g->nlist, dist, q0, q1,
+                       (unsigned*)pb, words, R.persist_blocks, after_level, R.d_ctl);
+  };
+  finish(false);
   int rounds = 0, launches = 0;
   const int rc = run_rounds(
       [&](long long) {
@@ -682,9 +878,9 @@ int style_do_hybrid(const igx_graph* g, int src, void* out, const void*, igx_run
         hipLaunchKernelGGL(bfs_do_level, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, g->nlist,
                            g->nodes, dist, q0, q1, (const Entry*)pq, (const int*)pc, (unsigned*)pb, words, R.d_ctl);
         ktimer_end("bfs_do_level");
-        launch_finalize(R.persist_blocks, 0x3, FinBfsDo{});
+        finish(true);
       },
-      (long long)g->nodes + 2, &rounds, &launches, 8);
+      (long long)g->nodes + 2, &rounds, &launches, 6);
   IGX_TRY(timer_stop(&info->seconds));
   info->iterations = rounds;
   info->launches = launches;

@@ -183,6 +183,7 @@ struct Ctl {
   int push_cut;          // SSSP: a push round relaxes only frontier vertices below this distance (0: all)
   int seeded;            // SSSP: the run has had its partial push round
   int force_all;         // SSSP: the next pull reads every neighbour (set after the partial push round)
+  int bm_phase;          // BFS: the current frontier's bitmap is (level + bm_phase) % 3
   int active;            // workgroups that take part in the next round (0: all); round_finalize reduces that many
 };
 
@@ -320,21 +321,18 @@ struct RoundTotals {
 
 constexpr int kFinBlock = 1024;  // 16 waves: two partials per thread for a 2048-block round
 
-// Finalize kernel (one workgroup of kFinBlock threads): reduces the partials
-// of the nparts blocks of the round kernel for the statistics in `stat_mask`
-// (bit k: integer k, summed, or the minimum for kStatMin; bit kStats + j:
-// FP64 j, summed), then runs fin(ctl, totals) on one thread.  All statistics
-// are reduced in one pass: every thread loads its strided partials of each
-// (independent loads), the waves reduce by shuffles and thread 0 adds the
-// waves in order, so FP64 totals are the same on every run.  Does nothing once
-// the run is done.
-template <typename Fin>
-__global__ void __launch_bounds__(kFinBlock) round_finalize(Ctl* ctl, int nparts, int stat_mask, Fin fin)
+// Totals of the round kernel's partials (one workgroup of kFinBlock threads,
+// all call): reduces the partials of its nparts blocks for the statistics in
+// `stat_mask` (bit k: integer k, summed, or the minimum for kStatMin; bit
+// kStats + j: FP64 j, summed).  All statistics are reduced in one pass: every
+// thread loads its strided partials of each (independent loads), the waves
+// reduce by shuffles and thread 0 adds the waves in order, so FP64 totals are
+// the same on every run.  The result holds on thread 0.
+__device__ __forceinline__ RoundTotals round_totals(Ctl* ctl, int nparts, int stat_mask)
 {
   constexpr int kFinWaves = kFinBlock / kWave;
   __shared__ long long s_l[kFinWaves][kStats];
   __shared__ double s_d[kFinWaves][kStatsD];
-  if (round_done(ctl)) return;
   long long acc[kStats];
   double accd[kStatsD];
   #pragma unroll
@@ -377,8 +375,8 @@ __global__ void __launch_bounds__(kFinBlock) round_finalize(Ctl* ctl, int nparts
     if (lane_id() == 0) s_d[w][k] = x;
   }
   __syncthreads();
+  RoundTotals tot = {};
   if (threadIdx.x == 0) {
-    RoundTotals tot;
     for (int k = 0; k < kStats; k++) {
       long long t = (k == kStatMin) ? LLONG_MAX : 0;
       for (int i = 0; i < kFinWaves; i++) t = (k == kStatMin) ? min(t, s_l[i][k]) : t + s_l[i][k];
@@ -389,8 +387,18 @@ __global__ void __launch_bounds__(kFinBlock) round_finalize(Ctl* ctl, int nparts
       for (int i = 0; i < kFinWaves; i++) t += s_d[i][k];
       tot.d[k] = ((stat_mask >> (kStats + k)) & 1) ? t : 0.0;
     }
-    fin(ctl, tot);
   }
+  return tot;
+}
+
+// Finalize kernel (one workgroup of kFinBlock threads): runs fin(ctl, totals)
+// on one thread.  Does nothing once the run is done.
+template <typename Fin>
+__global__ void __launch_bounds__(kFinBlock) round_finalize(Ctl* ctl, int nparts, int stat_mask, Fin fin)
+{
+  if (round_done(ctl)) return;
+  const RoundTotals tot = round_totals(ctl, nparts, stat_mask);
+  if (threadIdx.x == 0) fin(ctl, tot);
 }
 
 
