@@ -567,7 +567,7 @@ __global__ void __launch_bounds__(kFinBlock) bfs_do_finish(const int* __restrict
   if (round_done(ctl)) return;
   const int tid = threadIdx.x;
   if (after_level) {
-    const RoundTotals tot = round_totals(ctl, nparts, 0x3);
+    const RoundTotals tot = round_totals<0x3>(ctl, nparts);
     if (tid == 0) FinBfsDo{}(ctl, tot);
   }
   // workgroups of the next level: a queue level takes one per kLevelEdges edges, at least 64

@@ -702,7 +702,6 @@ int style_uf(const igx_graph* g, int, void* out, const void*, igx_run_info* info
   IGX_TRY(ws_get(WS_E, sizeof(int) * 64, &pc));
   const int grid = R.persist_blocks;
   IGX_TRY(timer_start());
-  hipLaunchKernelGGL(cc_fill, dim3(1), dim3(kBlock), 0, R.stream, (int*)pc, 0, 1LL);
   hipLaunchKernelGGL(uf_init, dim3(blocks_for(g->nodes, kBlock)), dim3(kBlock), 0, R.stream, g->nindex, g->nlist,
                      g->nodes, parent);
   IGX_TRY(big_rows(g, pq, (int*)pc));
@@ -714,7 +713,7 @@ int style_uf(const igx_graph* g, int, void* out, const void*, igx_run_info* info
   IGX_HIP(hipGetLastError());
   IGX_TRY(timer_stop(&info->seconds));
   info->iterations = 1;
-  info->launches = 5;
+  info->launches = 4;
   return IGX_OK;
 }
 
@@ -730,7 +729,6 @@ int style_afforest(const igx_graph* g, int, void* out, const void*, igx_run_info
   int* counters = (int*)pc;  // [0] big chunk count, [1] sampled giant root
   const int grid = R.persist_blocks;
   IGX_TRY(timer_start());
-  hipLaunchKernelGGL(cc_fill, dim3(1), dim3(kBlock), 0, R.stream, counters, 0, 2LL);
   hipLaunchKernelGGL(af_init, dim3(blocks_for(g->nodes, kBlock)), dim3(kBlock), 0, R.stream, g->nindex, g->nlist,
                      g->nodes, parent);
   IGX_TRY(big_rows(g, pq, counters));
@@ -745,7 +743,7 @@ int style_afforest(const igx_graph* g, int, void* out, const void*, igx_run_info
   IGX_HIP(hipGetLastError());
   IGX_TRY(timer_stop(&info->seconds));
   info->iterations = 1;
-  info->launches = 8;
+  info->launches = 7;
   return IGX_OK;
 }
 

@@ -103,11 +103,10 @@ int ctl_reset(int n);
 // kernel's per-block partials (round_finalize in igx_device.hpp).
 void launch_fin_flag();
 void launch_fin_worklist();
-template <typename Fin>
-inline void launch_finalize(int nparts, int stat_mask, Fin fin)
+template <int kMask, typename Fin>
+inline void launch_finalize(int nparts, Fin fin)
 {
-  hipLaunchKernelGGL((round_finalize<Fin>), dim3(1), dim3(kFinBlock), 0, rt().stream, rt().d_ctl, nparts, stat_mask,
-                     fin);
+  hipLaunchKernelGGL((round_finalize<kMask, Fin>), dim3(1), dim3(kFinBlock), 0, rt().stream, rt().d_ctl, nparts, fin);
 }
 
 // multiplier for spread_vertex: odd, coprime to n

@@ -426,7 +426,7 @@ int style_pull(const igx_graph* g, int, void* out, const void*, igx_run_info* in
         float* nxt = (r & 1) ? c0 : c1;
         hipLaunchKernelGGL((pr_pull<G>), dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, g->nlist,
                            g->nodes, base, score, cur, nxt, R.d_ctl, P.eps, P.max_iter);
-        launch_finalize(R.persist_blocks, 0x1, FinPr{P.eps, P.max_iter});
+        launch_finalize<0x1>(R.persist_blocks, FinPr{P.eps, P.max_iter});
       },
       P.max_iter, &rounds, &launches);
   IGX_TRY(timer_stop(&info->seconds));
@@ -471,7 +471,7 @@ int style_balanced(const igx_graph* g, int, void* out, const void*, igx_run_info
         ktimer_end("pr_bal_main");
         hipLaunchKernelGGL(pr_bal_big, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, base, score,
                            nxt, (const BigRow*)pbig, (const int*)pcnt, (const Pair*)ppart, R.d_ctl);
-        launch_finalize(R.persist_blocks, 0x3, FinPr{P.eps, P.max_iter});
+        launch_finalize<0x3>(R.persist_blocks, FinPr{P.eps, P.max_iter});
       },
       P.max_iter, &rounds, &launches);
   IGX_TRY(timer_stop(&info->seconds));
@@ -509,7 +509,7 @@ int style_push(const igx_graph* g, int, void* out, const void*, igx_run_info* in
         ktimer_end("pr_push");
         hipLaunchKernelGGL(pr_push_compute, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, n, base,
                            score, contrib, incoming, R.d_ctl);
-        launch_finalize(R.persist_blocks, 0x1, FinPr{P.eps, P.max_iter});
+        launch_finalize<0x1>(R.persist_blocks, FinPr{P.eps, P.max_iter});
       },
       P.max_iter, &rounds, &launches);
   IGX_TRY(timer_stop(&info->seconds));

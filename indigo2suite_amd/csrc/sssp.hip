@@ -482,13 +482,16 @@ constexpr int kSlice = 512;  // edges per streamed slice of a pull run
 
 enum { kStatFrontierEdges = 0, kStatScanned = 1, kStatRelaxed = 2, kStatRows = 3 };
 
-__global__ void __launch_bounds__(kBlock) sssp_do_init(int src, const int* __restrict__ nindex, Entry* __restrict__ q0,
+// Clears the control block and prepares the run: dist, bitmaps 0 and 1 with
+// src in 0, src's chunks in queue segment 0.
+__global__ void __launch_bounds__(kBlock) sssp_do_init(int src, const int* __restrict__ nindex, int n,
+                                                        int* __restrict__ dist, Entry* __restrict__ q0,
                                                         unsigned* __restrict__ bm, int words, Ctl* ctl)
 {
   const int stride = gridDim.x * kBlock;
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < 2 * words; i += stride) {
-    bm[i] = (i == (src >> 5)) ? (1u << (src & 31)) : 0u;
-  }
+  const int t = blockIdx.x * kBlock + threadIdx.x;
+  for (int v = t; v < n; v += stride) dist[v] = (v == src) ? 0 : kInf;
+  for (int i = t; i < 2 * words; i += stride) bm[i] = (i == (src >> 5)) ? (1u << (src & 31)) : 0u;
   if (blockIdx.x != 0) return;
   const int beg = nindex[src], end = nindex[src + 1];
   const int c = chunks_of(end - beg);
@@ -496,11 +499,17 @@ __global__ void __launch_bounds__(kBlock) sssp_do_init(int src, const int* __res
     const int b = beg + k * kChunk;
     q0[k] = Entry{src, b, (b + kChunk < end) ? b + kChunk : end, 0};
   }
+  if ((int)threadIdx.x < kGroups) {
+    GroupSlot* gs = ctl_groups(ctl) + threadIdx.x;
+    gs->qcount[0] = (threadIdx.x == 0) ? c : 0;
+    gs->qcount[1] = 0;
+    gs->tiles = 0;
+  }
   if (threadIdx.x == 0) {
-    ctl_groups(ctl)[0].qcount[0] = c;
-    ctl->mode = 0;
-    ctl->in_bits = 0;
-    ctl->edges_next = end - beg;  // edges of the current frontier
+    Ctl z = {};
+    z.n = n;
+    z.edges_next = end - beg;  // edges of the current frontier
+    *ctl = z;
   }
 }
 
@@ -1156,11 +1165,9 @@ int style_do(const igx_graph* g, int src, void* out, const void*, igx_run_info* 
   IGX_TRY(ws_get(WS_B, sizeof(int) * 64, &pc));
   const SegQ q0{(Entry*)p0, cap}, q1{(Entry*)p1, cap};
   IGX_TRY(timer_start());
-  IGX_TRY(ctl_reset(g->nodes));
-  hipLaunchKernelGGL(sssp_init, dim3(blocks_for(g->nodes, kBlock)), dim3(kBlock), 0, R.stream, src, dist, g->nodes);
+  hipLaunchKernelGGL(sssp_do_init, dim3(blocks_for(g->nodes, kBlock)), dim3(kBlock), 0, R.stream, src, g->nindex,
+                     g->nodes, dist, (Entry*)p0, (unsigned*)pm, words, R.d_ctl);
   IGX_TRY(big_rows(g, pb, (int*)pc));
-  hipLaunchKernelGGL(sssp_do_init, dim3(blocks_for(2 * (long long)words, kBlock)), dim3(kBlock), 0, R.stream, src,
-                     g->nindex, (Entry*)p0, (unsigned*)pm, words, R.d_ctl);
   int rounds = 0, launches = 0;
   const int rc = run_rounds(
       [&](long long) {
@@ -1169,7 +1176,7 @@ int style_do(const igx_graph* g, int src, void* out, const void*, igx_run_info* 
                            g->eweight, g->nodes, (long long)g->edges, dist, q0, q1, (const Entry*)pb,
                            (const int*)pc, (unsigned*)pm, words, grab, R.d_ctl);
         ktimer_end("sssp_do_round");
-        launch_finalize(R.persist_blocks, 0xF | (1 << kStatMin) | (3 << kStats),
+        launch_finalize<0xF | (1 << kStatMin) | (3 << kStats)>(R.persist_blocks,
                         FinSsspDo{(long long)g->edges, R.persist_blocks});
       },
       sssp_round_cap(g), &rounds, &launches, 8);
