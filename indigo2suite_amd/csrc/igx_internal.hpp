@@ -39,7 +39,8 @@ struct Runtime {
   hipStream_t stream = nullptr;
   hipEvent_t ev_start = nullptr, ev_stop = nullptr;
   Ctl* d_ctl = nullptr;        // device control block
-  Ctl* h_ctl = nullptr;        // pinned host mirror
+  Ctl* h_ctl = nullptr;        // pinned host mirror: the last control block read, then two slots for copies under way
+  hipEvent_t ev_batch[2] = {nullptr, nullptr};  // end of the copy to each slot
   int persist_blocks = 0;      // grid of persistent kernels
   double time_limit = 0.0;     // igx_set_time_limit: seconds per run, 0 = none
   std::chrono::steady_clock::time_point t_start;  // host clock at timer_start
@@ -55,43 +56,58 @@ enum WsSlot {
 };
 int ws_get(int slot, size_t bytes, void** ptr);
 
-// Enqueue round kernels in growing batches until the control block reports
-// done or max_rounds were enqueued.  `launch(r)` enqueues round r.  Batches:
-// first_batch, then 4, 8, 16, ... 64.  A round enqueued after convergence
-// returns at once on the device but still costs its host-side submission
-// (about 10 us, more than its device time), so the batch after the first
-// stays small: a run that needs a few rounds more than the first batch wastes
-// at most three submissions instead of a doubled batch.
+// Enqueue round kernels in batches until the control block reports done or
+// max_rounds were enqueued.  `launch(r)` enqueues round r.  A round enqueued
+// after convergence returns at once on the device (about 2 us a launch); a
+// wait for the device between two batches leaves it idle for about 20 us.  So
+// the first batch, which most runs that know their usual number of rounds end
+// in, is waited for alone, and after it one batch of kAheadRounds is always in
+// the stream behind the one that is waited for: at most two of them run empty,
+// where batches that doubled up to 64 cost PageRank up to 15 empty rounds of
+// three launches.  The batches grow slowly so that runs of thousands of
+// rounds wait seldom.
 // After each batch the run also stops, with IGX_ERR_TIMEOUT, once the host
 // clock since timer_start() passes the time limit set by igx_set_time_limit.
 // Returns IGX_OK, IGX_ERR_LIMIT when max_rounds did not converge, or an error.
+// From round first_batch on, R.h_ctl holds a control block of this run.
+constexpr int kAheadRounds = 4;
 bool past_time_limit();
+int batch_mark(int slot);    // copy the control block to slot's pinned mirror, behind the work so far
+int batch_wait(int slot);    // wait for it and make it *R.h_ctl
 template <typename F>
 int run_rounds(F launch, long long max_rounds, int* rounds_done, int* launches, int first_batch = 2)
 {
   Runtime& R = rt();
-  long long launched = 0;
-  int batch = first_batch;
-  while (true) {
+  long long launched = 0, batches = 0;
+  auto enqueue = [&](long long batch) -> int {
     const long long k = (launched + batch > max_rounds) ? (max_rounds - launched) : batch;
     for (long long i = 0; i < k; i++) {
       launch(launched + i);
     }
     IGX_HIP(hipGetLastError());
     launched += k;
-    IGX_HIP(hipMemcpyAsync(R.h_ctl, R.d_ctl, sizeof(Ctl), hipMemcpyDeviceToHost, R.stream));
-    IGX_HIP(hipStreamSynchronize(R.stream));
+    return batch_mark((int)(batches++ & 1));
+  };
+  IGX_TRY(enqueue(first_batch));
+  long long waited = 0;
+  int rc = IGX_OK;
+  while (true) {
+    IGX_TRY(batch_wait((int)(waited++ & 1)));
     if (R.h_ctl->done) break;
-    if (launched >= max_rounds || past_time_limit()) {
-      if (rounds_done) *rounds_done = R.h_ctl->iter;
-      if (launches) *launches = (int)launched;
-      return (launched >= max_rounds) ? IGX_ERR_LIMIT : IGX_ERR_TIMEOUT;
+    const bool stop = launched >= max_rounds || past_time_limit();
+    if (stop && waited == batches) {
+      rc = (launched >= max_rounds) ? IGX_ERR_LIMIT : IGX_ERR_TIMEOUT;
+      break;
     }
-    batch = (launched == k) ? 4 : ((batch < 64) ? batch * 2 : 64);
+    // two batches behind the first one, then one for each that came back
+    while (!stop && batches - waited < 2 && launched < max_rounds) {
+      const long long b = kAheadRounds + 2 * (batches / 8);
+      IGX_TRY(enqueue(b < 64 ? b : 64));
+    }
   }
   if (rounds_done) *rounds_done = R.h_ctl->iter;
   if (launches) *launches = (int)launched;
-  return IGX_OK;
+  return rc;
 }
 
 // Clear the control block on the stream (kernel, not a memset node).

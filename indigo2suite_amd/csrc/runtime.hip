@@ -373,6 +373,20 @@ void ktimer_end(const char* tag)
   g_prof_open = false;
 }
 
+int batch_mark(int slot)
+{
+  IGX_HIP(hipMemcpyAsync(g_rt.h_ctl + 1 + slot, g_rt.d_ctl, sizeof(Ctl), hipMemcpyDeviceToHost, g_rt.stream));
+  IGX_HIP(hipEventRecord(g_rt.ev_batch[slot], g_rt.stream));
+  return IGX_OK;
+}
+
+int batch_wait(int slot)
+{
+  IGX_HIP(hipEventSynchronize(g_rt.ev_batch[slot]));
+  *g_rt.h_ctl = g_rt.h_ctl[1 + slot];
+  return IGX_OK;
+}
+
 int timer_start()
 {
   IGX_HIP(hipEventRecord(g_rt.ev_start, g_rt.stream));
@@ -468,8 +482,9 @@ int igx_init(int device)
   IGX_HIP(hipEventCreate(&g_rt.ev_stop));
   IGX_HIP(hipMalloc((void**)&g_rt.d_ctl, kCtlAllocBytes));
   IGX_HIP(hipMemset(g_rt.d_ctl, 0, kCtlAllocBytes));
-  IGX_HIP(hipHostMalloc((void**)&g_rt.h_ctl, sizeof(Ctl), hipHostMallocDefault));
-  memset(g_rt.h_ctl, 0, sizeof(Ctl));
+  for (hipEvent_t& e : g_rt.ev_batch) IGX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  IGX_HIP(hipHostMalloc((void**)&g_rt.h_ctl, 3 * sizeof(Ctl), hipHostMallocDefault));
+  memset(g_rt.h_ctl, 0, 3 * sizeof(Ctl));
   IGX_TRY(batch_noalloc_setup(device));
   g_rt.ready = true;
   init_entry_styles();
@@ -522,6 +537,9 @@ int igx_shutdown(void)
   g_prof_tag[0] = 0;
   if (hipEventDestroy(g_rt.ev_start) != hipSuccess) rc = IGX_ERR_HIP;
   if (hipEventDestroy(g_rt.ev_stop) != hipSuccess) rc = IGX_ERR_HIP;
+  for (hipEvent_t e : g_rt.ev_batch) {
+    if (hipEventDestroy(e) != hipSuccess) rc = IGX_ERR_HIP;
+  }
   if (hipHostFree(g_rt.h_ctl) != hipSuccess) rc = IGX_ERR_HIP;
   if (hipFree(g_rt.d_ctl) != hipSuccess) rc = IGX_ERR_HIP;
   if (hipStreamDestroy(g_rt.stream) != hipSuccess) rc = IGX_ERR_HIP;
