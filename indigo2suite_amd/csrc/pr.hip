@@ -29,6 +29,8 @@
 // same kernel that produces the score, so one pass per iteration remains.
 #include "igx_internal.hpp"
 #include "igx_frontier.hpp"
+#include "igx_rank.hpp"
+#include "igx_scan.hpp"
 
 namespace igx {
 namespace {
@@ -102,13 +104,19 @@ __device__ __forceinline__ long long pr_finish(int v, Pair acc, float base, cons
 
 // End of an iteration (run by round_finalize): the L1 residual is the exact
 // integer sum of the per-block partials (slot 0: rows scored by the main
-// kernel, slot 1: rows merged from chunks), scaled back from 2^-50 units.
+// kernel, slot 1: rows merged from chunks, slot 2: rows of one chunk of a
+// renumbered graph), scaled back from 2^-50 units.  Also tells the host which
+// of the balanced style's kernels have work on this graph.
 struct FinPr {
   double eps;
   int max_iter;
+  const int* big_rows;
+  const int* relabel;
   __device__ void operator()(Ctl* ctl, const RoundTotals& t) const
   {
-    const double r = (double)(t.s[0] + t.s[1]) / kResScale;
+    ctl->aux_ll[0] = (big_rows != nullptr) ? *big_rows : 0;
+    ctl->aux_ll[1] = (relabel != nullptr) ? *relabel : 0;
+    const double r = (double)(t.s[0] + t.s[1] + t.s[2]) / kResScale;
     ctl->res_last = r;
     ctl->iter += 1;
     if (r < eps || ctl->iter >= max_iter) ctl->done = 1;
@@ -166,55 +174,236 @@ __global__ void __launch_bounds__(kBlock) pr_pull(const int* __restrict__ nindex
 // ------------------------------------------------------------- balanced ----
 // Row classes are built once per run: every row longer than kSmallRow is cut
 // into chunks of at most kChunk edges (its pieces in edge order, in a
-// contiguous run of chunk slots reserved with one atomic per wave).  A row of
-// one chunk is finished by the wave that sums it (Entry::pad = -1); the others
-// leave compensated partial sums that pr_bal_big merges in slot order, so the
-// result does not depend on the schedule.
+// contiguous run of chunk slots).  A row of one chunk is finished by the wave
+// that sums it (Entry::pad = -1); the others leave compensated partial sums
+// that pr_bal_big merges in a fixed order, so the result does not depend on
+// the schedule.
 struct BigRow {
   int v;
   int first;  // first chunk slot
   int count;  // number of chunks
 };
 
-__global__ void pr_zero(int* __restrict__ p, int count)
+// Degree order.  An iteration is bound by its gathers, one contribution per
+// edge.  On a graph with hubs most of them go to few vertices, which lie all
+// over the contribution array, so each costs a cache line of its own.  Where
+// the kHotRanks vertices of highest degree (a contribution each: 64 KB of LDS)
+// take at least a quarter of the edges, the run works on a copy of the graph
+// renumbered by degree rank, whose hot contributions lie side by side.  Rows keep their edges in the order they had, and their chunks, so
+// a row of one chunk sums the same values in the same order.  R-MAT 20: the
+// iterations without the hot values in LDS 190 -> 139 us, the copy 210 us per
+// run; whole run 3.37 -> 2.21 ms with the other changes.  Chung-Lu n = 1 M,
+// average degree 16: exponent 2.3 (35% hot) 2.04 -> 1.90 ms, exponent 2.7 1.71
+// -> 1.84 ms if it were copied (under the line).
+// On other graphs (a mesh, whose ids are local) the copy would cost its build
+// and lose what locality there is.
+constexpr int kHotRanks = 16384;
+constexpr int kRelabelMinNodes = 2 * kHotRanks;  // below, most of the array is close by anyway
+
+// The graph a run works on: as given, or renumbered when *relabel says so.
+struct PrSource {
+  const int* nindex[2];
+  const int* nlist[2];
+  float* score[2];
+  const int* relabel;  // nullptr: as given
+};
+struct PrGraph {
+  const int* nindex;
+  const int* nlist;
+  float* score;
+};
+__device__ __forceinline__ PrGraph pr_graph(const PrSource& s)
 {
-  for (int i = threadIdx.x; i < count; i += blockDim.x) p[i] = 0;
+  const int k = (s.relabel != nullptr && *s.relabel != 0) ? 1 : 0;
+  return PrGraph{k ? s.nindex[1] : s.nindex[0], k ? s.nlist[1] : s.nlist[0], k ? s.score[1] : s.score[0]};
 }
 
-// counts[1]: rows of several chunks (big); counts[2]: chunks
-__global__ void __launch_bounds__(kBlock) pr_classify(const int* __restrict__ nindex, int n,
-                                                       int* __restrict__ counts, Entry* __restrict__ chunks,
-                                                       BigRow* __restrict__ big)
+__global__ void __launch_bounds__(kBlock) pr_zero(int* __restrict__ p, int count)
 {
-  const int stride = gridDim.x * kBlock;
-  for (int base = blockIdx.x * kBlock; base < n; base += stride) {
-    const int v = base + threadIdx.x;
-    int deg = 0, beg = 0, end = 0;
-    if (v < n) {
-      beg = nindex[v];
-      end = nindex[v + 1];
-      deg = end - beg;
-    }
-    const int c = (deg > kSmallRow) ? chunks_of(deg) : 0;
-    const int first = wave_reserve(&counts[2], c);
-    const int bs = wave_push_slot(&counts[1], c > 1);
-    if (c > 1) big[bs] = BigRow{v, first, c};
-    for (int k = 0; k < c; k++) {
-      const int b = beg + k * kChunk;
-      chunks[first + k] = Entry{v, b, (b + kChunk < end) ? b + kChunk : end, (c == 1) ? -1 : 0};
+  for (int i = blockIdx.x * kBlock + threadIdx.x; i < count; i += gridDim.x * kBlock) p[i] = 0;
+}
+
+// the renumbered lists: edge (v, u) to the place it has in row rank[v]
+__global__ void __launch_bounds__(kBlock) pr_relabel(const int* __restrict__ nindex, const int* __restrict__ nlist, int n,
+                                                      int m, const int* __restrict__ rank,
+                                                      const int* __restrict__ tile_row,
+                                                      const int* __restrict__ nindex1, int* __restrict__ nlist1,
+                                                      const int* __restrict__ relabel)
+{
+  __shared__ __align__(16) int s_row[kEdgeTile];
+  __shared__ int s_red[kWavesPerBlock];
+  if (*relabel == 0) return;
+  const int tile = blockIdx.x;
+  const int base = tile * kEdgeTile;
+  const int r0 = tile_row[tile];
+  const int r1 = (tile + 1 < (int)gridDim.x) ? tile_row[tile + 1] : n - 1;
+  int u[kEdgePer], ru[kEdgePer];
+  #pragma unroll
+  for (int k = 0; k < kEdgePer; k++) {
+    const int i = k * kBlock + (int)threadIdx.x;
+    u[k] = (i < m - base) ? nlist[base + i] : -1;
+  }
+  #pragma unroll
+  for (int k = 0; k < kEdgePer; k++) ru[k] = (u[k] >= 0) ? rank[u[k]] : 0;
+  edge_tile_rows(nindex, base, r0, r1, s_row, s_red);
+  #pragma unroll
+  for (int k = 0; k < kEdgePer; k++) {
+    if (u[k] >= 0) {
+      const int i = k * kBlock + (int)threadIdx.x;
+      const int v = r0 + s_row[i];
+      nlist1[nindex1[rank[v]] + (base + i - nindex[v])] = ru[k];
     }
   }
 }
 
-// One iteration's sums: first the chunks (one wave each, kChunk / 64 loads per
-// lane issued together; chunks are at most kChunk edges, so a fixed
-// round-robin share balances), then the small rows in 64-row tiles, also
-// round robin.  Small rows:
-// consecutive small rows form runs whose edges are contiguous, streamed kSlice
-// at a time (independent loads, values parked in LDS); each lane then adds its
-// own row's values in edge order.
-__global__ void __launch_bounds__(kBlock) pr_bal_main(const int* __restrict__ nindex, const int* __restrict__ nlist,
-                                                       int n, float base, float* __restrict__ score,
+__global__ void __launch_bounds__(kBlock) pr_bal_init(PrSource src, int n, float* __restrict__ contrib)
+{
+  const PrGraph g = pr_graph(src);
+  const int v = blockIdx.x * kBlock + threadIdx.x;
+  if (v < n) {
+    const float s0 = 1.0f / (float)n;  // pr_cuda.h:133
+    g.score[v] = s0;
+    contrib[v] = s0 / (float)(g.nindex[v + 1] - g.nindex[v]);
+  }
+}
+
+// scores of a renumbered graph back in the caller's order
+__global__ void __launch_bounds__(kBlock) pr_scores_out(PrSource src, int n, const int* __restrict__ order)
+{
+  const int r = blockIdx.x * kBlock + threadIdx.x;
+  if (r < n) src.score[0][order[r]] = src.score[1][r];
+}
+
+// counts[1]: rows of several chunks (big); counts[2]: chunks.  kClassRows
+// consecutive rows per workgroup, which reserves their slots with one atomic
+// on each counter (one per wave had 170 us of them on R-MAT 20); the chunks
+// of a longer row are written by its wave together.
+constexpr int kClassPer = 2;
+constexpr int kClassRows = kClassPer * kBlock;
+__global__ void __launch_bounds__(kBlock) pr_classify(PrSource src, int n, int* __restrict__ counts,
+                                                       Entry* __restrict__ chunks, BigRow* __restrict__ big)
+{
+  __shared__ int s_red[kWavesPerBlock];
+  __shared__ int s_first, s_big;
+  const PrGraph g = pr_graph(src);
+  int beg[kClassPer], end[kClassPer], c[kClassPer];
+  int nc = 0, nb = 0;
+  #pragma unroll
+  for (int k = 0; k < kClassPer; k++) {
+    const long long v = (long long)blockIdx.x * kClassRows + k * kBlock + threadIdx.x;
+    beg[k] = (v < n) ? g.nindex[v] : 0;
+    end[k] = (v < n) ? g.nindex[v + 1] : 0;
+    c[k] = (end[k] - beg[k] > kSmallRow) ? chunks_of(end[k] - beg[k]) : 0;
+    nc += c[k];
+    nb += (c[k] > 1) ? 1 : 0;
+  }
+  int tc = 0, tb = 0;
+  int first = block_excl_scan(nc, s_red, &tc);
+  if (tc == 0) return;  // uniform
+  int bs = block_excl_scan(nb, s_red, &tb);
+  if (threadIdx.x == 0) {
+    s_first = atomicAdd(&counts[2], tc);
+    s_big = (tb > 0) ? atomicAdd(&counts[1], tb) : 0;
+  }
+  __syncthreads();
+  first += s_first;
+  bs += s_big;
+  #pragma unroll
+  for (int k = 0; k < kClassPer; k++) {
+    const int v = blockIdx.x * kClassRows + k * kBlock + (int)threadIdx.x;
+    if (c[k] == 1) chunks[first] = Entry{v, beg[k], end[k], -1};
+    if (c[k] > 1) big[bs++] = BigRow{v, first, c[k]};
+    for (uint64_t todo = ballot(c[k] > 1); todo != 0; todo &= todo - 1) {
+      const int L = __ffsll((unsigned long long)todo) - 1;
+      const int rb = __shfl(beg[k], L, kWave), re = __shfl(end[k], L, kWave), rc = __shfl(c[k], L, kWave);
+      const int rf = __shfl(first, L, kWave), rv = __shfl(v, L, kWave);
+      for (int j = lane_id(); j < rc; j += kWave) {
+        const int b = rb + j * kChunk;
+        chunks[rf + j] = Entry{rv, b, (b + kChunk < re) ? b + kChunk : re, 0};
+      }
+    }
+    first += c[k];
+  }
+}
+
+// One chunk's compensated sum by the wave, its values gathered by `value`
+// (kChunk / 64 loads per lane issued together); the row's score when the chunk
+// is the whole row.  Returns the residual term on lane 0.
+template <typename F>
+__device__ __forceinline__ long long pr_chunk(const Entry& en, int k, const PrGraph& g, float base,
+                                              float* __restrict__ contrib_next, Pair* __restrict__ partial, F value)
+{
+  constexpr int kPer = kChunk / kWave;
+  const int lane = lane_id();
+  int u[kPer];
+  #pragma unroll
+  for (int j = 0; j < kPer; j++) {
+    const int i = en.beg + j * kWave + lane;
+    u[j] = (i < en.end) ? g.nlist[i] : -1;
+  }
+  float x[kPer];
+  value(u, x);
+  Pair acc{0.0f, 0.0f};
+  #pragma unroll
+  for (int j = 0; j < kPer; j++) {
+    if (u[j] >= 0) two_sum_add(acc, x[j]);
+  }
+  acc = wave_merge(acc);
+  if (lane == 0) {
+    if (en.pad < 0) return pr_finish(en.v, acc, base, g.nindex, g.score, contrib_next);
+    partial[k] = acc;
+  }
+  return 0;
+}
+
+// The chunks of a renumbered graph, with the kHotRanks hot contributions in
+// LDS (64 KB, so two workgroups of 16 waves fill a CU).  A gather that misses
+// LDS moves a cache line from L2, which is what an iteration is bound by:
+// R-MAT 20 (57% of the edges hot): 128 -> 104 us an iteration together with
+// the small rows.
+constexpr int kHotBlock = 1024;
+__global__ void __launch_bounds__(kHotBlock) pr_hot_chunks(PrSource src, int n, float base,
+                                                            const float* __restrict__ contrib_cur,
+                                                            float* __restrict__ contrib_next,
+                                                            const int* __restrict__ counts,
+                                                            const Entry* __restrict__ chunks,
+                                                            Pair* __restrict__ partial, int nparts, Ctl* ctl)
+{
+  __shared__ float s_hot[kHotRanks];
+  __shared__ long long s_red[kHotBlock / kWave];
+  if (round_done(ctl)) return;
+  // partial slots past this grid (the round's other kernels have a wider one)
+  if (blockIdx.x == 0) {
+    for (int i = gridDim.x + threadIdx.x; i < nparts; i += kHotBlock) ctl_parts(ctl)[(size_t)2 * kMaxParts + i] = 0;
+  }
+  long long err = 0;
+  if (*src.relabel != 0) {  // uniform
+    const PrGraph g = pr_graph(src);
+    for (int i = threadIdx.x; i < kHotRanks && i < n; i += kHotBlock) s_hot[i] = contrib_cur[i];
+    __syncthreads();
+    const int nch = counts[2];
+    const int waves = gridDim.x * (kHotBlock / kWave);
+    for (int k = blockIdx.x * (kHotBlock / kWave) + threadIdx.x / kWave; k < nch; k += waves) {  // uniform per wave
+      err += pr_chunk(chunks[k], k, g, base, contrib_next, partial, [&](const int* u, float* x) {
+        #pragma unroll
+        for (int j = 0; j < kChunk / kWave; j++) x[j] = (u[j] >= kHotRanks) ? contrib_cur[u[j]] : 0.0f;
+        #pragma unroll
+        for (int j = 0; j < kChunk / kWave; j++) {
+          if (u[j] >= 0 && u[j] < kHotRanks) x[j] = s_hot[u[j]];
+        }
+      });
+    }
+  }
+  round_partial_ll(ctl, 2, err, s_red);
+}
+
+// One iteration's sums: first the chunks, unless pr_hot_chunks does them (one
+// wave each; chunks are at most kChunk edges, so a fixed round-robin share
+// balances), then the small rows in 64-row tiles, also round robin.  Small
+// rows: consecutive small rows form runs whose edges are contiguous, streamed
+// kSlice at a time (independent loads, values parked in LDS); each lane then
+// adds its own row's values in edge order.
+__global__ void __launch_bounds__(kBlock) pr_bal_main(PrSource src, int n, float base,
                                                        const float* __restrict__ contrib_cur,
                                                        float* __restrict__ contrib_next,
                                                        const int* __restrict__ counts,
@@ -224,33 +413,20 @@ __global__ void __launch_bounds__(kBlock) pr_bal_main(const int* __restrict__ ni
   __shared__ long long s_red[kWavesPerBlock];
   __shared__ float s_val[kWavesPerBlock][kSlice];
   if (round_done(ctl)) return;
+  const PrGraph g = pr_graph(src);
+  const int* __restrict__ nindex = g.nindex;
+  const int* __restrict__ nlist = g.nlist;
+  float* __restrict__ score = g.score;
   long long err = 0;
   const int waves = gridDim.x * kWavesPerBlock;
   const int gw = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
   const int lane = lane_id();
-  constexpr int kPer = kChunk / kWave;
-  const int nch = counts[2];
+  const int nch = (src.relabel != nullptr && *src.relabel != 0) ? 0 : counts[2];
   for (int k = gw; k < nch; k += waves) {  // uniform per wave
-    const Entry en = chunks[k];
-    int u[kPer];
-    #pragma unroll
-    for (int j = 0; j < kPer; j++) {
-      const int i = en.beg + j * kWave + lane;
-      u[j] = (i < en.end) ? nlist[i] : -1;
-    }
-    float x[kPer];
-    #pragma unroll
-    for (int j = 0; j < kPer; j++) x[j] = (u[j] >= 0) ? contrib_cur[u[j]] : 0.0f;
-    Pair acc{0.0f, 0.0f};
-    #pragma unroll
-    for (int j = 0; j < kPer; j++) {
-      if (u[j] >= 0) two_sum_add(acc, x[j]);
-    }
-    acc = wave_merge(acc);
-    if (lane == 0) {
-      if (en.pad < 0) err += pr_finish(en.v, acc, base, nindex, score, contrib_next);
-      else partial[k] = acc;
-    }
+    err += pr_chunk(chunks[k], k, g, base, contrib_next, partial, [&](const int* u, float* x) {
+      #pragma unroll
+      for (int j = 0; j < kChunk / kWave; j++) x[j] = (u[j] >= 0) ? contrib_cur[u[j]] : 0.0f;
+    });
   }
   float* vbuf = s_val[threadIdx.x / kWave];
   for (int v0 = gw * kWave; v0 < n; v0 += waves * kWave) {  // uniform per wave
@@ -300,21 +476,34 @@ __global__ void __launch_bounds__(kBlock) pr_bal_main(const int* __restrict__ ni
   round_partial_ll(ctl, 0, err, s_red);
 }
 
-__global__ void __launch_bounds__(kBlock) pr_bal_big(const int* __restrict__ nindex, float base,
-                                                      float* __restrict__ score, float* __restrict__ contrib_next,
+// The partial sums of the rows of several chunks, kBigLanes lanes a row: each
+// merges every kBigLanes-th one, then the lanes merge in lane order.  (One
+// lane a row left the longest row's chain, 273 merges on R-MAT 20, as the
+// kernel's time: 29 us.)
+constexpr int kBigLanes = 8;
+__global__ void __launch_bounds__(kBlock) pr_bal_big(PrSource src, float base, float* __restrict__ contrib_next,
                                                       const BigRow* __restrict__ big, const int* __restrict__ counts,
                                                       const Pair* __restrict__ partial, Ctl* ctl)
 {
   __shared__ long long s_red[kWavesPerBlock];
   if (round_done(ctl)) return;
+  const PrGraph g = pr_graph(src);
   long long err = 0;
   const int nb = counts[1];
-  const int stride = gridDim.x * kBlock;
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < nb; i += stride) {
+  const int l = threadIdx.x % kBigLanes;
+  const int stride = gridDim.x * (kBlock / kBigLanes);
+  for (int i = blockIdx.x * (kBlock / kBigLanes) + threadIdx.x / kBigLanes; i < nb; i += stride) {
     const BigRow b = big[i];
     Pair acc{0.0f, 0.0f};
-    for (int k = 0; k < b.count; k++) acc = pair_merge(acc, partial[b.first + k]);
-    err += pr_finish(b.v, acc, base, nindex, score, contrib_next);
+    for (int k = l; k < b.count; k += kBigLanes) acc = pair_merge(acc, partial[b.first + k]);
+    #pragma unroll
+    for (int d = 1; d < kBigLanes; d <<= 1) {
+      Pair o;
+      o.s = __shfl_xor(acc.s, d, kWave);
+      o.e = __shfl_xor(acc.e, d, kWave);
+      acc = ((l & d) == 0) ? pair_merge(acc, o) : pair_merge(o, acc);
+    }
+    if (l == 0) err += pr_finish(b.v, acc, base, g.nindex, g.score, contrib_next);
   }
   round_partial_ll(ctl, 1, err, s_red);
 }
@@ -426,7 +615,7 @@ int style_pull(const igx_graph* g, int, void* out, const void*, igx_run_info* in
         float* nxt = (r & 1) ? c0 : c1;
         hipLaunchKernelGGL((pr_pull<G>), dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, g->nlist,
                            g->nodes, base, score, cur, nxt, R.d_ctl, P.eps, P.max_iter);
-        launch_finalize<0x1>(R.persist_blocks, FinPr{P.eps, P.max_iter});
+        launch_finalize<0x1>(R.persist_blocks, FinPr{P.eps, P.max_iter, nullptr, nullptr});
       },
       P.max_iter, &rounds, &launches);
   IGX_TRY(timer_stop(&info->seconds));
@@ -439,41 +628,95 @@ int style_pull(const igx_graph* g, int, void* out, const void*, igx_run_info* in
 int style_balanced(const igx_graph* g, int, void* out, const void*, igx_run_info* info)
 {
   Runtime& R = rt();
-  float* score = (float*)out;
   float *c0 = nullptr, *c1 = nullptr;
   IGX_TRY(pr_buffers(g, &c0, &c1));
   const int n = g->nodes;
+  const int m = g->edges;
   // rows above kSmallRow: at most edges / (kSmallRow + 1) of them, each with
   // at most deg / kChunk + 1 chunks
-  const size_t nrows = (size_t)g->edges / (kSmallRow + 1) + 64;
-  const size_t nchunks = (size_t)g->edges / kChunk + nrows;
-  void *pcnt = nullptr, *pch = nullptr, *pbig = nullptr, *ppart = nullptr;
-  IGX_TRY(ws_get(WS_B, sizeof(int) * 64, &pcnt));
+  const size_t nrows = (size_t)m / (kSmallRow + 1) + 64;
+  const size_t nchunks = (size_t)m / kChunk + nrows;
+  // counters and the degree bins; the relabel flag is kept at kFlag
+  constexpr int kFlag = 8, kSmall = 64 + kRankBins;
+  constexpr int kFirstBatch = 4;
+  const int tiles = (int)(((long long)m + kEdgeTile - 1) / kEdgeTile);
+  void *pcnt = nullptr, *pch = nullptr, *pbig = nullptr, *ppart = nullptr, *pr1 = nullptr, *pl1 = nullptr,
+       *ptile = nullptr;
+  IGX_TRY(ws_get(WS_B, sizeof(int) * kSmall, &pcnt));
   IGX_TRY(ws_get(WS_D, sizeof(Entry) * nchunks, &pch));
   IGX_TRY(ws_get(WS_C, sizeof(BigRow) * nrows, &pbig));
   IGX_TRY(ws_get(WS_H, sizeof(Pair) * nchunks, &ppart));
+  // the renumbered copy; without the memory for it the run does without
+  const bool may = n >= kRelabelMinNodes && m > 0 &&
+                   ws_get(WS_A, sizeof(int) * 5 * ((size_t)n + 1), &pr1) == IGX_OK &&
+                   ws_get(WS_E, sizeof(int) * (size_t)m, &pl1) == IGX_OK &&
+                   ws_get(WS_BLOCKS, sizeof(int) * ((size_t)tiles + scan_tiles_for(n + 1) + 64), &ptile) == IGX_OK;
+  int* counts = (int*)pcnt;
+  int* bins = counts + 64;
+  int* rank = (int*)pr1;
+  int* order = rank + n;
+  int* degree = order + n;             // n + 1
+  int* nindex1 = degree + n + 1;       // n + 1
+  float* score1 = (float*)(nindex1 + n + 1);
+  int* tile_row = (int*)ptile;
+  int* tile_sum = tile_row + tiles;
+  const PrSource src = {{g->nindex, may ? nindex1 : g->nindex},
+                        {g->nlist, may ? (int*)pl1 : g->nlist},
+                        {(float*)out, may ? score1 : (float*)out},
+                        may ? counts + kFlag : (int*)nullptr};
   const PrParams P = pr_params();
   const float base = (1.0f - kDamp) / (float)n;
   IGX_TRY(timer_start());
   IGX_TRY(ctl_reset(n));
-  hipLaunchKernelGGL(pr_zero, dim3(1), dim3(64), 0, R.stream, (int*)pcnt, 64);
-  hipLaunchKernelGGL(pr_init, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, R.stream, g->nindex, n, score, c0);
-  hipLaunchKernelGGL(pr_classify, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, n, (int*)pcnt,
+  hipLaunchKernelGGL(pr_zero, dim3(blocks_for(kSmall, kBlock)), dim3(kBlock), 0, R.stream, counts, kSmall);
+  if (may) {
+    const int* go = counts + kFlag;
+    const int rank_blocks = blocks_for(n, kRankRows);
+    hipLaunchKernelGGL(rank_hist, dim3(rank_blocks), dim3(kBlock), 0, R.stream, g->nindex, n, bins, tile_row);
+    hipLaunchKernelGGL(rank_bins, dim3(1), dim3(kBlock), 0, R.stream, bins, kSmallRow, counts + kFlag + 1,
+                       kHotRanks, m, counts + kFlag);
+    hipLaunchKernelGGL(rank_assign, dim3(rank_blocks), dim3(kBlock), 0, R.stream, g->nindex, n, bins, rank, order,
+                       degree, go);
+    exclusive_scan(degree, nindex1, n + 1, tile_sum, tile_sum + scan_tiles_for(n + 1), R.stream, go);
+    hipLaunchKernelGGL(pr_relabel, dim3(tiles), dim3(kBlock), 0, R.stream, g->nindex, g->nlist, n, m,
+                       (const int*)rank, (const int*)tile_row, (const int*)nindex1, (int*)pl1, go);
+  }
+  hipLaunchKernelGGL(pr_bal_init, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, R.stream, src, n, c0);
+  hipLaunchKernelGGL(pr_classify, dim3(blocks_for(n, kClassRows)), dim3(kBlock), 0, R.stream, src, n, counts,
                      (Entry*)pch, (BigRow*)pbig);
   int rounds = 0, launches = 0;
   const int rc = run_rounds(
       [&](long long r) {
         float* cur = (r & 1) ? c1 : c0;
         float* nxt = (r & 1) ? c0 : c1;
+        // once a batch of iterations has come back, the kernels that have
+        // nothing to do on this graph are left out
+        const bool known = r >= kFirstBatch;
+        const bool hot = may && (!known || R.h_ctl->aux_ll[1] != 0);
+        const bool big = !known || R.h_ctl->aux_ll[0] != 0;
+        if (hot) {
+          hipLaunchKernelGGL(pr_hot_chunks, dim3(2 * R.cus), dim3(kHotBlock), 0, R.stream, src, n, base, cur, nxt,
+                             (const int*)counts, (const Entry*)pch, (Pair*)ppart, R.persist_blocks, R.d_ctl);
+        }
         ktimer_begin("pr_bal_main");
-        hipLaunchKernelGGL(pr_bal_main, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, g->nlist, n,
-                           base, score, cur, nxt, (const int*)pcnt, (const Entry*)pch, (Pair*)ppart, R.d_ctl);
+        hipLaunchKernelGGL(pr_bal_main, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, src, n, base, cur, nxt,
+                           (const int*)counts, (const Entry*)pch, (Pair*)ppart, R.d_ctl);
         ktimer_end("pr_bal_main");
-        hipLaunchKernelGGL(pr_bal_big, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, base, score,
-                           nxt, (const BigRow*)pbig, (const int*)pcnt, (const Pair*)ppart, R.d_ctl);
-        launch_finalize<0x3>(R.persist_blocks, FinPr{P.eps, P.max_iter});
+        if (big) {
+          hipLaunchKernelGGL(pr_bal_big, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, src, base, nxt,
+                             (const BigRow*)pbig, (const int*)counts, (const Pair*)ppart, R.d_ctl);
+        }
+        const FinPr fin{P.eps, P.max_iter, counts + 1, src.relabel};
+        if (hot && big) launch_finalize<0x7>(R.persist_blocks, fin);
+        else if (hot) launch_finalize<0x5>(R.persist_blocks, fin);
+        else if (big) launch_finalize<0x3>(R.persist_blocks, fin);
+        else launch_finalize<0x1>(R.persist_blocks, fin);
       },
-      P.max_iter, &rounds, &launches);
+      P.max_iter, &rounds, &launches, kFirstBatch);
+  if (may && R.h_ctl->aux_ll[1] != 0) {
+    hipLaunchKernelGGL(pr_scores_out, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, R.stream, src, n,
+                       (const int*)order);
+  }
   IGX_TRY(timer_stop(&info->seconds));
   info->iterations = rounds;
   info->launches = launches;
@@ -509,7 +752,7 @@ int style_push(const igx_graph* g, int, void* out, const void*, igx_run_info* in
         ktimer_end("pr_push");
         hipLaunchKernelGGL(pr_push_compute, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, n, base,
                            score, contrib, incoming, R.d_ctl);
-        launch_finalize<0x1>(R.persist_blocks, FinPr{P.eps, P.max_iter});
+        launch_finalize<0x1>(R.persist_blocks, FinPr{P.eps, P.max_iter, nullptr, nullptr});
       },
       P.max_iter, &rounds, &launches);
   IGX_TRY(timer_stop(&info->seconds));

@@ -28,6 +28,7 @@
 
 #include "igx_internal.hpp"
 #include "igx_frontier.hpp"
+#include "igx_rank.hpp"
 #include "igx_scan.hpp"
 
 namespace igx {
@@ -224,12 +225,7 @@ __global__ void __launch_bounds__(kBlock) tc_edge_bsearch(const int* __restrict_
 // of its out-neighbours, orientation by a row map, flags and a scan over the
 // edges) and now: R-MAT 20 (n = 1,048,576, m = 31.4 M) 38.4 -> 3.7 ms;
 // Erdos-Renyi n = 2,097,152, average degree 16: 2.76 -> 1.27 ms.
-constexpr int kTcTile = 2048;                    // edges per workgroup of the flat edge passes
-constexpr int kTcPer = kTcTile / kBlock;
-constexpr int kTcWords = kTcTile / kWave;        // keep-bit words per tile
-constexpr int kTcExact = 2048;                   // degrees below it have a bin of their own
-constexpr int kTcBins = kTcExact + 21 * 64;
-constexpr int kTcRankRows = 4096;                // vertices per workgroup of the rank passes
+constexpr int kTcWords = kEdgeTile / kWave;      // keep-bit words per tile
 constexpr int kTcShort = 32;                     // lists up to this length: 16-byte groups against a list in LDS
 constexpr int kTcBitWords = 4096;                // bitmap of 2^17 ranks, 16 KB
 constexpr int kTcHashSlice = kTcBitWords / 4;    // list elements per pass where ranks exceed the bitmap
@@ -240,137 +236,9 @@ constexpr int kTcShortRows = 32;                 // rows per wave step of the sh
 
 typedef int TcInt4 __attribute__((ext_vector_type(4), aligned(4)));
 
-// degree -> bin: exact below kTcExact, then 64 per octave.  Any order of the
-// vertices within a bin is a valid order of the whole.
-__device__ __forceinline__ int tc_bin(int deg)
-{
-  if (deg < kTcExact) return deg;
-  const int e = 31 - __clz(deg);
-  return kTcExact + (e - 11) * 64 + ((deg >> (e - 6)) & 63);
-}
-
 __global__ void __launch_bounds__(kBlock) tc_clear(int* __restrict__ p, int count)
 {
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < count; i += gridDim.x * kBlock) p[i] = 0;
-}
-
-// bins[k] += vertices of bin k, and tile_row[t] = the row that holds edge
-// t * kTcTile
-__global__ void __launch_bounds__(kBlock) tc_hist(const int* __restrict__ nindex, int n, int* __restrict__ bins,
-                                                   int* __restrict__ tile_row)
-{
-  __shared__ int s_bin[kTcBins];
-  for (int i = threadIdx.x; i < kTcBins; i += kBlock) s_bin[i] = 0;
-  __syncthreads();
-  const long long base = (long long)blockIdx.x * kTcRankRows;
-  for (int i = threadIdx.x; i < kTcRankRows; i += kBlock) {
-    const long long v = base + i;
-    if (v >= n) break;
-    const int b = nindex[v], e = nindex[v + 1];
-    atomicAdd(&s_bin[tc_bin(e - b)], 1);
-    if (e == b) continue;
-    for (int t = (int)(((long long)b + kTcTile - 1) / kTcTile); (long long)t * kTcTile < e; t++) tile_row[t] = (int)v;
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < kTcBins; i += kBlock) {
-    if (s_bin[i] != 0) atomicAdd(&bins[i], s_bin[i]);
-  }
-}
-
-// bins become the first rank of each (highest degree first); *heavy = number
-// of vertices of degree above kTcShort.  One workgroup.
-__global__ void __launch_bounds__(kBlock) tc_bin_ranks(int* __restrict__ bins, int* __restrict__ heavy)
-{
-  __shared__ int s_red[kWavesPerBlock];
-  constexpr int kPerT = (kTcBins + kBlock - 1) / kBlock;
-  int c[kPerT];
-  int local = 0;
-  #pragma unroll
-  for (int k = 0; k < kPerT; k++) {
-    const int i = kTcBins - 1 - ((int)threadIdx.x * kPerT + k);
-    c[k] = (i >= 0) ? bins[i] : 0;
-    local += c[k];
-  }
-  int tot = 0;
-  int run = block_excl_scan(local, s_red, &tot);
-  #pragma unroll
-  for (int k = 0; k < kPerT; k++) {
-    const int i = kTcBins - 1 - ((int)threadIdx.x * kPerT + k);
-    if (i >= 0) bins[i] = run;
-    if (i == kTcShort) *heavy = run;
-    run += c[k];
-  }
-}
-
-// rank[v] and its inverse order[]: a workgroup reserves a run of ranks in
-// each bin for its vertices
-__global__ void __launch_bounds__(kBlock) tc_rank(const int* __restrict__ nindex, int n, int* __restrict__ bins,
-                                                   int* __restrict__ rank, int* __restrict__ order)
-{
-  __shared__ int s_bin[kTcBins];
-  for (int i = threadIdx.x; i < kTcBins; i += kBlock) s_bin[i] = 0;
-  __syncthreads();
-  const long long base = (long long)blockIdx.x * kTcRankRows;
-  int bin[kTcRankRows / kBlock];
-  #pragma unroll
-  for (int k = 0; k < kTcRankRows / kBlock; k++) {
-    const long long v = base + k * kBlock + threadIdx.x;
-    bin[k] = (v < n) ? tc_bin(nindex[v + 1] - nindex[v]) : 0;
-    if (v < n) atomicAdd(&s_bin[bin[k]], 1);
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < kTcBins; i += kBlock) {
-    if (s_bin[i] != 0) s_bin[i] = atomicAdd(&bins[i], s_bin[i]);
-  }
-  __syncthreads();
-  #pragma unroll
-  for (int k = 0; k < kTcRankRows / kBlock; k++) {
-    const long long v = base + k * kBlock + threadIdx.x;
-    if (v < n) {
-      const int r = atomicAdd(&s_bin[bin[k]], 1);
-      rank[v] = r;
-      order[r] = (int)v;
-    }
-  }
-}
-
-// s_row[i] = row of edge base + i, minus r0 (the row of edge base), for the
-// tile's kTcTile edges: the rows that start inside the tile mark their first
-// edge, and a running maximum carries each to the next.  r1: the row of the
-// next tile's first edge (n - 1 for the last tile).
-__device__ __forceinline__ void tc_tile_rows(const int* __restrict__ nindex, int base, int r0, int r1, int* s_row,
-                                             int* s_red)
-{
-  const int tid = threadIdx.x;
-  for (int i = tid; i < kTcTile; i += kBlock) s_row[i] = 0;
-  __syncthreads();
-  for (int r = r0 + 1 + tid; r <= r1; r += kBlock) {
-    const int p = nindex[r] - base;  // empty rows share the place of the row after them, the larger one stays
-    if (p < kTcTile) atomicMax(&s_row[p], r - r0);
-  }
-  __syncthreads();
-  int x[kTcPer];
-  int mx = 0;
-  #pragma unroll
-  for (int k = 0; k < kTcPer; k++) {
-    mx = max(mx, s_row[tid * kTcPer + k]);
-    x[k] = mx;
-  }
-  int incl = mx;
-  #pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const int t = __shfl_up(incl, d, kWave);
-    if (lane_id() >= d) incl = max(incl, t);
-  }
-  const int w = tid / kWave;
-  if (lane_id() == kWave - 1) s_red[w] = incl;
-  int before = __shfl_up(incl, 1, kWave);
-  if (lane_id() == 0) before = 0;
-  __syncthreads();
-  for (int k = 0; k < w; k++) before = max(before, s_red[k]);
-  #pragma unroll
-  for (int k = 0; k < kTcPer; k++) s_row[tid * kTcPer + k] = max(before, x[k]);
-  __syncthreads();
 }
 
 // keep bit of edge (v, u): u ranks above v.  Also the sorted check of the
@@ -385,29 +253,29 @@ __global__ void __launch_bounds__(kBlock) tc_keep(const int* __restrict__ nindex
                                                    unsigned long long* __restrict__ keep, int* __restrict__ tile_count,
                                                    int* __restrict__ bad)
 {
-  __shared__ __align__(16) int s_row[kTcTile];
+  __shared__ __align__(16) int s_row[kEdgeTile];
   __shared__ int s_red[kWavesPerBlock];
   const int tile = blockIdx.x;
-  const int base = tile * kTcTile;
+  const int base = tile * kEdgeTile;
   const int r0 = tile_row[tile];
   const int r1 = (tile + 1 < (int)gridDim.x) ? tile_row[tile + 1] : n - 1;
-  int u[kTcPer], prev[kTcPer];
+  int u[kEdgePer], prev[kEdgePer];
   #pragma unroll
-  for (int k = 0; k < kTcPer; k++) {
+  for (int k = 0; k < kEdgePer; k++) {
     const int i = k * kBlock + (int)threadIdx.x;
     const bool in = i < m - base;
     u[k] = in ? nlist[base + i] : -1;
     prev[k] = (in && base + i > 0) ? nlist[base + i - 1] : -1;
   }
-  int ru[kTcPer];
+  int ru[kEdgePer];
   #pragma unroll
-  for (int k = 0; k < kTcPer; k++) ru[k] = (u[k] >= 0) ? rank[u[k]] : 0;
-  tc_tile_rows(nindex, base, r0, r1, s_row, s_red);
+  for (int k = 0; k < kEdgePer; k++) ru[k] = (u[k] >= 0) ? rank[u[k]] : 0;
+  edge_tile_rows(nindex, base, r0, r1, s_row, s_red);
   const int head0 = nindex[r0];  // the first row may start before the tile
   int count = 0;
   bool wrong = false;
   #pragma unroll
-  for (int k = 0; k < kTcPer; k++) {
+  for (int k = 0; k < kEdgePer; k++) {
     const int i = k * kBlock + (int)threadIdx.x;
     bool kept = false;
     if (u[k] >= 0) {
@@ -443,7 +311,7 @@ __global__ void __launch_bounds__(kBlock) tc_orient(const int* __restrict__ nind
   __shared__ unsigned long long s_word[kTcWords + 1];
   __shared__ int s_pre[kTcWords + 1];
   const int tile = blockIdx.x;
-  const int base = tile * kTcTile;
+  const int base = tile * kEdgeTile;
   const int lane = lane_id();
   if (threadIdx.x < kWave) {
     const unsigned long long word = (lane < kTcWords) ? keep[(size_t)tile * kTcWords + lane] : 0ull;
@@ -457,7 +325,7 @@ __global__ void __launch_bounds__(kBlock) tc_orient(const int* __restrict__ nind
   __syncthreads();
   const int off = tile_off[tile];
   #pragma unroll
-  for (int k = 0; k < kTcPer; k++) {
+  for (int k = 0; k < kEdgePer; k++) {
     const int i = k * kBlock + (int)threadIdx.x;
     const unsigned long long word = s_word[i / kWave];
     if ((word >> lane) & 1ull) {
@@ -472,7 +340,7 @@ __global__ void __launch_bounds__(kBlock) tc_orient(const int* __restrict__ nind
   const int first = (tile == 0) ? 0 : tile_row[tile] + 1;
   const int to = last ? n : tile_row[tile + 1];
   for (int r = first + (int)threadIdx.x; r <= to; r += kBlock) {
-    const int p = nindex[r] - base;  // 0 .. kTcTile
+    const int p = nindex[r] - base;  // 0 .. kEdgeTile
     const unsigned long long below = s_word[p >> 6] & ((1ull << (p & 63)) - 1ull);
     onidx[r] = off + s_pre[p >> 6] + __popcll(below);
   }
@@ -782,8 +650,8 @@ int style_oriented(const igx_graph* g, int, void* out, const void*, igx_run_info
   Runtime& R = rt();
   const int n = g->nodes;
   const int m = g->edges;
-  const int tiles = (int)(((long long)m + kTcTile - 1) / kTcTile);
-  const int rank_blocks = blocks_for(n, kTcRankRows);
+  const int tiles = (int)(((long long)m + kEdgeTile - 1) / kEdgeTile);
+  const int rank_blocks = blocks_for(n, kRankRows);
   void *pidx = nullptr, *plist = nullptr, *prl = nullptr, *ptile = nullptr, *pkeep = nullptr, *prank = nullptr,
        *psmall = nullptr;
   IGX_TRY(ws_get(WS_B, sizeof(int) * ((size_t)n + 1), &pidx));
@@ -797,7 +665,7 @@ int style_oriented(const igx_graph* g, int, void* out, const void*, igx_run_info
   IGX_TRY(ws_get(WS_G, sizeof(unsigned long long) * ((size_t)scan_n * kTcWords), &pkeep));
   IGX_TRY(ws_get(WS_A, sizeof(int) * 2 * (size_t)n, &prank));
   // [0,1] count, [2] sorted check, [3] heavy, then the claim counters and the bins
-  constexpr int kSmall = 64 + kGroups * kTcClaimStride + kTcBins;
+  constexpr int kSmall = 64 + kGroups * kTcClaimStride + kRankBins;
   IGX_TRY(ws_get(WS_D, sizeof(int) * kSmall, &psmall));
   int* onidx = (int*)pidx;
   int* olist = (int*)plist;
@@ -818,9 +686,11 @@ int style_oriented(const igx_graph* g, int, void* out, const void*, igx_run_info
   IGX_TRY(timer_start());
   hipLaunchKernelGGL(tc_clear, dim3(blocks_for(kSmall, kBlock)), dim3(kBlock), 0, R.stream, small, kSmall);
   if (m > 0) {
-    hipLaunchKernelGGL(tc_hist, dim3(rank_blocks), dim3(kBlock), 0, R.stream, g->nindex, n, bins, tile_row);
-    hipLaunchKernelGGL(tc_bin_ranks, dim3(1), dim3(kBlock), 0, R.stream, bins, heavy);
-    hipLaunchKernelGGL(tc_rank, dim3(rank_blocks), dim3(kBlock), 0, R.stream, g->nindex, n, bins, rank, order);
+    hipLaunchKernelGGL(rank_hist, dim3(rank_blocks), dim3(kBlock), 0, R.stream, g->nindex, n, bins, tile_row);
+    hipLaunchKernelGGL(rank_bins, dim3(1), dim3(kBlock), 0, R.stream, bins, kTcShort, heavy, 0, m,
+                       (int*)nullptr);
+    hipLaunchKernelGGL(rank_assign, dim3(rank_blocks), dim3(kBlock), 0, R.stream, g->nindex, n, bins, rank, order,
+                       (int*)nullptr, (const int*)nullptr);
     hipLaunchKernelGGL(tc_keep, dim3(tiles), dim3(kBlock), 0, R.stream, g->nindex, g->nlist, n, m, (const int*)rank,
                        (const int*)tile_row, keep, tile_count, bad);
     exclusive_scan(tile_count, tile_off, tiles, tile_sum, tile_sum + scan_tiles_for(scan_n), R.stream);
