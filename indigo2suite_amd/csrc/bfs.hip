@@ -35,12 +35,6 @@ __global__ void __launch_bounds__(kBlock) fill_int(int* __restrict__ p, int valu
   for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < count; i += stride) p[i] = value;
 }
 
-__device__ __forceinline__ void raise_flag(Ctl* ctl, bool updated)
-{
-  const uint64_t any = ballot(updated);
-  if (any != 0 && lane_id() == (__ffsll((unsigned long long)any) - 1)) store_relaxed(&ctl->flag, 1);
-}
-
 // --------------------------------------------------- vertex, topology ----
 template <int G, int AK, bool DETERM, bool PERSIST>
 __global__ void __launch_bounds__(kBlock) bfs_vtopo_push(const int* __restrict__ nindex,

@@ -36,13 +36,6 @@ __global__ void __launch_bounds__(kBlock) cc_fill(int* __restrict__ p, int value
   for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < count; i += stride) p[i] = value;
 }
 
-
-__device__ __forceinline__ void cc_raise_flag(Ctl* ctl, bool updated)
-{
-  const uint64_t any = ballot(updated);
-  if (any != 0 && lane_id() == (__ffsll((unsigned long long)any) - 1)) store_relaxed(&ctl->flag, 1);
-}
-
 template <int G, int AK, bool PERSIST>
 __global__ void __launch_bounds__(kBlock) cc_vtopo_push(const int* __restrict__ nindex,
                                                          const int* __restrict__ nlist, int n,
@@ -78,7 +71,7 @@ __global__ void __launch_bounds__(kBlock) cc_vtopo_push(const int* __restrict__ 
       }
     }
   }
-  cc_raise_flag(ctl, updated);
+  raise_flag(ctl, updated);
 }
 
 __global__ void __launch_bounds__(kBlock) cc_vtopo_pull(const int* __restrict__ nindex,
@@ -97,7 +90,7 @@ __global__ void __launch_bounds__(kBlock) cc_vtopo_pull(const int* __restrict__ 
       updated = true;
     }
   }
-  cc_raise_flag(ctl, updated);
+  raise_flag(ctl, updated);
 }
 
 // ------------------------------------------------ deterministic (Jacobi) ----
@@ -140,7 +133,7 @@ __global__ void __launch_bounds__(kBlock) cc_determ_push(const int* __restrict__
       for (int i = nindex[v] + lane; i < nindex[v + 1]; i += kWave) push(i, l);
     }
   }
-  cc_raise_flag(ctl, updated);
+  raise_flag(ctl, updated);
 }
 
 template <int G>
@@ -174,7 +167,7 @@ __global__ void __launch_bounds__(kBlock) cc_determ_pull(const int* __restrict__
       }
     }
   }
-  cc_raise_flag(ctl, updated);
+  raise_flag(ctl, updated);
 }
 
 __global__ void __launch_bounds__(kBlock) cc_etopo_push(const int* __restrict__ nlist, const int* __restrict__ sp,
@@ -188,7 +181,7 @@ __global__ void __launch_bounds__(kBlock) cc_etopo_push(const int* __restrict__ 
     const int dst = nlist[e];
     if (label[dst] > lv && atomic_min_relaxed(&label[dst], lv) > lv) updated = true;
   }
-  cc_raise_flag(ctl, updated);
+  raise_flag(ctl, updated);
 }
 
 // worklist seeded with all items [0, count)

@@ -290,6 +290,19 @@ __device__ __forceinline__ void round_partial_d(Ctl* ctl, int slot, double v, do
   }
 }
 
+// Round kernel side of the common topology-driven rule: any lane with `again`
+// asks for another round.  A wave stores the flag only if it reads 0, and
+// plainly (the kernel boundary publishes it): agent-scope stores of thousands
+// of waves to the one address take about 11 ns each, which was 60-100 us of
+// every round in which most waves had something pending.
+__device__ __forceinline__ void raise_flag(Ctl* ctl, bool again)
+{
+  const uint64_t any = ballot(again);
+  if (any == 0 || lane_id() != __ffsll((unsigned long long)any) - 1) return;
+  volatile int* flag = &ctl->flag;
+  if (*flag == 0) *flag = 1;
+}
+
 // the common topology-driven rule: stop after a round without updates
 __device__ __forceinline__ void finalize_flag_round(Ctl* ctl)
 {

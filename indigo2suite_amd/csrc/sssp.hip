@@ -38,12 +38,6 @@ __global__ void __launch_bounds__(kBlock) sssp_fill(int* __restrict__ p, int val
   for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < count; i += stride) p[i] = value;
 }
 
-__device__ __forceinline__ void sssp_raise_flag(Ctl* ctl, bool updated)
-{
-  const uint64_t any = ballot(updated);
-  if (any != 0 && lane_id() == (__ffsll((unsigned long long)any) - 1)) store_relaxed(&ctl->flag, 1);
-}
-
 template <int G, int AK>
 __global__ void __launch_bounds__(kBlock) sssp_vtopo_push(const int* __restrict__ nindex,
                                                            const int* __restrict__ nlist,
@@ -89,7 +83,7 @@ __global__ void __launch_bounds__(kBlock) sssp_vtopo_push(const int* __restrict_
       }
     }
   }
-  sssp_raise_flag(ctl, updated);
+  raise_flag(ctl, updated);
 }
 
 __global__ void __launch_bounds__(kBlock) sssp_vtopo_pull(const int* __restrict__ nindex,
@@ -112,7 +106,7 @@ __global__ void __launch_bounds__(kBlock) sssp_vtopo_pull(const int* __restrict_
       updated = true;
     }
   }
-  sssp_raise_flag(ctl, updated);
+  raise_flag(ctl, updated);
 }
 
 __global__ void __launch_bounds__(kBlock) sssp_etopo_push(const int* __restrict__ nlist,
@@ -130,7 +124,7 @@ __global__ void __launch_bounds__(kBlock) sssp_etopo_push(const int* __restrict_
       if (dist[dst] > nd && atomic_min_relaxed(&dist[dst], nd) > nd) updated = true;
     }
   }
-  sssp_raise_flag(ctl, updated);
+  raise_flag(ctl, updated);
 }
 
 // ------------------------------------------------ deterministic (Jacobi) ----
@@ -184,7 +178,7 @@ __global__ void __launch_bounds__(kBlock) sssp_determ_push(const int* __restrict
       }
     }
   }
-  sssp_raise_flag(ctl, updated);
+  raise_flag(ctl, updated);
 }
 
 template <int G>
@@ -225,7 +219,7 @@ __global__ void __launch_bounds__(kBlock) sssp_determ_pull(const int* __restrict
       }
     }
   }
-  sssp_raise_flag(ctl, updated);
+  raise_flag(ctl, updated);
 }
 
 // ------------------------------------------------------- vertex, data ----
