@@ -232,8 +232,7 @@ __global__ void __launch_bounds__(kBlock) bfs_edata_push(const int* __restrict__
                                                           int* __restrict__ dist, int* __restrict__ wl0,
                                                           int* __restrict__ wl1, int* __restrict__ vstamp, Ctl* ctl)
 {
-  __shared__ int s_excl[kWavesPerBlock][kWave];
-  __shared__ int s_beg[kWavesPerBlock][kWave];
+  __shared__ ListLds s_list;
   if (round_done(ctl)) return;
   const int iter = ctl->iter;
   const int p = iter & 1;
@@ -242,26 +241,38 @@ __global__ void __launch_bounds__(kBlock) bfs_edata_push(const int* __restrict__
   int* wl_out = p ? wl0 : wl1;
   int* out_count = &ctl->wl_count[p ^ 1];
   const int tag = iter + 1;
-  const int w = threadIdx.x / kWave;
-  const int stride = gridDim.x * kBlock;
-  for (int base = blockIdx.x * kBlock; base < count; base += stride) {  // uniform per wave
-    const int idx = base + (int)threadIdx.x;
-    int rbeg = 0, rlen = 0;
-    if (idx < count) {
-      const int e = wl_in[idx];
-      const int s = dist[sp[e]];
-      if (s != kInf) {
-        const int nd = s + 1;
-        const int dst = nlist[e];
-        if (dist[dst] > nd && atomic_min_relaxed(&dist[dst], nd) > nd &&
-            atomic_max_relaxed(&vstamp[dst], tag) != tag) {
-          rbeg = nindex[dst];
-          rlen = nindex[dst + 1] - rbeg;
+  const int per = list_items_per_thread(count);
+  const long long step = (long long)gridDim.x * kBlock * per;
+  with_list_items(per, [&](auto items) {
+    constexpr int kPer = decltype(items)::value;
+    for (long long base = (long long)blockIdx.x * kBlock * per; base < count; base += step) {  // uniform per workgroup
+      int e[kPer], rbeg[kPer], rlen[kPer];
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) {
+        const long long idx = base + k * kBlock + (int)threadIdx.x;
+        e[k] = (k < per && idx < count) ? wl_in[idx] : -1;
+        rbeg[k] = rlen[k] = 0;
+      }
+      int s[kPer], dst[kPer], d[kPer];
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) {
+        s[k] = (e[k] >= 0) ? dist[sp[e[k]]] : kInf;
+        dst[k] = (e[k] >= 0) ? nlist[e[k]] : 0;
+      }
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) d[k] = (e[k] >= 0) ? dist[dst[k]] : 0;
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) {
+        if (s[k] == kInf) continue;
+        const int nd = s[k] + 1;
+        if (d[k] > nd && atomic_min_relaxed(&dist[dst[k]], nd) > nd && atomic_max_relaxed(&vstamp[dst[k]], tag) != tag) {
+          rbeg[k] = nindex[dst[k]];
+          rlen[k] = nindex[dst[k] + 1] - rbeg[k];
         }
       }
+      block_push_edge_ranges(wl_out, out_count, rbeg, rlen, count <= kListAlone, s_list);
     }
-    wave_push_edge_ranges(wl_out, out_count, rbeg, rlen, s_excl[w], s_beg[w]);
-  }
+  });
 }
 
 // ------------------------------------------ direction-optimizing hybrid ----

@@ -232,8 +232,7 @@ __global__ void __launch_bounds__(kBlock) cc_edata_push(const int* __restrict__ 
                                                          int* __restrict__ label, int* __restrict__ wl0,
                                                          int* __restrict__ wl1, int* __restrict__ vstamp, Ctl* ctl)
 {
-  __shared__ int s_excl[kWavesPerBlock][kWave];
-  __shared__ int s_beg[kWavesPerBlock][kWave];
+  __shared__ ListLds s_list;
   if (round_done(ctl)) return;
   const int iter = ctl->iter;
   const int p = iter & 1;
@@ -242,23 +241,37 @@ __global__ void __launch_bounds__(kBlock) cc_edata_push(const int* __restrict__ 
   int* wl_out = p ? wl0 : wl1;
   int* out_count = &ctl->wl_count[p ^ 1];
   const int tag = iter + 1;
-  const int w = threadIdx.x / kWave;
-  const int stride = gridDim.x * kBlock;
-  for (int base = blockIdx.x * kBlock; base < count; base += stride) {  // uniform per wave
-    const int idx = base + (int)threadIdx.x;
-    int rbeg = 0, rlen = 0;
-    if (idx < count) {
-      const int e = wl_in[idx];
-      const int lv = label[sp[e]];
-      const int dst = nlist[e];
-      if (label[dst] > lv && atomic_min_relaxed(&label[dst], lv) > lv &&
-          atomic_max_relaxed(&vstamp[dst], tag) != tag) {
-        rbeg = nindex[dst];
-        rlen = nindex[dst + 1] - rbeg;
+  const int per = list_items_per_thread(count);
+  const long long step = (long long)gridDim.x * kBlock * per;
+  with_list_items(per, [&](auto items) {
+    constexpr int kPer = decltype(items)::value;
+    for (long long base = (long long)blockIdx.x * kBlock * per; base < count; base += step) {  // uniform per workgroup
+      int e[kPer], rbeg[kPer], rlen[kPer];
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) {
+        const long long idx = base + k * kBlock + (int)threadIdx.x;
+        e[k] = (k < per && idx < count) ? wl_in[idx] : -1;
+        rbeg[k] = rlen[k] = 0;
       }
+      int s[kPer], dst[kPer], d[kPer];
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) {
+        s[k] = (e[k] >= 0) ? label[sp[e[k]]] : kInf;
+        dst[k] = (e[k] >= 0) ? nlist[e[k]] : 0;
+      }
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) d[k] = (e[k] >= 0) ? label[dst[k]] : 0;
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) {
+        if (e[k] >= 0 && d[k] > s[k] && atomic_min_relaxed(&label[dst[k]], s[k]) > s[k] &&
+            atomic_max_relaxed(&vstamp[dst[k]], tag) != tag) {
+          rbeg[k] = nindex[dst[k]];
+          rlen[k] = nindex[dst[k] + 1] - rbeg[k];
+        }
+      }
+      block_push_edge_ranges(wl_out, out_count, rbeg, rlen, count <= kListAlone, s_list);
     }
-    wave_push_edge_ranges(wl_out, out_count, rbeg, rlen, s_excl[w], s_beg[w]);
-  }
+  });
 }
 
 // ------------------------------------------------------------- union-find --

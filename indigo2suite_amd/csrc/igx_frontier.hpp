@@ -11,6 +11,8 @@
 // kept in LDS.  All lanes stay busy regardless of the degree mix.
 #pragma once
 
+#include <type_traits>
+
 #include "igx_device.hpp"
 
 namespace igx {
@@ -138,41 +140,117 @@ __device__ __forceinline__ void for_each_bitmap_tile(const unsigned* __restrict_
   }
 }
 
-// Append the edge ids [beg, beg + len) of every lane to an edge worklist:
-// one atomic per wave reserves the wave's total, then the 64 lanes write the
-// concatenated ranges together (each lane finds its range by binary search
-// over the exclusive prefixes in LDS), so a hub's ids go out 64 at a time in
-// contiguous stores.  All lanes of the wave call this together; lanes with
-// nothing to push pass len = 0.  lds_excl / lds_beg: this wave's 64-slot LDS
-// rows.
-__device__ __forceinline__ void wave_push_edge_ranges(int* __restrict__ out, int* counter, int beg, int len,
-                                                      int* lds_excl, int* lds_beg)
+// Edge worklists: a workgroup takes up to kListPer * kBlock consecutive items
+// per step (fewer when the list is short, so that it still spreads over the
+// grid) and appends what they queue together.  Items per thread and step:
+constexpr int kListPer = 4;
+__device__ __forceinline__ int list_items_per_thread(int count)
+{
+  const long long lanes = (long long)gridDim.x * kBlock;
+  const long long per = (count + lanes - 1) / lanes;
+  return (int)(per < kListPer ? (per < 1 ? 1 : per) : kListPer);
+}
+
+// The items per thread as a constant for the loops over them: body(1) for a
+// short list, whose rounds are latency alone, else body(kListPer).
+template <typename F>
+__device__ __forceinline__ void with_list_items(int per, F body)
+{
+  if (per == 1) body(std::integral_constant<int, 1>{});
+  else body(std::integral_constant<int, kListPer>{});
+}
+
+// LDS of block_push_edge_ranges
+struct ListLds {
+  int excl[kWavesPerBlock][kWave];
+  int beg[kWavesPerBlock][kWave];
+  int total[kWavesPerBlock];
+  int base;
+};
+
+// Append the edge ids [beg[k], beg[k] + len[k]) of every thread to an edge
+// worklist.  One atomic per workgroup reserves the places: the counter is one
+// address, where an atomic per 64 items took 11 ns each and was the time of
+// the large rounds (R-MAT 20, SSSP edge worklist: 300 k of them in a round of
+// 3.3 ms).  A short list (`alone`, at most kListAlone items) has few waves to
+// meet there, and each reserves for itself, without the workgroup's barriers.
+// Then each wave writes its ranges one k after the other, its 64 lanes
+// together: those of at most kListLong ids as one concatenation, each lane
+// finding its range by binary search over the exclusive prefixes in LDS, and
+// longer ones one by one without a search (a hub's neighbours are the other
+// hubs, in the same few waves: a million ids each on R-MAT 20, 3.3 ms of
+// searches in the first round).  All threads of the workgroup call this
+// together; threads with nothing to push pass len = 0.
+constexpr int kListAlone = 1 << 16;
+constexpr int kListLong = 256;
+
+template <int kPer>
+__device__ __forceinline__ void block_push_edge_ranges(int* __restrict__ out, int* counter, const int (&beg)[kPer],
+                                                       const int (&len)[kPer], bool alone, ListLds& L)
 {
   const int lane = lane_id();
-  const int incl = wave_incl_scan(len);
-  const int total = wave_bcast(incl, kWave - 1);
-  if (total == 0) return;
-  int base = 0;
-  if (lane == kWave - 1) base = atomicAdd(counter, total);
-  base = wave_bcast(base, kWave - 1);
-  __builtin_amdgcn_wave_barrier();
-  lds_excl[lane] = incl - len;
-  lds_beg[lane] = beg;
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  for (int tb = 0; tb < total; tb += kWave) {
-    const int t = tb + lane;
-    if (t < total) {
-      int lo = 0, hi = kWave;
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (lds_excl[mid] <= t) lo = mid;
-        else hi = mid;
-      }
-      out[base + t] = lds_beg[lo] + (t - lds_excl[lo]);
+  const int w = threadIdx.x / kWave;
+  int incl[kPer];  // inclusive prefix of the short ranges
+  int total = 0;
+  #pragma unroll
+  for (int k = 0; k < kPer; k++) {
+    incl[k] = 0;
+    if (ballot(len[k] != 0) != 0) {  // uniform per wave
+      incl[k] = wave_incl_scan((len[k] <= kListLong) ? len[k] : 0);
+      total += wave_bcast(incl[k], kWave - 1);
+      if (ballot(len[k] > kListLong) != 0) total += wave_sum((len[k] > kListLong) ? len[k] : 0);
     }
   }
-  __builtin_amdgcn_wave_barrier();
+  int base = 0;
+  if (alone) {
+    if (total == 0) return;
+    if (lane == 0) base = atomicAdd(counter, total);
+    base = wave_bcast(base, 0);
+  } else {
+    if (lane == 0) L.total[w] = total;
+    __syncthreads();
+    int before = 0, all = 0;
+    #pragma unroll
+    for (int k = 0; k < kWavesPerBlock; k++) {
+      if (k < w) before += L.total[k];
+      all += L.total[k];
+    }
+    if (threadIdx.x == 0 && all != 0) L.base = atomicAdd(counter, all);
+    __syncthreads();
+    base = L.base + before;
+  }
+  int* excl = L.excl[w];
+  int* rbeg = L.beg[w];
+  #pragma unroll
+  for (int k = 0; k < kPer; k++) {
+    const int sum = wave_bcast(incl[k], kWave - 1);
+    if (sum != 0) {  // uniform per wave
+      __builtin_amdgcn_wave_barrier();
+      excl[lane] = incl[k] - ((len[k] <= kListLong) ? len[k] : 0);
+      rbeg[lane] = beg[k];
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      for (int t = lane; t < sum; t += kWave) {
+        int lo = 0, hi = kWave;
+        while (hi - lo > 1) {
+          const int mid = (lo + hi) >> 1;
+          if (excl[mid] <= t) lo = mid;
+          else hi = mid;
+        }
+        out[base + t] = rbeg[lo] + (t - excl[lo]);
+      }
+      base += sum;
+      __builtin_amdgcn_wave_barrier();
+    }
+    for (uint64_t todo = ballot(len[k] > kListLong); todo != 0; todo &= todo - 1) {
+      const int owner = __ffsll((unsigned long long)todo) - 1;
+      const int b = __shfl(beg[k], owner, kWave), n = __shfl(len[k], owner, kWave);
+      #pragma unroll 4
+      for (int t = lane; t < n; t += kWave) out[base + t] = b + t;
+      base += n;
+    }
+  }
+  if (!alone) __syncthreads();
 }
 
 // Walk all edges of the queue entries [0, qsize) with the calling wave among

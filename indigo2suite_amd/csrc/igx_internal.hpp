@@ -64,8 +64,8 @@ int ws_get(int slot, size_t bytes, void** ptr);
 // in, is waited for alone, and after it one batch of kAheadRounds is always in
 // the stream behind the one that is waited for: at most two of them run empty,
 // where batches that doubled up to 64 cost PageRank up to 15 empty rounds of
-// three launches.  The batches grow slowly so that runs of thousands of
-// rounds wait seldom.
+// three launches.  The batches are an eighth of the rounds so far, so that
+// runs of hundreds of rounds copy the control block seldom (about 4 us each).
 // After each batch the run also stops, with IGX_ERR_TIMEOUT, once the host
 // clock since timer_start() passes the time limit set by igx_set_time_limit.
 // Returns IGX_OK, IGX_ERR_LIMIT when max_rounds did not converge, or an error.
@@ -101,8 +101,8 @@ int run_rounds(F launch, long long max_rounds, int* rounds_done, int* launches, 
     }
     // two batches behind the first one, then one for each that came back
     while (!stop && batches - waited < 2 && launched < max_rounds) {
-      const long long b = kAheadRounds + 2 * (batches / 8);
-      IGX_TRY(enqueue(b < 64 ? b : 64));
+      const long long b = launched / 8;
+      IGX_TRY(enqueue(b < kAheadRounds ? kAheadRounds : (b < 64 ? b : 64)));
     }
   }
   if (rounds_done) *rounds_done = R.h_ctl->iter;

@@ -315,8 +315,7 @@ __global__ void __launch_bounds__(kBlock) sssp_edata_push(const int* __restrict_
                                                            int* __restrict__ wl1, int* __restrict__ vstamp,
                                                            int* __restrict__ estamp, Ctl* ctl)
 {
-  __shared__ int s_excl[kWavesPerBlock][kWave];
-  __shared__ int s_beg[kWavesPerBlock][kWave];
+  __shared__ ListLds s_list;
   if (round_done(ctl)) return;
   const int iter = ctl->iter;
   const int p = iter & 1;
@@ -325,38 +324,54 @@ __global__ void __launch_bounds__(kBlock) sssp_edata_push(const int* __restrict_
   int* wl_out = p ? wl0 : wl1;
   int* out_count = &ctl->wl_count[p ^ 1];
   const int tag = iter + 1;
-  const int w = threadIdx.x / kWave;
-  const int stride = gridDim.x * kBlock;
-  for (int base = blockIdx.x * kBlock; base < count; base += stride) {  // uniform per wave
-    const int idx = base + (int)threadIdx.x;
-    int rbeg = 0, rlen = 0;
-    if (idx < count) {
-      const int e = wl_in[idx];
-      const int s = load_relaxed(&dist[sp[e]]);
-      if (s != kInf) {
-        const int nd = s + ew[e];
-        const int dst = nlist[e];
-        bool improved;
+  const int per = list_items_per_thread(count);
+  const long long step = (long long)gridDim.x * kBlock * per;
+  with_list_items(per, [&](auto items) {
+    constexpr int kPer = decltype(items)::value;
+    for (long long base = (long long)blockIdx.x * kBlock * per; base < count; base += step) {  // uniform per workgroup
+      int e[kPer], rbeg[kPer], rlen[kPer];
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) {
+        const long long idx = base + k * kBlock + (int)threadIdx.x;
+        e[k] = (k < per && idx < count) ? wl_in[idx] : -1;
+        rbeg[k] = rlen[k] = 0;
+      }
+      // the source's distance by a plain load, but for RW: a value lowered in
+      // this round that it misses is queued again with the source's edges
+      int s[kPer], dst[kPer], wt[kPer], d[kPer];
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) {
+        const int src = (e[k] >= 0) ? sp[e[k]] : 0;
+        s[k] = (e[k] < 0) ? kInf : (RW ? load_relaxed(&dist[src]) : dist[src]);
+        dst[k] = (e[k] >= 0) ? nlist[e[k]] : 0;
+        wt[k] = (e[k] >= 0) ? ew[e[k]] : 0;
+      }
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) d[k] = (e[k] < 0) ? 0 : (RW ? load_relaxed(&dist[dst[k]]) : dist[dst[k]]);
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) {
+        if (s[k] == kInf) continue;
+        const int nd = s[k] + wt[k];
+        bool improved = d[k] > nd;
         if (RW) {
-          improved = load_relaxed(&dist[dst]) > nd;
           if (improved) {
-            store_relaxed(&dist[dst], nd);
-            if (atomic_max_relaxed(&estamp[e], tag) != tag) {
+            store_relaxed(&dist[dst[k]], nd);
+            if (atomic_max_relaxed(&estamp[e[k]], tag) != tag) {
               const int slot = atomicAdd(out_count, 1);
-              wl_out[slot] = e;
+              wl_out[slot] = e[k];
             }
           }
         } else {
-          improved = dist[dst] > nd && atomic_min_relaxed(&dist[dst], nd) > nd;
+          improved = improved && atomic_min_relaxed(&dist[dst[k]], nd) > nd;
         }
-        if (improved && atomic_max_relaxed(&vstamp[dst], tag) != tag) {
-          rbeg = nindex[dst];
-          rlen = nindex[dst + 1] - rbeg;
+        if (improved && atomic_max_relaxed(&vstamp[dst[k]], tag) != tag) {
+          rbeg[k] = nindex[dst[k]];
+          rlen[k] = nindex[dst[k] + 1] - rbeg[k];
         }
       }
+      block_push_edge_ranges(wl_out, out_count, rbeg, rlen, count <= kListAlone, s_list);
     }
-    wave_push_edge_ranges(wl_out, out_count, rbeg, rlen, s_excl[w], s_beg[w]);
-  }
+  });
 }
 
 // --------------------------------------------- balanced vertex worklist ----
