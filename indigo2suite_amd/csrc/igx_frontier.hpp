@@ -117,17 +117,21 @@ __device__ __forceinline__ Entry segq_at(const SegQ& q, const SegPrefix& sp, int
 // the bitmap, one wave per tile: body(v0, bit) with `bit` this lane's vertex
 // v0 + lane.  A wave loads 64 words (2048 vertices) at once and skips empty
 // tiles without further loads, so a sparse frontier costs one coalesced pass
-// over the bitmap.  All lanes of the wave call this together; bits at or past
-// n must be clear.
+// over the bitmap; a bitmap of fewer words than that gives all waves work is
+// read in smaller pieces (300 k vertices are 147 pieces of 64 words for 8192
+// waves: a push round took 180 us).  All lanes of the wave call this together;
+// bits at or past n must be clear.
 template <typename F>
 __device__ __forceinline__ void for_each_bitmap_tile(const unsigned* __restrict__ bits, int n, int gw, int nwaves,
                                                      F body)
 {
   const int lane = lane_id();
   const int nwords = (n + 31) >> 5;
-  for (int wb = gw * kWave; wb < nwords; wb += nwaves * kWave) {  // uniform
+  int piece = kWave;
+  while (piece > 2 && (long long)nwaves * piece > nwords) piece >>= 1;
+  for (int wb = gw * piece; wb < nwords; wb += nwaves * piece) {  // uniform
     const int wi = wb + lane;
-    const unsigned word = (wi < nwords) ? bits[wi] : 0u;
+    const unsigned word = (lane < piece && wi < nwords) ? bits[wi] : 0u;
     const uint64_t nz = ballot(word != 0u);
     uint64_t pair = (nz | (nz >> 1)) & 0x5555555555555555ull;  // even j: word j or j + 1 non-empty
     while (pair != 0) {

@@ -200,12 +200,17 @@ int big_rows(const igx_graph* g, void* bigq, int* d_count);
 
 // Tiles of 64 rows a wave claims at once in the kernels that hand out tiles
 // dynamically: about 4096 edges of work per claim (two tiles on R-MAT 22,
-// sixteen on a 2-D grid), so the shared claim counters stay cold.
+// sixteen on a 2-D grid), so the shared claim counters stay cold, but no more
+// than leaves a claim for every wave of the grid (on 2000 vertices, claims of
+// eight tiles left the whole round to four waves: 30-100 us).
 inline int tile_grab(const igx_graph* g)
 {
   const long long tiles = ((long long)g->nodes + 63) / 64;
-  const long long grab = 4096LL * tiles / (g->edges > 0 ? (long long)g->edges : 1LL);
-  return (int)(grab < 1 ? 1 : (grab > 32 ? 32 : grab));
+  const long long share = tiles / ((long long)rt().persist_blocks * kWavesPerBlock);
+  long long grab = 4096LL * tiles / (g->edges > 0 ? (long long)g->edges : 1LL);
+  if (grab > 32) grab = 32;
+  if (grab > share) grab = share;
+  return (int)(grab < 1 ? 1 : grab);
 }
 
 // events bracketing the timed region

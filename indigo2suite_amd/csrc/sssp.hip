@@ -916,7 +916,9 @@ __global__ void __launch_bounds__(kBlock) sssp_do_round(const int* __restrict__ 
 // Round decision (run by round_finalize after each sssp_do_round).
 struct FinSsspDo {
   long long m;
-  int nblocks;  // the round kernel's grid
+  int nblocks;            // the round kernel's grid
+  long long claims;       // claims of row tiles in a pull round
+  const int* long_chunks; // chunks of long rows
   __device__ void operator()(Ctl* ctl, const RoundTotals& t) const
   {
     const long long ef = t.s[kStatFrontierEdges];
@@ -973,11 +975,15 @@ struct FinSsspDo {
     } else {
       ctl->mode = 0;
     }
-    // a push from a queue (the frontier was small) needs few workgroups:
-    // one per kEdgesPerBlock edges of the frontier, at least 16
+    // a push from a queue (the frontier was small) needs few workgroups: one
+    // per kEdgesPerBlock edges of the frontier, at least 16; a pull needs a
+    // wave per claim of tiles or per two chunks, and every further wave costs
+    // a claim that finds nothing (8192 of them 15-30 us)
     int act = 0;
-    if (!ctl->done && ctl->mode == 0 && ctl->in_bits == 0) {
-      const long long want = (ef + kEdgesPerBlock - 1) / kEdgesPerBlock;
+    if (!ctl->done && (ctl->mode == 1 || ctl->in_bits == 0)) {
+      const long long want = (ctl->mode == 1)
+                                 ? (max(claims, (*long_chunks + 1LL) / 2) + kWavesPerBlock - 1) / kWavesPerBlock
+                                 : (ef + kEdgesPerBlock - 1) / kEdgesPerBlock;
       act = (int)min(max(want, 16LL), (long long)nblocks);
       if (act >= nblocks) act = 0;
     }
@@ -1165,6 +1171,7 @@ int style_do(const igx_graph* g, int src, void* out, const void*, igx_run_info* 
   const long long cap = (long long)g->nodes + g->edges / kChunk + 64;  // chunks of all rows
   const int words = ((g->nodes + kWave - 1) / kWave) * 2;
   const int grab = tile_grab(g);
+  const long long claims = (((long long)g->nodes + kWave - 1) / kWave + grab - 1) / grab;
   void *p0 = nullptr, *p1 = nullptr, *pm = nullptr, *pb = nullptr, *pc = nullptr;
   IGX_TRY(ws_get(WS_D, sizeof(Entry) * (size_t)cap * kGroups, &p0));
   IGX_TRY(ws_get(WS_E, sizeof(Entry) * (size_t)cap * kGroups, &p1));
@@ -1186,7 +1193,7 @@ int style_do(const igx_graph* g, int src, void* out, const void*, igx_run_info* 
                            (const int*)pc, (unsigned*)pm, words, grab, R.d_ctl);
         ktimer_end("sssp_do_round");
         launch_finalize<0xF | (1 << kStatMin) | (3 << kStats)>(R.persist_blocks,
-                        FinSsspDo{(long long)g->edges, R.persist_blocks});
+                        FinSsspDo{(long long)g->edges, R.persist_blocks, claims, (const int*)pc});
       },
       sssp_round_cap(g), &rounds, &launches, 8);
   IGX_TRY(timer_stop(&info->seconds));
