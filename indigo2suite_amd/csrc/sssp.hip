@@ -555,9 +555,10 @@ __global__ void __launch_bounds__(kBlock) sssp_do_round(const int* __restrict__ 
   const SegQ q_out = p ? q0 : q1;
   Entry* q_mine = segq_mine(q_out);
   int* out_count = segq_counter(ctl, p ^ 1, my_group());
-  const unsigned* cur = bm + (size_t)(iter % 3) * words;
-  unsigned* next = bm + (size_t)((iter + 1) % 3) * words;
-  unsigned* stale = bm + (size_t)((iter + 2) % 3) * words;
+  const int turn = iter + ctl->bm_phase;
+  const unsigned* cur = bm + (size_t)(turn % 3) * words;
+  unsigned* next = bm + (size_t)((turn + 1) % 3) * words;
+  unsigned* stale = bm + (size_t)((turn + 2) % 3) * words;
   const int w = threadIdx.x / kWave;
   const int lane = lane_id();
   const int gw = blockIdx.x * kWavesPerBlock + w;
@@ -913,7 +914,7 @@ __global__ void __launch_bounds__(kBlock) sssp_do_round(const int* __restrict__ 
   }
 }
 
-// Round decision (run by round_finalize after each sssp_do_round).
+// Round decision (thread 0 of sssp_do_finish after each sssp_do_round).
 struct FinSsspDo {
   long long m;
   int nblocks;            // the round kernel's grid
@@ -990,6 +991,222 @@ struct FinSsspDo {
     ctl->active = act;
   }
 };
+
+// Ends a round (after_round; the first launch of a run has none to end) and
+// runs the narrow push rounds that follow it: while the frontier has at most
+// kNarrowEdges edges, this one workgroup relaxes them itself, as
+// bfs_do_finish does with levels (a round by launches costs 17-25 us however
+// small its frontier).  The frontier is a list of (edge, source) in LDS.  A
+// vertex enters the next one by the relaxation that found it at its distance
+// of the round's start: the distances of a round are read before a barrier
+// and lowered after it, so that is exactly one, and no mark is needed.  They
+// are read at agent scope, since a copy in the CU's L1 could be older than the
+// workgroup's own atomics.
+//
+// The frontier comes from the queue and goes back to it and to its bitmap; in
+// between the bitmaps are not kept, see bfs_do_finish.  The last narrow round
+// is ended by the same rule as any other (FinSsspDo).  Grid 100 x 100: 205
+// rounds in 3.66 -> 0.83 ms; Erdos-Renyi n = 2000: 353 -> 240 us; R-MAT 22 1.83
+// -> 1.75 ms (its last rounds).
+constexpr int kNarrowEdges = 4096;
+constexpr int kNarrowRounds = 256;  // per launch, so that the host can look at its time limit
+constexpr int kNarrowShift = 21;    // a wave's edges, cut off: 256 * (kNarrowEdges + 1) < 2^21; its vertices above
+typedef int NarrowRow __attribute__((ext_vector_type(2), aligned(4)));  // a row's two offsets in one load
+constexpr int kSsspStats = 0xF | (1 << kStatMin) | (3 << kStats);
+
+__global__ void __launch_bounds__(kFinBlock) sssp_do_finish(const int* __restrict__ nindex,
+                                                             const int* __restrict__ nlist,
+                                                             const int* __restrict__ ew, int* __restrict__ dist, SegQ q0,
+                                                             SegQ q1, unsigned* __restrict__ bm, int words, int nparts,
+                                                             bool after_round, FinSsspDo fin, Ctl* ctl)
+{
+  constexpr int kFinWaves = kFinBlock / kWave;
+  __shared__ int s_edge[2][kNarrowEdges];
+  __shared__ int s_src[2][kNarrowEdges];
+  __shared__ int s_vert[kNarrowEdges];    // vertices of the next frontier (at most one per edge relaxed)
+  __shared__ unsigned long long s_found;  // vertices (high half) and edges of the next frontier
+  __shared__ long long s_low[kFinWaves];
+  __shared__ double s_sum[kFinWaves], s_cnt[kFinWaves];
+  __shared__ int s_edges, s_over, s_chunks, s_go;
+  if (round_done(ctl)) return;
+  const int tid = threadIdx.x;
+  const int lane = lane_id();
+  if (after_round) {
+    const RoundTotals tot = round_totals<kSsspStats>(ctl, nparts);
+    if (tid == 0) fin(ctl, tot);
+  }
+  if (tid == 0) {
+    s_go = !ctl->done && ctl->mode == 0 && ctl->in_bits == 0 && ctl->push_cut == 0 && ctl->edges_next <= kNarrowEdges;
+    s_edges = 0;
+    s_chunks = 0;
+  }
+  __syncthreads();
+  if (!s_go) return;
+  const int iter0 = ctl->iter;
+  const int phase0 = ctl->bm_phase;
+  unsigned* cur = bm + (size_t)((iter0 + phase0) % 3) * words;
+  {
+    const SegQ q_in = (iter0 & 1) ? q1 : q0;
+    const SegPrefix pre = segq_prefix(ctl, iter0 & 1);
+    for (int i = tid; i < pre.pre[kGroups]; i += kFinBlock) {
+      const Entry en = segq_at(q_in, pre, i);
+      cur[en.v >> 5] = 0u;
+      const int len = en.end - en.beg;
+      const int at = atomicAdd(&s_edges, len);
+      for (int k = 0; k < len; k++) {
+        s_edge[0][at + k] = en.beg + k;
+        s_src[0][at + k] = en.v;
+      }
+    }
+  }
+  __syncthreads();
+  int count = s_edges;   // edges of the current frontier
+  int next = 0;          // of the next one
+  int found = 0;         // its vertices
+  int rounds = 0;
+  long long scanned = 0, rows = 0;  // of the rounds before the last
+  long long low = LLONG_MAX;
+  double lsum = 0.0, lcnt = 0.0;
+  for (;;) {  // uniform
+    if (tid == 0) {
+      s_found = 0;
+      s_over = 0;
+    }
+    const int* in_e = s_edge[rounds & 1];
+    const int* in_v = s_src[rounds & 1];
+    int* out_e = s_edge[(rounds & 1) ^ 1];
+    int* out_v = s_src[(rounds & 1) ^ 1];
+    constexpr int kPer = kNarrowEdges / kFinBlock;
+    int u[kPer], nd[kPer], d[kPer];
+    #pragma unroll
+    for (int k = 0; k < kPer; k++) {
+      const int i = k * kFinBlock + tid;
+      u[k] = -1;
+      nd[k] = 0;
+      if (i < count) {
+        const int e = in_e[i];
+        u[k] = nlist[e];
+        nd[k] = load_relaxed(&dist[in_v[i]]) + ew[e];
+      }
+    }
+    #pragma unroll
+    for (int k = 0; k < kPer; k++) d[k] = (u[k] >= 0) ? load_relaxed(&dist[u[k]]) : INT_MIN;
+    __syncthreads();  // every distance of the round is read before one is lowered
+    low = LLONG_MAX;
+    lsum = lcnt = 0.0;
+    bool won[kPer];
+    #pragma unroll
+    for (int k = 0; k < kPer; k++) {
+      won[k] = false;
+      if (d[k] > nd[k]) {
+        const int old = atomic_min_relaxed(&dist[u[k]], nd[k]);
+        if (old > nd[k]) {
+          low = min(low, (long long)nd[k]);
+          lsum += nd[k];
+          lcnt += 1.0;
+        }
+        won[k] = old == d[k];
+      }
+    }
+    NarrowRow row[kPer];
+    #pragma unroll
+    for (int k = 0; k < kPer; k++) row[k] = won[k] ? *(const NarrowRow*)(nindex + u[k]) : NarrowRow{0, 0};
+    // places for the thread's vertices and their edges: one scan and one LDS
+    // atomic per wave, of (vertices, edges) in one number; lengths enter it
+    // cut off just above kNarrowEdges, what is cut goes to s_over
+    unsigned mine = 0;
+    #pragma unroll
+    for (int k = 0; k < kPer; k++) {
+      const int len = row[k][1] - row[k][0];
+      if (won[k]) mine += (1u << kNarrowShift) + (unsigned)min(len, kNarrowEdges + 1);
+      if (len > kNarrowEdges + 1) atomicAdd(&s_over, len - (kNarrowEdges + 1));
+    }
+    if (ballot(mine != 0) != 0) {
+      const unsigned incl = (unsigned)wave_incl_scan((int)mine);
+      unsigned long long base = 0;
+      if (lane == kWave - 1) {
+        base = atomicAdd(&s_found, ((unsigned long long)(incl >> kNarrowShift) << 32) |
+                                       (incl & ((1u << kNarrowShift) - 1u)));
+      }
+      base = __shfl(base, kWave - 1, kWave);
+      const unsigned excl = incl - mine;
+      int vat = (int)(base >> 32) + (int)(excl >> kNarrowShift);
+      int eat = (int)(base & 0xffffffffull) + (int)(excl & ((1u << kNarrowShift) - 1u));
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) {
+        if (!won[k]) continue;
+        s_vert[vat++] = u[k];
+        const int len = min(row[k][1] - row[k][0], kNarrowEdges + 1);
+        if (eat <= kNarrowEdges - len) {  // else the frontier is not narrow: the list is not used
+          for (int j = 0; j < len; j++) {
+            out_e[eat + j] = row[k][0] + j;
+            out_v[eat + j] = u[k];
+          }
+        }
+        eat += len;
+      }
+    }
+    __syncthreads();
+    next = (int)(s_found & 0xffffffffull) + s_over;
+    found = (int)(s_found >> 32);
+    __syncthreads();
+    rounds++;
+    if (next == 0 || next > kNarrowEdges || rounds >= kNarrowRounds) break;
+    scanned += count;
+    rows += found;
+    count = next;
+  }
+  // the last round's statistics, as a round kernel would leave them
+  low = wave_min_ll(low);
+  lsum = wave_sum_d(lsum);
+  lcnt = wave_sum_d(lcnt);
+  if (lane == 0) {
+    s_low[tid / kWave] = low;
+    s_sum[tid / kWave] = lsum;
+    s_cnt[tid / kWave] = lcnt;
+  }
+  __syncthreads();
+  const int iter1 = iter0 + rounds;
+  if (next != 0) {
+    const SegQ q = (iter1 & 1) ? q1 : q0;
+    for (int i = tid; i < found; i += kFinBlock) {
+      const int v = s_vert[i];
+      const int vb = nindex[v], ve = nindex[v + 1];
+      atomicOr(&cur[v >> 5], 1u << (v & 31));
+      const int c = chunks_of(ve - vb);
+      const int at = atomicAdd(&s_chunks, c);
+      for (int k = 0; k < c; k++) {
+        const int x = vb + k * kChunk;
+        q.base[at + k] = Entry{v, x, (x + kChunk < ve) ? x + kChunk : ve, 0};
+      }
+    }
+  }
+  if (tid < kGroups) {
+    ctl_groups(ctl)[tid].qcount[0] = 0;
+    ctl_groups(ctl)[tid].qcount[1] = 0;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    RoundTotals t = {};
+    t.s[kStatFrontierEdges] = next;
+    t.s[kStatScanned] = t.s[kStatRelaxed] = count;
+    t.s[kStatRows] = found;
+    t.s[kStatMin] = LLONG_MAX;
+    for (int k = 0; k < kFinWaves; k++) {
+      t.s[kStatMin] = min(t.s[kStatMin], s_low[k]);
+      t.d[0] += s_sum[k];
+      t.d[1] += s_cnt[k];
+    }
+    ctl->work_edges += scanned;
+    ctl->aux_ll[0] += scanned;
+    ctl->work_vertices += rows;
+    ctl->iter = iter1 - 1;
+    ctl->edges_next = count;
+    ctl->bm_phase = (phase0 + 2 * rounds) % 3;  // iter + bm_phase stays the same modulo 3
+    fin(ctl, t);
+    ctl_groups(ctl)[0].qcount[iter1 & 1] = s_chunks;
+  }
+}
 
 // ------------------------------------------------------------ host side ----
 template <typename K>
@@ -1184,6 +1401,12 @@ int style_do(const igx_graph* g, int src, void* out, const void*, igx_run_info* 
   hipLaunchKernelGGL(sssp_do_init, dim3(blocks_for(g->nodes, kBlock)), dim3(kBlock), 0, R.stream, src, g->nindex,
                      g->nodes, dist, (Entry*)p0, (unsigned*)pm, words, R.d_ctl);
   IGX_TRY(big_rows(g, pb, (int*)pc));
+  const FinSsspDo fin{(long long)g->edges, R.persist_blocks, claims, (const int*)pc};
+  auto finish = [&](bool after_round) {
+    hipLaunchKernelGGL(sssp_do_finish, dim3(1), dim3(kFinBlock), 0, R.stream, g->nindex, g->nlist, g->eweight, dist,
+                       q0, q1, (unsigned*)pm, words, R.persist_blocks, after_round, fin, R.d_ctl);
+  };
+  finish(false);
   int rounds = 0, launches = 0;
   const int rc = run_rounds(
       [&](long long) {
@@ -1192,8 +1415,7 @@ int style_do(const igx_graph* g, int src, void* out, const void*, igx_run_info* 
                            g->eweight, g->nodes, (long long)g->edges, dist, q0, q1, (const Entry*)pb,
                            (const int*)pc, (unsigned*)pm, words, grab, R.d_ctl);
         ktimer_end("sssp_do_round");
-        launch_finalize<0xF | (1 << kStatMin) | (3 << kStats)>(R.persist_blocks,
-                        FinSsspDo{(long long)g->edges, R.persist_blocks, claims, (const int*)pc});
+        finish(true);
       },
       sssp_round_cap(g), &rounds, &launches, 8);
   IGX_TRY(timer_stop(&info->seconds));
