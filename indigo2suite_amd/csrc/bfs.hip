@@ -309,7 +309,7 @@ constexpr long long kQueueEdges = 1 << 16;
 // after kNarrowLevels levels, so that the host can look at its time limit.
 // Levels from a queue above the limit run on few workgroups, one per
 // kLevelEdges edges.  Grid 1024 x 1024, whole run: 21.3 -> 11.0 ms.
-constexpr int kNarrowEdges = 4096;
+constexpr int kNarrowEdges = 4 * kFinBlock;
 constexpr int kNarrowLevels = 512;
 constexpr long long kLevelEdges = 256;  // frontier edges per workgroup of a level from a queue
 constexpr int kNarrowShift = 21;  // a wave's edges, cut off: 256 * (kNarrowEdges + 1) < 2^21; its vertices above
@@ -621,62 +621,65 @@ __global__ void __launch_bounds__(kFinBlock) bfs_do_finish(const int* __restrict
     const int* in = s_edge[(level - level0) & 1];
     int* out = s_edge[((level - level0) & 1) ^ 1];
     const int nd = level + 1;
-    constexpr int kPer = kNarrowEdges / kFinBlock;
-    int u[kPer], d[kPer];
-    #pragma unroll
-    for (int k = 0; k < kPer; k++) {
-      const int i = k * kFinBlock + tid;
-      u[k] = (i < count) ? nlist[in[i]] : -1;
-    }
-    #pragma unroll
-    for (int k = 0; k < kPer; k++) d[k] = (u[k] >= 0) ? dist[u[k]] : 0;
-    bool won[kPer];
-    #pragma unroll
-    for (int k = 0; k < kPer; k++) {
-      won[k] = false;
-      if (d[k] == kInf) {
-        int expected = kInf;
-        won[k] = __hip_atomic_compare_exchange_strong(&dist[u[k]], &expected, nd, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                      __HIP_MEMORY_SCOPE_AGENT);
-      }
-    }
-    // the rows of the winners only: one CU takes in about one cache line a
-    // cycle, and with thousands of scattered edges that rate is the level's time
-    NarrowRow row[kPer];
-    #pragma unroll
-    for (int k = 0; k < kPer; k++) row[k] = won[k] ? *(const NarrowRow*)(nindex + u[k]) : NarrowRow{0, 0};
-    // places for the thread's winners and their edges: one scan and one LDS
-    // atomic per wave, of (winners, edges) in one number; lengths enter it cut
-    // off just above kNarrowEdges, what is cut goes to s_over
-    unsigned mine = 0;
-    #pragma unroll
-    for (int k = 0; k < kPer; k++) {
-      const int len = row[k][1] - row[k][0];
-      if (won[k]) mine += (1u << kNarrowShift) + (unsigned)min(len, kNarrowEdges + 1);
-      if (len > kNarrowEdges + 1) atomicAdd(&s_over, len - (kNarrowEdges + 1));
-    }
-    if (ballot(mine != 0) != 0) {
-      const unsigned incl = (unsigned)wave_incl_scan((int)mine);
-      unsigned long long base = 0;
-      if (lane_id() == kWave - 1) {
-        base = atomicAdd(&s_found, ((unsigned long long)(incl >> kNarrowShift) << 32) |
-                                       (incl & ((1u << kNarrowShift) - 1u)));
-      }
-      base = __shfl(base, kWave - 1, kWave);
-      const unsigned excl = incl - mine;
-      int vat = (int)(base >> 32) + (int)(excl >> kNarrowShift);
-      int eat = (int)(base & 0xffffffffull) + (int)(excl & ((1u << kNarrowShift) - 1u));
+    with_narrow_items(count, [&](auto items) {
+      constexpr int kPer = decltype(items)::value;
+      if ((tid & ~(kWave - 1)) >= count) return;  // uniform per wave
+      int u[kPer], d[kPer];
       #pragma unroll
       for (int k = 0; k < kPer; k++) {
-        if (!won[k]) continue;
-        s_vert[vat++] = u[k];
-        const int len = min(row[k][1] - row[k][0], kNarrowEdges + 1);
-        if (eat <= kNarrowEdges - len) {  // else the frontier is not narrow: the list is not used
-          for (int j = 0; j < len; j++) out[eat + j] = row[k][0] + j;
-        }
-        eat += len;
+        const int i = k * kFinBlock + tid;
+        u[k] = (i < count) ? nlist[in[i]] : -1;
       }
-    }
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) d[k] = (u[k] >= 0) ? dist[u[k]] : 0;
+      bool won[kPer];
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) {
+        won[k] = false;
+        if (d[k] == kInf) {
+          int expected = kInf;
+          won[k] = __hip_atomic_compare_exchange_strong(&dist[u[k]], &expected, nd, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_AGENT);
+        }
+      }
+      // the rows of the winners only: one CU takes in about one cache line a
+      // cycle, and with thousands of scattered edges that rate is the level's time
+      NarrowRow row[kPer];
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) row[k] = won[k] ? *(const NarrowRow*)(nindex + u[k]) : NarrowRow{0, 0};
+      // places for the thread's winners and their edges: one scan and one LDS
+      // atomic per wave, of (winners, edges) in one number; lengths enter it cut
+      // off just above kNarrowEdges, what is cut goes to s_over
+      unsigned mine = 0;
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) {
+        const int len = row[k][1] - row[k][0];
+        if (won[k]) mine += (1u << kNarrowShift) + (unsigned)min(len, kNarrowEdges + 1);
+        if (len > kNarrowEdges + 1) atomicAdd(&s_over, len - (kNarrowEdges + 1));
+      }
+      if (ballot(mine != 0) != 0) {
+        const unsigned incl = (unsigned)wave_incl_scan((int)mine);
+        unsigned long long base = 0;
+        if (lane_id() == kWave - 1) {
+          base = atomicAdd(&s_found, ((unsigned long long)(incl >> kNarrowShift) << 32) |
+                                         (incl & ((1u << kNarrowShift) - 1u)));
+        }
+        base = __shfl(base, kWave - 1, kWave);
+        const unsigned excl = incl - mine;
+        int vat = (int)(base >> 32) + (int)(excl >> kNarrowShift);
+        int eat = (int)(base & 0xffffffffull) + (int)(excl & ((1u << kNarrowShift) - 1u));
+        #pragma unroll
+        for (int k = 0; k < kPer; k++) {
+          if (!won[k]) continue;
+          s_vert[vat++] = u[k];
+          const int len = min(row[k][1] - row[k][0], kNarrowEdges + 1);
+          if (eat <= kNarrowEdges - len) {  // else the frontier is not narrow: the list is not used
+            for (int j = 0; j < len; j++) out[eat + j] = row[k][0] + j;
+          }
+          eat += len;
+        }
+      }
+    });
     __syncthreads();
     count = (int)(s_found & 0xffffffffull) + s_over;
     found = (int)(s_found >> 32);

@@ -164,6 +164,18 @@ __device__ __forceinline__ void with_list_items(int per, F body)
   else body(std::integral_constant<int, kListPer>{});
 }
 
+// Edges per thread of a narrow level or round (bfs_do_finish, sssp_do_finish),
+// as a constant for the loops over them.  One workgroup's instructions are much
+// of the time of such a level, so no thread goes through the loops for edges
+// that are not there.
+template <typename F>
+__device__ __forceinline__ void with_narrow_items(int count, F body)
+{
+  if (count <= kFinBlock) body(std::integral_constant<int, 1>{});
+  else if (count <= 2 * kFinBlock) body(std::integral_constant<int, 2>{});
+  else body(std::integral_constant<int, 4>{});
+}
+
 // LDS of block_push_edge_ranges
 struct ListLds {
   int excl[kWavesPerBlock][kWave];

@@ -1008,7 +1008,7 @@ struct FinSsspDo {
 // is ended by the same rule as any other (FinSsspDo).  Grid 100 x 100: 205
 // rounds in 3.66 -> 0.83 ms; Erdos-Renyi n = 2000: 353 -> 240 us; R-MAT 22 1.83
 // -> 1.75 ms (its last rounds).
-constexpr int kNarrowEdges = 4096;
+constexpr int kNarrowEdges = 4 * kFinBlock;
 constexpr int kNarrowRounds = 256;  // per launch, so that the host can look at its time limit
 constexpr int kNarrowShift = 21;    // a wave's edges, cut off: 256 * (kNarrowEdges + 1) < 2^21; its vertices above
 typedef int NarrowRow __attribute__((ext_vector_type(2), aligned(4)));  // a row's two offsets in one load
@@ -1076,76 +1076,79 @@ __global__ void __launch_bounds__(kFinBlock) sssp_do_finish(const int* __restric
     const int* in_v = s_src[rounds & 1];
     int* out_e = s_edge[(rounds & 1) ^ 1];
     int* out_v = s_src[(rounds & 1) ^ 1];
-    constexpr int kPer = kNarrowEdges / kFinBlock;
-    int u[kPer], nd[kPer], d[kPer];
-    #pragma unroll
-    for (int k = 0; k < kPer; k++) {
-      const int i = k * kFinBlock + tid;
-      u[k] = -1;
-      nd[k] = 0;
-      if (i < count) {
-        const int e = in_e[i];
-        u[k] = nlist[e];
-        nd[k] = load_relaxed(&dist[in_v[i]]) + ew[e];
-      }
-    }
-    #pragma unroll
-    for (int k = 0; k < kPer; k++) d[k] = (u[k] >= 0) ? load_relaxed(&dist[u[k]]) : INT_MIN;
-    __syncthreads();  // every distance of the round is read before one is lowered
-    low = LLONG_MAX;
-    lsum = lcnt = 0.0;
-    bool won[kPer];
-    #pragma unroll
-    for (int k = 0; k < kPer; k++) {
-      won[k] = false;
-      if (d[k] > nd[k]) {
-        const int old = atomic_min_relaxed(&dist[u[k]], nd[k]);
-        if (old > nd[k]) {
-          low = min(low, (long long)nd[k]);
-          lsum += nd[k];
-          lcnt += 1.0;
-        }
-        won[k] = old == d[k];
-      }
-    }
-    NarrowRow row[kPer];
-    #pragma unroll
-    for (int k = 0; k < kPer; k++) row[k] = won[k] ? *(const NarrowRow*)(nindex + u[k]) : NarrowRow{0, 0};
-    // places for the thread's vertices and their edges: one scan and one LDS
-    // atomic per wave, of (vertices, edges) in one number; lengths enter it
-    // cut off just above kNarrowEdges, what is cut goes to s_over
-    unsigned mine = 0;
-    #pragma unroll
-    for (int k = 0; k < kPer; k++) {
-      const int len = row[k][1] - row[k][0];
-      if (won[k]) mine += (1u << kNarrowShift) + (unsigned)min(len, kNarrowEdges + 1);
-      if (len > kNarrowEdges + 1) atomicAdd(&s_over, len - (kNarrowEdges + 1));
-    }
-    if (ballot(mine != 0) != 0) {
-      const unsigned incl = (unsigned)wave_incl_scan((int)mine);
-      unsigned long long base = 0;
-      if (lane == kWave - 1) {
-        base = atomicAdd(&s_found, ((unsigned long long)(incl >> kNarrowShift) << 32) |
-                                       (incl & ((1u << kNarrowShift) - 1u)));
-      }
-      base = __shfl(base, kWave - 1, kWave);
-      const unsigned excl = incl - mine;
-      int vat = (int)(base >> 32) + (int)(excl >> kNarrowShift);
-      int eat = (int)(base & 0xffffffffull) + (int)(excl & ((1u << kNarrowShift) - 1u));
+    with_narrow_items(count, [&](auto items) {
+      constexpr int kPer = decltype(items)::value;
+      int u[kPer], nd[kPer], d[kPer];
       #pragma unroll
       for (int k = 0; k < kPer; k++) {
-        if (!won[k]) continue;
-        s_vert[vat++] = u[k];
-        const int len = min(row[k][1] - row[k][0], kNarrowEdges + 1);
-        if (eat <= kNarrowEdges - len) {  // else the frontier is not narrow: the list is not used
-          for (int j = 0; j < len; j++) {
-            out_e[eat + j] = row[k][0] + j;
-            out_v[eat + j] = u[k];
-          }
+        const int i = k * kFinBlock + tid;
+        u[k] = -1;
+        nd[k] = 0;
+        if (i < count) {
+          const int e = in_e[i];
+          u[k] = nlist[e];
+          nd[k] = load_relaxed(&dist[in_v[i]]) + ew[e];
         }
-        eat += len;
       }
-    }
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) d[k] = (u[k] >= 0) ? load_relaxed(&dist[u[k]]) : INT_MIN;
+      __syncthreads();  // every distance of the round is read before one is lowered
+      low = LLONG_MAX;
+      lsum = lcnt = 0.0;
+      if ((tid & ~(kWave - 1)) >= count) return;  // uniform per wave
+      bool won[kPer];
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) {
+        won[k] = false;
+        if (d[k] > nd[k]) {
+          const int old = atomic_min_relaxed(&dist[u[k]], nd[k]);
+          if (old > nd[k]) {
+            low = min(low, (long long)nd[k]);
+            lsum += nd[k];
+            lcnt += 1.0;
+          }
+          won[k] = old == d[k];
+        }
+      }
+      NarrowRow row[kPer];
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) row[k] = won[k] ? *(const NarrowRow*)(nindex + u[k]) : NarrowRow{0, 0};
+      // places for the thread's vertices and their edges: one scan and one LDS
+      // atomic per wave, of (vertices, edges) in one number; lengths enter it
+      // cut off just above kNarrowEdges, what is cut goes to s_over
+      unsigned mine = 0;
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) {
+        const int len = row[k][1] - row[k][0];
+        if (won[k]) mine += (1u << kNarrowShift) + (unsigned)min(len, kNarrowEdges + 1);
+        if (len > kNarrowEdges + 1) atomicAdd(&s_over, len - (kNarrowEdges + 1));
+      }
+      if (ballot(mine != 0) != 0) {
+        const unsigned incl = (unsigned)wave_incl_scan((int)mine);
+        unsigned long long base = 0;
+        if (lane == kWave - 1) {
+          base = atomicAdd(&s_found, ((unsigned long long)(incl >> kNarrowShift) << 32) |
+                                         (incl & ((1u << kNarrowShift) - 1u)));
+        }
+        base = __shfl(base, kWave - 1, kWave);
+        const unsigned excl = incl - mine;
+        int vat = (int)(base >> 32) + (int)(excl >> kNarrowShift);
+        int eat = (int)(base & 0xffffffffull) + (int)(excl & ((1u << kNarrowShift) - 1u));
+        #pragma unroll
+        for (int k = 0; k < kPer; k++) {
+          if (!won[k]) continue;
+          s_vert[vat++] = u[k];
+          const int len = min(row[k][1] - row[k][0], kNarrowEdges + 1);
+          if (eat <= kNarrowEdges - len) {  // else the frontier is not narrow: the list is not used
+            for (int j = 0; j < len; j++) {
+              out_e[eat + j] = row[k][0] + j;
+              out_v[eat + j] = u[k];
+            }
+          }
+          eat += len;
+        }
+      }
+    });
     __syncthreads();
     next = (int)(s_found & 0xffffffffull) + s_over;
     found = (int)(s_found >> 32);
