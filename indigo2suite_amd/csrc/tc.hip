@@ -223,14 +223,15 @@ __global__ void __launch_bounds__(kBlock) tc_edge_bsearch(const int* __restrict_
 //
 // Whole call, before (one wave per vertex hashing N+(v) and probing the lists
 // of its out-neighbours, orientation by a row map, flags and a scan over the
-// edges) and now: R-MAT 20 (n = 1,048,576, m = 31.4 M) 38.4 -> 3.7 ms;
+// edges) and now: R-MAT 20 (n = 1,048,576, m = 31.4 M) 38.4 -> 2.0 ms;
 // Erdos-Renyi n = 2,097,152, average degree 16: 2.76 -> 1.27 ms.
 constexpr int kTcWords = kEdgeTile / kWave;      // keep-bit words per tile
 constexpr int kTcShort = 32;                     // lists up to this length: 16-byte groups against a list in LDS
 constexpr int kTcBitWords = 4096;                // bitmap of 2^17 ranks, 16 KB
 constexpr int kTcHashSlice = kTcBitWords / 4;    // list elements per pass where ranks exceed the bitmap
 constexpr int kTcPad = 128;                      // ints that 16-byte reads may pass the end of a list array
-constexpr int kTcClaim = 4;                      // ranks per claim of the count
+constexpr int kTcSingle = 32768;                 // ranks claimed one by one by the count; beyond, kTcClaim at once
+constexpr int kTcClaim = 8;
 constexpr int kTcClaimStride = 64;               // ints between the groups' claim counters
 constexpr int kTcShortRows = 32;                 // rows per wave step of the short count
 
@@ -348,7 +349,8 @@ __global__ void __launch_bounds__(kBlock) tc_orient(const int* __restrict__ nind
 
 // Edges with an endpoint whose list is longer than kTcShort, at the endpoint
 // x with the longer list (ties: the larger id), one workgroup per x in rank
-// order, hubs first.  All neighbours y of x are looked at; those with the
+// order, hubs first, claimed one at a time while they are heavy (four hubs at
+// a time were up to 3.4 times a workgroup's share of R-MAT 20).  All neighbours y of x are looked at; those with the
 // shorter list stream it past the set of x, 16 lanes a list and four
 // consecutive elements a lane, so a step of a wave tests 256 elements and
 // needs no search for their owner.  The set is a bitmap of ranks in LDS
@@ -356,7 +358,7 @@ __global__ void __launch_bounds__(kBlock) tc_orient(const int* __restrict__ nind
 // bits, an exact hash set of slices of N+(x) in the same 16 KB, at most a
 // quarter full.  On R-MAT 20 99.9% of the probes meet the bitmap.  Between
 // two x the LDS words are all zero (both forms clear what they set).
-// R-MAT 20: 36.8 -> 3.24 ms for the count.
+// R-MAT 20: 36.8 -> 1.6 ms for the count (3.24 ms with four ranks a claim).
 __global__ void __launch_bounds__(kBlock) tc_count_long(const int* __restrict__ nindex, const int* __restrict__ nlist,
                                                          const int* __restrict__ order,
                                                          const int* __restrict__ heavy,
@@ -380,9 +382,11 @@ __global__ void __launch_bounds__(kBlock) tc_count_long(const int* __restrict__ 
     if (tid == 0) s_claim = atomicAdd(next, 1);
     __syncthreads();
     const long long unit = grp + (long long)s_claim * kGroups;
-    if (unit * kTcClaim >= total) break;
-    for (int q = 0; q < kTcClaim; q++) {
-      const int rx = (int)(unit * kTcClaim) + q;
+    const long long rank0 = (unit < kTcSingle) ? unit : kTcSingle + (unit - kTcSingle) * kTcClaim;
+    const int ranks = (unit < kTcSingle) ? 1 : kTcClaim;
+    if (rank0 >= total) break;
+    for (int q = 0; q < ranks; q++) {
+      const int rx = (int)rank0 + q;
       if (rx >= total) break;
       const int x = order[rx];
       const int beg = onidx[x], len = onidx[x + 1] - beg;
