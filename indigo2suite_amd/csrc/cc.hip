@@ -290,21 +290,37 @@ __device__ __forceinline__ int uf_find(int* __restrict__ parent, int x)
   }
 }
 
-__device__ __forceinline__ void uf_unite(int* __restrict__ parent, int a, int b)
+// Link the larger of two roots under the smaller, from `ra` and `rb`, the roots
+// that the finds returned.  The finds read plainly, so a root may have been
+// linked by another XCD since this one's L2 took its copy, and in a graph that
+// is nearly one component everybody arrives at the same few stale roots: a
+// compare-and-swap each, one address, 15 ns apiece (Erdos-Renyi n = 1 M: 1.86
+// of 1.90 ms).  So the root is looked at past the caches first, and what was
+// found is stored back plainly: a true parent of a vertex that is no root any
+// more, which refreshes this XCD's copy for those who come after.
+__device__ __forceinline__ void uf_link_roots(int* __restrict__ parent, int ra, int rb)
 {
-  int ra = uf_find(parent, a);
-  int rb = uf_find(parent, b);
   while (ra != rb) {
     const int hi = max(ra, rb), lo = min(ra, rb);
-    int expected = hi;
-    if (__hip_atomic_compare_exchange_strong(&parent[hi], &expected, lo, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT)) {
-      return;
+    int now = load_relaxed(&parent[hi]);
+    if (now == hi) {
+      if (__hip_atomic_compare_exchange_strong(&parent[hi], &now, lo, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT)) {
+        return;
+      }
+      // hi was linked meanwhile: `now` holds its current parent
     }
-    // hi was linked meanwhile: `expected` holds its current parent
-    ra = uf_find(parent, expected);
+    parent[hi] = now;
+    ra = uf_find(parent, now);
     rb = uf_find(parent, lo);
   }
+}
+
+__device__ __forceinline__ void uf_unite(int* __restrict__ parent, int a, int b)
+{
+  const int ra = uf_find(parent, a);
+  const int rb = uf_find(parent, b);
+  uf_link_roots(parent, ra, rb);
 }
 
 // parent[v] = the first neighbour if it is smaller (else v).
@@ -392,18 +408,9 @@ __global__ void __launch_bounds__(kBlock) uf_hook(const int* __restrict__ nindex
       for (int k = 0; k < kIlp; k++) {
         if (!need[k]) continue;
         // two levels are resolved above; deeper trees fall back to the loop
-        int ru = (pu[k] == u[k]) ? u[k] : ((ppu[k] == pu[k]) ? pu[k] : uf_find(parent, ppu[k]));
-        int ra = (ph[k] == hint[k]) ? hint[k] : uf_find(parent, ph[k]);
-        while (ra != ru) {
-          const int hi2 = max(ra, ru), lo2 = min(ra, ru);
-          int expected = hi2;
-          if (__hip_atomic_compare_exchange_strong(&parent[hi2], &expected, lo2, __ATOMIC_RELAXED,
-                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-            break;
-          }
-          ra = uf_find(parent, expected);
-          ru = uf_find(parent, lo2);
-        }
+        const int ru = (pu[k] == u[k]) ? u[k] : ((ppu[k] == pu[k]) ? pu[k] : uf_find(parent, ppu[k]));
+        const int ra = (ph[k] == hint[k]) ? hint[k] : uf_find(parent, ph[k]);
+        uf_link_roots(parent, ra, ru);
       }
     }
     __builtin_amdgcn_wave_barrier();
