@@ -311,6 +311,7 @@ constexpr long long kQueueEdges = 1 << 16;
 // kLevelEdges edges.  Grid 1024 x 1024, whole run: 21.3 -> 11.0 ms.
 constexpr int kNarrowEdges = 4 * kFinBlock;
 constexpr int kNarrowLevels = 512;
+constexpr int kFewEdges = 1 << 20;  // graphs below it seldom need more than four levels beyond the narrow ones
 constexpr long long kLevelEdges = 256;  // frontier edges per workgroup of a level from a queue
 constexpr int kNarrowShift = 21;  // a wave's edges, cut off: 256 * (kNarrowEdges + 1) < 2^21; its vertices above
 typedef int NarrowRow __attribute__((ext_vector_type(2), aligned(4)));  // a row's two offsets in one load
@@ -357,7 +358,8 @@ __global__ void __launch_bounds__(kBlock) bfs_do_level(const int* __restrict__ n
                                                         int* __restrict__ dist, SegQ q0, SegQ q1,
                                                         const Entry* __restrict__ bigq,
                                                         const int* __restrict__ bigq_count,
-                                                        unsigned* __restrict__ bm, int words, Ctl* ctl)
+                                                        unsigned* __restrict__ bm, int words, bool short_rows,
+                                                        Ctl* ctl)
 {
   __shared__ int s_excl[kWavesPerBlock][kWave];
   __shared__ Entry s_ent[kWavesPerBlock][kWave];
@@ -456,70 +458,96 @@ __global__ void __launch_bounds__(kBlock) bfs_do_level(const int* __restrict__ n
     }
   } else {
     // kSub 64-vertex sub-tiles per step, their loads issued together (the
-    // chain dist -> row -> first neighbours -> frontier bits is latency-bound)
+    // chain dist -> row -> first neighbours -> frontier bits is latency-bound),
+    // side by side on a large graph and one grid apart on a small one, so that
+    // every wave has some.  Rows that go on: by their lanes, kStep neighbours
+    // at once up to kLaneRow, and only the rest by the wave, one after the
+    // other (Erdos-Renyi n = 20 k, average degree 8, all by the wave: the whole
+    // run 158 us, 97 us this way); on a large graph with long rows, where few
+    // go past the first four, by the wave at once (R-MAT 22 219 -> 217 us)
     constexpr int kFirst = 4;
     constexpr int kSub = 4;
-    for (int base = gw * kWave * kSub; base < n; base += nwaves * kWave * kSub) {
-      bool unvisited[kSub], found[kSub];
-      int ub[kSub], ue[kSub];
-      #pragma unroll
-      for (int s = 0; s < kSub; s++) {
-        const int u = base + s * kWave + lane;
-        unvisited[s] = (u < n) && dist[u] == kInf;
-        found[s] = false;
-        ub[s] = ue[s] = 0;
-      }
-      #pragma unroll
-      for (int s = 0; s < kSub; s++) {
-        const int u = base + s * kWave + lane;
-        if (unvisited[s]) {
-          ub[s] = nindex[u];
-          ue[s] = nindex[u + 1];
+    constexpr int kStep = 4;
+    constexpr int kLaneRow = 36;
+    const int ntiles = (n + kWave - 1) / kWave;
+    auto bottom_up = [&](auto dense) {
+      constexpr bool kDense = decltype(dense)::value;
+      const int apart = kDense ? 1 : nwaves;
+      const bool by_lanes = !kDense || short_rows;
+      for (int tile0 = gw * (kDense ? kSub : 1); tile0 < ntiles; tile0 += nwaves * kSub) {  // uniform per wave
+        bool unvisited[kSub], found[kSub];
+        int ub[kSub], ue[kSub];
+        #pragma unroll
+        for (int s = 0; s < kSub; s++) {
+          const long long u = ((long long)tile0 + (long long)s * apart) * kWave + lane;
+          unvisited[s] = (u < n) && dist[u] == kInf;
+          found[s] = false;
+          ub[s] = ue[s] = 0;
         }
-      }
-      int nb[kSub][kFirst];
-      #pragma unroll
-      for (int s = 0; s < kSub; s++) {
         #pragma unroll
-        for (int k = 0; k < kFirst; k++) nb[s][k] = (unvisited[s] && ub[s] + k < ue[s]) ? nlist[ub[s] + k] : -1;
-      }
-      #pragma unroll
-      for (int s = 0; s < kSub; s++) {
-        #pragma unroll
-        for (int k = 0; k < kFirst; k++) found[s] = found[s] || (nb[s][k] >= 0 && in_bits(cur, nb[s][k]));
-      }
-      #pragma unroll
-      for (int s = 0; s < kSub; s++) {
-        if (base + s * kWave >= n) break;  // uniform
-        uint64_t pending = ballot(unvisited[s] && !found[s] && ue[s] - ub[s] > kFirst);
-        while (pending != 0) {
-          const int L = __ffsll((unsigned long long)pending) - 1;
-          pending &= pending - 1;
-          const int s0 = __shfl(ub[s], L, kWave) + kFirst;
-          const int e0 = __shfl(ue[s], L, kWave);
-          bool hit = false;
-          for (int i0 = s0; i0 < e0; i0 += kWave) {
-            const int i = i0 + lane;
-            const bool h = (i < e0) && in_bits(cur, nlist[i]);
-            if (ballot(h) != 0) {
-              hit = true;
-              break;
-            }
+        for (int s = 0; s < kSub; s++) {
+          const long long u = ((long long)tile0 + (long long)s * apart) * kWave + lane;
+          if (unvisited[s]) {
+            ub[s] = nindex[u];
+            ue[s] = nindex[u + 1];
           }
-          if (lane == L) found[s] = hit;
         }
-        const int u = base + s * kWave + lane;
-        if (found[s]) {
-          dist[u] = nd;
-          found_v += 1;
-          found_e += ue[s] - ub[s];
+        int nb[kSub][kFirst];
+        #pragma unroll
+        for (int s = 0; s < kSub; s++) {
+          #pragma unroll
+          for (int k = 0; k < kFirst; k++) nb[s][k] = (unvisited[s] && ub[s] + k < ue[s]) ? nlist[ub[s] + k] : -1;
         }
-        const uint64_t mask = ballot(found[s]);
-        const int wd = (base + s * kWave) >> 5;
-        if (lane == 0) next[wd] = (unsigned)mask;
-        if (lane == 1) next[wd + 1] = (unsigned)(mask >> 32);
+        #pragma unroll
+        for (int s = 0; s < kSub; s++) {
+          #pragma unroll
+          for (int k = 0; k < kFirst; k++) found[s] = found[s] || (nb[s][k] >= 0 && in_bits(cur, nb[s][k]));
+        }
+        #pragma unroll
+        for (int s = 0; s < kSub; s++) {
+          const long long tile = (long long)tile0 + (long long)s * apart;
+          if (tile >= ntiles) break;  // uniform
+          int at = ub[s] + kFirst;
+          const int stop = by_lanes ? min(ue[s], ub[s] + kLaneRow) : at;
+          while (unvisited[s] && !found[s] && at < stop) {
+            int u[kStep];
+            #pragma unroll
+            for (int k = 0; k < kStep; k++) u[k] = (at + k < stop) ? nlist[at + k] : -1;
+            #pragma unroll
+            for (int k = 0; k < kStep; k++) found[s] = found[s] || (u[k] >= 0 && in_bits(cur, u[k]));
+            at += kStep;
+          }
+          uint64_t pending = ballot(unvisited[s] && !found[s] && ue[s] > stop);
+          while (pending != 0) {
+            const int L = __ffsll((unsigned long long)pending) - 1;
+            pending &= pending - 1;
+            const int s0 = __shfl(stop, L, kWave);
+            const int e0 = __shfl(ue[s], L, kWave);
+            bool hit = false;
+            for (int i0 = s0; i0 < e0; i0 += kWave) {
+              const int i = i0 + lane;
+              const bool h = (i < e0) && in_bits(cur, nlist[i]);
+              if (ballot(h) != 0) {
+                hit = true;
+                break;
+              }
+            }
+            if (lane == L) found[s] = hit;
+          }
+          if (found[s]) {
+            dist[tile * kWave + lane] = nd;
+            found_v += 1;
+            found_e += ue[s] - ub[s];
+          }
+          const uint64_t mask = ballot(found[s]);
+          const long long wd = tile * 2;
+          if (lane == 0) next[wd] = (unsigned)mask;
+          if (lane == 1) next[wd + 1] = (unsigned)(mask >> 32);
+        }
       }
-    }
+    };
+    if (ntiles >= nwaves * kSub) bottom_up(std::true_type{});
+    else bottom_up(std::false_type{});
   }
   round_partials(ctl, found_v, found_e, 0, 0, s_red);
 }
@@ -884,11 +912,12 @@ int style_do_hybrid(const igx_graph* g, int src, void* out, const void*, igx_run
       [&](long long) {
         ktimer_begin("bfs_do_level");
         hipLaunchKernelGGL(bfs_do_level, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, g->nlist,
-                           g->nodes, dist, q0, q1, (const Entry*)pq, (const int*)pc, (unsigned*)pb, words, R.d_ctl);
+                           g->nodes, dist, q0, q1, (const Entry*)pq, (const int*)pc, (unsigned*)pb, words,
+                           g->edges / 16 < g->nodes, R.d_ctl);
         ktimer_end("bfs_do_level");
         finish(true);
       },
-      (long long)g->nodes + 2, &rounds, &launches, 6);
+      (long long)g->nodes + 2, &rounds, &launches, g->edges < kFewEdges ? 4 : 6);
   IGX_TRY(timer_stop(&info->seconds));
   info->iterations = rounds;
   info->launches = launches;
