@@ -476,6 +476,7 @@ constexpr int kSeedDiv = IGX_SSSP_SEED_DIV;  // 0: no partial push round
 #endif
 constexpr double kHubRatio = IGX_SSSP_HUB_RATIO;
 constexpr long long kQueueEdgesS = 1 << 16;
+constexpr long long kClaimsPerWave = 4;      // claims per running wave from which a pull leaves waiting workgroups out
 constexpr long long kEdgesPerBlock = 2048;  // frontier edges per workgroup of a push round from a queue
 // A pull round whose frontier holds more than this percentage of the edges
 // reads every neighbour's distance instead of testing its frontier bit first:
@@ -919,6 +920,7 @@ struct FinSsspDo {
   long long m;
   int nblocks;            // the round kernel's grid
   long long claims;       // claims of row tiles in a pull round
+  int resident;           // workgroups of the round kernel that run at once
   const int* long_chunks; // chunks of long rows
   __device__ void operator()(Ctl* ctl, const RoundTotals& t) const
   {
@@ -986,6 +988,12 @@ struct FinSsspDo {
                                  ? (max(claims, (*long_chunks + 1LL) / 2) + kWavesPerBlock - 1) / kWavesPerBlock
                                  : (ef + kEdgesPerBlock - 1) / kEdgesPerBlock;
       act = (int)min(max(want, 16LL), (long long)nblocks);
+      // Workgroups beyond those that run at once start when the first ones
+      // have walked all tiles, and only then take their share of the chunks.
+      // With many claims a wave they are left out (R-MAT 22, three pull
+      // rounds 508 + 365 + 341 -> 476 + 341 + 205 us); with few, the later
+      // ones fill the ends of the earlier (R-MAT 20 without them 360 -> 387).
+      if (ctl->mode == 1 && claims >= kClaimsPerWave * resident * kWavesPerBlock) act = min(act, resident);
       if (act >= nblocks) act = 0;
     }
     ctl->active = act;
@@ -1404,7 +1412,9 @@ int style_do(const igx_graph* g, int src, void* out, const void*, igx_run_info* 
   hipLaunchKernelGGL(sssp_do_init, dim3(blocks_for(g->nodes, kBlock)), dim3(kBlock), 0, R.stream, src, g->nindex,
                      g->nodes, dist, (Entry*)p0, (unsigned*)pm, words, R.d_ctl);
   IGX_TRY(big_rows(g, pb, (int*)pc));
-  const FinSsspDo fin{(long long)g->edges, R.persist_blocks, claims, (const int*)pc};
+  int per_cu = 0;
+  IGX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, sssp_do_round, kBlock, 0));
+  const FinSsspDo fin{(long long)g->edges, R.persist_blocks, claims, (per_cu > 0 ? per_cu : 1) * R.cus, (const int*)pc};
   auto finish = [&](bool after_round) {
     hipLaunchKernelGGL(sssp_do_finish, dim3(1), dim3(kFinBlock), 0, R.stream, g->nindex, g->nlist, g->eweight, dist,
                        q0, q1, (unsigned*)pm, words, R.persist_blocks, after_round, fin, R.d_ctl);
