@@ -223,19 +223,21 @@ __global__ void __launch_bounds__(kBlock) tc_edge_bsearch(const int* __restrict_
 //
 // Whole call, before (one wave per vertex hashing N+(v) and probing the lists
 // of its out-neighbours, orientation by a row map, flags and a scan over the
-// edges) and now: R-MAT 20 (n = 1,048,576, m = 31.4 M) 38.4 -> 2.0 ms;
+// edges) and now: R-MAT 20 (n = 1,048,576, m = 31.4 M) 38.4 -> 1.37 ms;
 // Erdos-Renyi n = 2,097,152, average degree 16: 2.76 -> 1.27 ms.
 constexpr int kTcWords = kEdgeTile / kWave;      // keep-bit words per tile
 constexpr int kTcShort = 32;                     // lists up to this length: 16-byte groups against a list in LDS
 constexpr int kTcBitWords = 4096;                // bitmap of 2^17 ranks, 16 KB
 constexpr int kTcHashSlice = kTcBitWords / 4;    // list elements per pass where ranks exceed the bitmap
-constexpr int kTcPad = 128;                      // ints that 16-byte reads may pass the end of a list array
+constexpr int kTcPad = 128;                      // elements that 16-byte reads may pass the end of a list array
+constexpr int kTcHalf = 65535;                   // ranks of x up to which the lists are read as 16 bits
 constexpr int kTcSingle = 32768;                 // ranks claimed one by one by the count; beyond, kTcClaim at once
 constexpr int kTcClaim = 8;
 constexpr int kTcClaimStride = 64;               // ints between the groups' claim counters
 constexpr int kTcShortRows = 32;                 // rows per wave step of the short count
 
 typedef int TcInt4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned TcHalf8 __attribute__((ext_vector_type(4), aligned(2)));  // eight 16-bit ranks
 
 __global__ void __launch_bounds__(kBlock) tc_clear(int* __restrict__ p, int count)
 {
@@ -301,13 +303,15 @@ __global__ void __launch_bounds__(kBlock) tc_keep(const int* __restrict__ nindex
 }
 
 // The oriented lists, in the order of the rows and of each row: olist by id
-// (sorted within the row), rlist by rank, and the row starts.
+// (sorted within the row), rlist by rank, hlist by rank in 16 bits (kTcHalf for
+// all ranks from there on), and the row starts.
 __global__ void __launch_bounds__(kBlock) tc_orient(const int* __restrict__ nindex, const int* __restrict__ nlist, int n,
                                                      int m, const int* __restrict__ rank,
                                                      const int* __restrict__ tile_row,
                                                      const unsigned long long* __restrict__ keep,
                                                      const int* __restrict__ tile_off, int* __restrict__ onidx,
-                                                     int* __restrict__ olist, int* __restrict__ rlist)
+                                                     int* __restrict__ olist, int* __restrict__ rlist,
+                                                     unsigned short* __restrict__ hlist)
 {
   __shared__ unsigned long long s_word[kTcWords + 1];
   __shared__ int s_pre[kTcWords + 1];
@@ -333,7 +337,9 @@ __global__ void __launch_bounds__(kBlock) tc_orient(const int* __restrict__ nind
       const int u = nlist[base + i];
       const int pos = off + s_pre[i / kWave] + mbcnt(word);
       olist[pos] = u;
-      rlist[pos] = rank[u];
+      const int z = rank[u];
+      rlist[pos] = z;
+      hlist[pos] = (unsigned short)min(z, kTcHalf);
     }
   }
   // starts of the rows that begin in the tile (up to the next tile's first row)
@@ -350,19 +356,26 @@ __global__ void __launch_bounds__(kBlock) tc_orient(const int* __restrict__ nind
 // Edges with an endpoint whose list is longer than kTcShort, at the endpoint
 // x with the longer list (ties: the larger id), one workgroup per x in rank
 // order, hubs first, claimed one at a time while they are heavy (four hubs at
-// a time were up to 3.4 times a workgroup's share of R-MAT 20).  All neighbours y of x are looked at; those with the
-// shorter list stream it past the set of x, 16 lanes a list and four
-// consecutive elements a lane, so a step of a wave tests 256 elements and
-// needs no search for their owner.  The set is a bitmap of ranks in LDS
+// a time were up to 3.4 times a workgroup's share of R-MAT 20).  All
+// neighbours y of x are looked at; those with the shorter list stream it past
+// the set of x.  Where r(x) <= kTcHalf every rank of N+(x) is below kTcHalf,
+// so the lists are read as 16 bits, larger ranks as kTcHalf, a bit that is
+// never set: half the bytes past L2, which bound the count with 32-bit lists
+// (10 GB on R-MAT 20), and a probe without a compare or a branch, 8 lanes a
+// list and eight consecutive elements a lane, the next eight under way.
+// R-MAT 20: whole call 1.96 -> 1.36 ms.  Other x read 32 bits, 16 lanes a
+// list and four elements a lane.  A step of a wave needs no search for the
+// owners of its elements.  The set is a bitmap of ranks in LDS
 // (16 KB, so that eight workgroups fit a CU); where r(x) exceeds its 2^17
 // bits, an exact hash set of slices of N+(x) in the same 16 KB, at most a
 // quarter full.  On R-MAT 20 99.9% of the probes meet the bitmap.  Between
 // two x the LDS words are all zero (both forms clear what they set).
-// R-MAT 20: 36.8 -> 1.6 ms for the count (3.24 ms with four ranks a claim).
+// R-MAT 20: 36.8 -> 1.0 ms for the count.
 __global__ void __launch_bounds__(kBlock) tc_count_long(const int* __restrict__ nindex, const int* __restrict__ nlist,
                                                          const int* __restrict__ order,
                                                          const int* __restrict__ heavy,
                                                          const int* __restrict__ onidx, const int* __restrict__ rlist,
+                                                         const unsigned short* __restrict__ hlist,
                                                          int* __restrict__ claim,
                                                          unsigned long long* __restrict__ count)
 {
@@ -393,6 +406,7 @@ __global__ void __launch_bounds__(kBlock) tc_count_long(const int* __restrict__ 
       if (len <= kTcShort) continue;
       const int nb = nindex[x], ne = nindex[x + 1];
       const bool bits = rx <= kTcBitWords * 32;
+      const bool half = rx <= kTcHalf;
       const int passes = bits ? 1 : (len + kTcHashSlice - 1) / kTcHashSlice;
       for (int ps = 0; ps < passes; ps++) {
         const int pb = bits ? beg : beg + ps * kTcHashSlice;
@@ -422,6 +436,38 @@ __global__ void __launch_bounds__(kBlock) tc_count_long(const int* __restrict__ 
           const int cnt = __popcll(some);
           __builtin_amdgcn_wave_barrier();
           __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          if (half) {
+            int idx = lane >> 3;
+            const int off = (lane & 7) * 8;
+            int pos = 0, end = 0;
+            if (idx < cnt) {
+              pos = s_ent[w][idx].x + off;
+              end = s_ent[w][idx].y;
+            }
+            TcHalf8 next8 = {};
+            if (idx < cnt) next8 = *(const TcHalf8*)(hlist + pos);
+            while (idx < cnt) {
+              const TcHalf8 z8 = next8;
+              const int left = end - pos;
+              pos += 64;
+              if (pos - off >= end) {
+                idx += 8;
+                if (idx < cnt) {
+                  pos = s_ent[w][idx].x + off;
+                  end = s_ent[w][idx].y;
+                }
+              }
+              if (idx < cnt) next8 = *(const TcHalf8*)(hlist + pos);
+              #pragma unroll
+              for (int k = 0; k < 8; k++) {
+                const unsigned z = (k & 1) ? z8[k / 2] >> 16 : z8[k / 2] & 0xffffu;
+                const unsigned bit = (s_set[z >> 5] >> (z & 31)) & 1u;
+                found += (k < left) ? bit : 0u;
+              }
+            }
+            __builtin_amdgcn_wave_barrier();
+            continue;
+          }
           int idx = lane >> 4;
           const int off = (lane & 15) * 4;
           int pos = 0, end = 0;
@@ -656,13 +702,14 @@ int style_oriented(const igx_graph* g, int, void* out, const void*, igx_run_info
   const int m = g->edges;
   const int tiles = (int)(((long long)m + kEdgeTile - 1) / kEdgeTile);
   const int rank_blocks = blocks_for(n, kRankRows);
-  void *pidx = nullptr, *plist = nullptr, *prl = nullptr, *ptile = nullptr, *pkeep = nullptr, *prank = nullptr,
+  void *pidx = nullptr, *plist = nullptr, *prl = nullptr, *phl = nullptr, *ptile = nullptr, *pkeep = nullptr, *prank = nullptr,
        *psmall = nullptr;
   IGX_TRY(ws_get(WS_B, sizeof(int) * ((size_t)n + 1), &pidx));
   // an undirected graph has exactly edges/2 oriented edges; size for edges so
   // that an asymmetric input cannot overrun the lists
   IGX_TRY(ws_get(WS_C, sizeof(int) * ((size_t)m + kTcPad), &plist));
   IGX_TRY(ws_get(WS_F, sizeof(int) * ((size_t)m + kTcPad), &prl));
+  IGX_TRY(ws_get(WS_H, sizeof(unsigned short) * ((size_t)m + kTcPad), &phl));
   // per tile: first row, kept edges, their prefix, and the scan's tile sums
   const int scan_n = tiles > 0 ? tiles : 1;
   IGX_TRY(ws_get(WS_E, sizeof(int) * (3 * (size_t)scan_n + scan_tiles_for(scan_n) + 64), &ptile));
@@ -700,10 +747,11 @@ int style_oriented(const igx_graph* g, int, void* out, const void*, igx_run_info
     exclusive_scan(tile_count, tile_off, tiles, tile_sum, tile_sum + scan_tiles_for(scan_n), R.stream);
     hipLaunchKernelGGL(tc_orient, dim3(tiles), dim3(kBlock), 0, R.stream, g->nindex, g->nlist, n, m, (const int*)rank,
                        (const int*)tile_row, (const unsigned long long*)keep, (const int*)tile_off, onidx, olist,
-                       rlist);
+                       rlist, (unsigned short*)phl);
     ktimer_begin("tc_oriented_count");
     hipLaunchKernelGGL(tc_count_long, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, g->nlist,
-                       (const int*)order, (const int*)heavy, (const int*)onidx, (const int*)rlist, claim, count);
+                       (const int*)order, (const int*)heavy, (const int*)onidx, (const int*)rlist,
+                       (const unsigned short*)phl, claim, count);
     hipLaunchKernelGGL(tc_count_short, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, (const int*)onidx,
                        (const int*)olist, n, count);
     ktimer_end("tc_oriented_count");

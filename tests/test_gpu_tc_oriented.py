@@ -1,6 +1,7 @@
 """Triangle counting by the default style at the edges of its kernels: lists
 of 32 and 33 (short and long count), rows that cross the 2048-edge tiles of
-the flat passes, runs of empty rows, ranks beyond the bitmap (hash set), hubs.
+the flat passes, runs of empty rows, ranks around 16 bits and
+beyond the bitmap (hash set), hubs.
 Counts are exact, against the serial oracle (tc_vertex_omp.h)."""
 import numpy as np
 import pytest
@@ -36,6 +37,8 @@ CASES = {
     "er_tiles": lambda: G.erdos_renyi(2051, 2.0, seed=3),
     "star_plus": lambda: G.from_edges(6001, np.r_[np.zeros(6000), np.arange(1, 6000)].astype(np.int32),
                                       np.r_[np.arange(1, 6001), np.arange(2, 6001)].astype(np.int32), "wheel"),
+    # ranks on both sides of 2^16 - 1, up to which the lists are read as 16 bits
+    "around_16bit": lambda: G.erdos_renyi(70000, 90.0, seed=4),
     # more than 2^17 vertices with out-lists above 32: ranks beyond the bitmap
     "beyond_bitmap": lambda: G.erdos_renyi(150000, 90.0, seed=2),
 }
