@@ -223,7 +223,7 @@ __global__ void __launch_bounds__(kBlock) tc_edge_bsearch(const int* __restrict_
 //
 // Whole call, before (one wave per vertex hashing N+(v) and probing the lists
 // of its out-neighbours, orientation by a row map, flags and a scan over the
-// edges) and now: R-MAT 20 (n = 1,048,576, m = 31.4 M) 38.4 -> 1.37 ms;
+// edges) and now: R-MAT 20 (n = 1,048,576, m = 31.4 M) 38.4 -> 1.36 ms;
 // Erdos-Renyi n = 2,097,152, average degree 16: 2.76 -> 1.27 ms.
 constexpr int kTcWords = kEdgeTile / kWave;      // keep-bit words per tile
 constexpr int kTcShort = 32;                     // lists up to this length: 16-byte groups against a list in LDS
@@ -363,8 +363,13 @@ __global__ void __launch_bounds__(kBlock) tc_orient(const int* __restrict__ nind
 // never set: half the bytes past L2, which bound the count with 32-bit lists
 // (10 GB on R-MAT 20), and a probe without a compare or a branch, 8 lanes a
 // list and eight consecutive elements a lane, the next eight under way.
-// R-MAT 20: whole call 1.96 -> 1.36 ms.  Other x read 32 bits, 16 lanes a
-// list and four elements a lane.  A step of a wave needs no search for the
+// Their hits are shifted into one register, so that the list's end costs one
+// field extract for eight elements, not a compare and a select for each
+// (R-MAT 18 415 -> 405 us).  R-MAT 20: whole call 1.96 -> 1.36 ms.  Other x
+// read 32 bits, 16 lanes a list and four elements a lane, the bitmap and the
+// hash set in loops of their own so that the bitmap's probes are not waited
+// for one by one (Erdos-Renyi n = 131,072, average degree 60: 573 -> 537 us).
+// A step of a wave needs no search for the
 // owners of its elements.  The set is a bitmap of ranks in LDS
 // (16 KB, so that eight workgroups fit a CU); where r(x) exceeds its 2^17
 // bits, an exact hash set of slices of N+(x) in the same 16 KB, at most a
@@ -458,12 +463,14 @@ __global__ void __launch_bounds__(kBlock) tc_count_long(const int* __restrict__ 
                 }
               }
               if (idx < cnt) next8 = *(const TcHalf8*)(hlist + pos);
+              unsigned hits = 0;  // element k's bit shifted in from the top: bit 24 + k
               #pragma unroll
               for (int k = 0; k < 8; k++) {
                 const unsigned z = (k & 1) ? z8[k / 2] >> 16 : z8[k / 2] & 0xffffu;
-                const unsigned bit = (s_set[z >> 5] >> (z & 31)) & 1u;
-                found += (k < left) ? bit : 0u;
+                hits = __builtin_amdgcn_alignbit(s_set[z >> 5] >> (z & 31), hits, 1);
               }
+              const int valid = min(max(left, 0), 8);
+              found += (unsigned)__popc(__builtin_amdgcn_ubfe(hits, 24, valid));
             }
             __builtin_amdgcn_wave_barrier();
             continue;
@@ -475,32 +482,51 @@ __global__ void __launch_bounds__(kBlock) tc_count_long(const int* __restrict__ 
             pos = s_ent[w][idx].x + off;
             end = s_ent[w][idx].y;
           }
-          while (idx < cnt) {
-            const TcInt4 z4 = *(const TcInt4*)(rlist + pos);
-            #pragma unroll
-            for (int k = 0; k < 4; k++) {
-              // past the list, or above every rank of N+(x): not in the set
-              const unsigned z = (pos + k < end) ? (unsigned)z4[k] : ~0u;
-              const bool in = z < (unsigned)rx;
-              if (bits) {
+          if (bits) {
+            while (idx < cnt) {
+              const TcInt4 z4 = *(const TcInt4*)(rlist + pos);
+              #pragma unroll
+              for (int k = 0; k < 4; k++) {
+                // past the list, or above every rank of N+(x): not in the set
+                const unsigned z = (unsigned)z4[k];
+                const bool in = pos + k < end && z < (unsigned)rx;
                 const unsigned word = s_set[in ? z >> 5 : 0u];
-                found += in ? (word >> (z & 31)) & 1u : 0u;
-              } else if (in) {
-                unsigned h = (z * 0x9E3779B1u) % (unsigned)kTcBitWords;
-                unsigned y = s_set[h];
-                while (y != 0u && y != z + 1u) {
-                  h = (h + 1) % (unsigned)kTcBitWords;
-                  y = s_set[h];
+                found += (word >> (z & 31)) & (in ? 1u : 0u);
+              }
+              pos += 64;
+              if (pos - off >= end) {
+                idx += 4;
+                if (idx < cnt) {
+                  pos = s_ent[w][idx].x + off;
+                  end = s_ent[w][idx].y;
                 }
-                found += (y != 0u) ? 1u : 0u;
               }
             }
-            pos += 64;
-            if (pos - off >= end) {
-              idx += 4;
-              if (idx < cnt) {
-                pos = s_ent[w][idx].x + off;
-                end = s_ent[w][idx].y;
+          } else {
+            while (idx < cnt) {
+              const TcInt4 z4 = *(const TcInt4*)(rlist + pos);
+              #pragma unroll
+              for (int k = 0; k < 4; k++) {
+                // past the list, or above every rank of N+(x): not in the set
+                const unsigned z = (pos + k < end) ? (unsigned)z4[k] : ~0u;
+                const bool in = z < (unsigned)rx;
+                if (in) {
+                  unsigned h = (z * 0x9E3779B1u) % (unsigned)kTcBitWords;
+                  unsigned y = s_set[h];
+                  while (y != 0u && y != z + 1u) {
+                    h = (h + 1) % (unsigned)kTcBitWords;
+                    y = s_set[h];
+                  }
+                  found += (y != 0u) ? 1u : 0u;
+                }
+              }
+              pos += 64;
+              if (pos - off >= end) {
+                idx += 4;
+                if (idx < cnt) {
+                  pos = s_ent[w][idx].x + off;
+                  end = s_ent[w][idx].y;
+                }
               }
             }
           }
