@@ -256,17 +256,6 @@ __global__ void __launch_bounds__(kBlock) pr_relabel(const int* __restrict__ nin
   }
 }
 
-__global__ void __launch_bounds__(kBlock) pr_bal_init(PrSource src, int n, float* __restrict__ contrib)
-{
-  const PrGraph g = pr_graph(src);
-  const int v = blockIdx.x * kBlock + threadIdx.x;
-  if (v < n) {
-    const float s0 = 1.0f / (float)n;  // pr_cuda.h:133
-    g.score[v] = s0;
-    contrib[v] = s0 / (float)(g.nindex[v + 1] - g.nindex[v]);
-  }
-}
-
 // scores of a renumbered graph back in the caller's order
 __global__ void __launch_bounds__(kBlock) pr_scores_out(PrSource src, int n, const int* __restrict__ order)
 {
@@ -277,10 +266,12 @@ __global__ void __launch_bounds__(kBlock) pr_scores_out(PrSource src, int n, con
 // counts[1]: rows of several chunks (big); counts[2]: chunks.  kClassRows
 // consecutive rows per workgroup, which reserves their slots with one atomic
 // on each counter (one per wave had 170 us of them on R-MAT 20); the chunks
-// of a longer row are written by its wave together.
+// of a longer row are written by its wave together.  Also the first scores and
+// contributions: one launch and one read of the row starts less (7 us at
+// n = 1,000,000).
 constexpr int kClassPer = 2;
 constexpr int kClassRows = kClassPer * kBlock;
-__global__ void __launch_bounds__(kBlock) pr_classify(PrSource src, int n, int* __restrict__ counts,
+__global__ void __launch_bounds__(kBlock) pr_classify(PrSource src, int n, float* __restrict__ contrib, int* __restrict__ counts,
                                                        Entry* __restrict__ chunks, BigRow* __restrict__ big)
 {
   __shared__ int s_red[kWavesPerBlock];
@@ -293,6 +284,11 @@ __global__ void __launch_bounds__(kBlock) pr_classify(PrSource src, int n, int* 
     const long long v = (long long)blockIdx.x * kClassRows + k * kBlock + threadIdx.x;
     beg[k] = (v < n) ? g.nindex[v] : 0;
     end[k] = (v < n) ? g.nindex[v + 1] : 0;
+    if (v < n) {
+      const float s0 = 1.0f / (float)n;  // pr_cuda.h:133
+      g.score[v] = s0;
+      contrib[v] = s0 / (float)(end[k] - beg[k]);
+    }
     c[k] = (end[k] - beg[k] > kSmallRow) ? chunks_of(end[k] - beg[k]) : 0;
     nc += c[k];
     nb += (c[k] > 1) ? 1 : 0;
@@ -664,6 +660,8 @@ int style_balanced(const igx_graph* g, int, void* out, const void*, igx_run_info
                         {g->nlist, may ? (int*)pl1 : g->nlist},
                         {(float*)out, may ? score1 : (float*)out},
                         may ? counts + kFlag : (int*)nullptr};
+  // for a graph that is known to be worked on as given: no flag to read
+  const PrSource given = {{g->nindex, g->nindex}, {g->nlist, g->nlist}, {(float*)out, (float*)out}, nullptr};
   const PrParams P = pr_params();
   const float base = (1.0f - kDamp) / (float)n;
   IGX_TRY(timer_start());
@@ -681,9 +679,8 @@ int style_balanced(const igx_graph* g, int, void* out, const void*, igx_run_info
     hipLaunchKernelGGL(pr_relabel, dim3(tiles), dim3(kBlock), 0, R.stream, g->nindex, g->nlist, n, m,
                        (const int*)rank, (const int*)tile_row, (const int*)nindex1, (int*)pl1, go);
   }
-  hipLaunchKernelGGL(pr_bal_init, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, R.stream, src, n, c0);
-  hipLaunchKernelGGL(pr_classify, dim3(blocks_for(n, kClassRows)), dim3(kBlock), 0, R.stream, src, n, counts,
-                     (Entry*)pch, (BigRow*)pbig);
+  hipLaunchKernelGGL(pr_classify, dim3(blocks_for(n, kClassRows)), dim3(kBlock), 0, R.stream, src, n, c0,
+                     counts, (Entry*)pch, (BigRow*)pbig);
   int rounds = 0, launches = 0;
   const int rc = run_rounds(
       [&](long long r) {
@@ -694,19 +691,20 @@ int style_balanced(const igx_graph* g, int, void* out, const void*, igx_run_info
         const bool known = r >= kFirstBatch;
         const bool hot = may && (!known || R.h_ctl->aux_ll[1] != 0);
         const bool big = !known || R.h_ctl->aux_ll[0] != 0;
+        const PrSource& from = hot ? src : given;
         if (hot) {
           hipLaunchKernelGGL(pr_hot_chunks, dim3(2 * R.cus), dim3(kHotBlock), 0, R.stream, src, n, base, cur, nxt,
                              (const int*)counts, (const Entry*)pch, (Pair*)ppart, R.persist_blocks, R.d_ctl);
         }
         ktimer_begin("pr_bal_main");
-        hipLaunchKernelGGL(pr_bal_main, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, src, n, base, cur, nxt,
+        hipLaunchKernelGGL(pr_bal_main, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, from, n, base, cur, nxt,
                            (const int*)counts, (const Entry*)pch, (Pair*)ppart, R.d_ctl);
         ktimer_end("pr_bal_main");
         if (big) {
-          hipLaunchKernelGGL(pr_bal_big, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, src, base, nxt,
+          hipLaunchKernelGGL(pr_bal_big, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, from, base, nxt,
                              (const BigRow*)pbig, (const int*)counts, (const Pair*)ppart, R.d_ctl);
         }
-        const FinPr fin{P.eps, P.max_iter, counts + 1, src.relabel};
+        const FinPr fin{P.eps, P.max_iter, counts + 1, from.relabel};
         if (hot && big) launch_finalize<0x7>(R.persist_blocks, fin);
         else if (hot) launch_finalize<0x5>(R.persist_blocks, fin);
         else if (big) launch_finalize<0x3>(R.persist_blocks, fin);
