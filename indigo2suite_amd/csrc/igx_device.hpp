@@ -185,6 +185,7 @@ struct Ctl {
   int force_all;         // SSSP: the next pull reads every neighbour (set after the partial push round)
   int bm_phase;          // BFS: the current frontier's bitmap is (level + bm_phase) % 3
   int active;            // workgroups that take part in the next round (0: all); round_finalize reduces that many
+  int sample[3];         // PR: what the sample of the edges counted
 };
 
 // Round epilogue.  Ending a round inside the round kernel ("the last block to

@@ -75,14 +75,18 @@ int ws_get(int slot, size_t bytes, void** ptr);
 // what is in the stream then, two batches of at most kMaxAhead rounds, is
 // waited for.
 // Returns IGX_OK, IGX_ERR_LIMIT when max_rounds did not converge, or an error.
-// From round first_batch on, R.h_ctl holds a control block of this run.
+// From round first_batch on, R.h_ctl holds a control block of this run.  With
+// behind_first, for runs that seldom end in the first batch, the second one is
+// in the stream before the first is waited for (that wait leaves the device
+// idle for about 30 us).
 constexpr int kAheadRounds = 4;
 constexpr int kMaxAhead = 32;
 bool past_time_limit();
 int batch_mark(int slot);    // copy the control block to slot's pinned mirror, behind the work so far
 int batch_wait(int slot);    // wait for it and make it *R.h_ctl
 template <typename F>
-int run_rounds(F launch, long long max_rounds, int* rounds_done, int* launches, int first_batch = 2)
+int run_rounds(F launch, long long max_rounds, int* rounds_done, int* launches, int first_batch = 2,
+               bool behind_first = false)
 {
   Runtime& R = rt();
   long long launched = 0, batches = 0;
@@ -96,6 +100,7 @@ int run_rounds(F launch, long long max_rounds, int* rounds_done, int* launches, 
     return batch_mark((int)(batches++ & 1));
   };
   IGX_TRY(enqueue(first_batch));
+  if (behind_first && launched < max_rounds) IGX_TRY(enqueue(kAheadRounds));
   long long waited = 0;
   int rc = IGX_OK;
   while (true) {

@@ -62,15 +62,20 @@ static __global__ void __launch_bounds__(kBlock) rank_hist(const int* __restrict
   }
 }
 
+// the vertices whose bins lie whole within the first `ranks` ranks
+struct RankHead {
+  long long edges;   // their edges, at least
+  long long degree;  // their least degree; INT_MAX: there are none
+};
+
 // bins become the first rank of each (highest degree first); *above = number
-// of vertices of degree above `limit` (below kRankExact).  With hot_ranks > 0,
-// *hot = the vertices of the first hot_ranks ranks take at least a quarter of
-// the m edges.  One workgroup.
+// of vertices of degree above `limit` (below kRankExact); *head, if asked for,
+// describes the first `ranks` ranks.  One workgroup.
 static __global__ void __launch_bounds__(kBlock) rank_bins(int* __restrict__ bins, int limit, int* __restrict__ above,
-                                                            int hot_ranks, int m, int* __restrict__ hot)
+                                                            int ranks, RankHead* __restrict__ head)
 {
   __shared__ int s_red[kWavesPerBlock];
-  __shared__ long long s_hot[kWavesPerBlock];
+  __shared__ long long s_edges[kWavesPerBlock], s_degree[kWavesPerBlock];
   constexpr int kPerT = (kRankBins + kBlock - 1) / kBlock;
   int c[kPerT];
   int local = 0;
@@ -82,7 +87,8 @@ static __global__ void __launch_bounds__(kBlock) rank_bins(int* __restrict__ bin
   }
   int tot = 0;
   int run = block_excl_scan(local, s_red, &tot);
-  long long edges = 0;  // of the hot ranks, by the least degree of each bin
+  long long edges = 0;  // of the head, by the least degree of each bin
+  long long least = INT_MAX;
   #pragma unroll
   for (int k = 0; k < kPerT; k++) {
     const int i = kRankBins - 1 - ((int)threadIdx.x * kPerT + k);
@@ -90,31 +96,39 @@ static __global__ void __launch_bounds__(kBlock) rank_bins(int* __restrict__ bin
       bins[i] = run;
       const int over = i - kRankExact;
       const long long deg = (over < 0) ? i : ((long long)(64 + (over & 63)) << (5 + over / 64));
-      edges += deg * (min(run + c[k], hot_ranks) - min(run, hot_ranks));
+      if (c[k] > 0 && run + c[k] <= ranks) {
+        edges += deg * c[k];
+        least = min(least, deg);
+      }
     }
-    if (i == limit) *above = run;
+    if (i == limit && above != nullptr) *above = run;
     run += c[k];
   }
-  if (hot_ranks <= 0) return;
+  if (head == nullptr) return;
   edges = wave_sum_ll(edges);
-  if (lane_id() == 0) s_hot[threadIdx.x / kWave] = edges;
+  least = wave_min_ll(least);
+  if (lane_id() == 0) {
+    s_edges[threadIdx.x / kWave] = edges;
+    s_degree[threadIdx.x / kWave] = least;
+  }
   __syncthreads();
   if (threadIdx.x == 0) {
-    long long t = 0;
-    for (int k = 0; k < kWavesPerBlock; k++) t += s_hot[k];
-    *hot = (t >= m / 4) ? 1 : 0;
+    RankHead h{0, INT_MAX};
+    for (int k = 0; k < kWavesPerBlock; k++) {
+      h.edges += s_edges[k];
+      h.degree = min(h.degree, s_degree[k]);
+    }
+    *head = h;
   }
 }
 
 // rank[v] and its inverse order[] (and the degrees in rank order, when asked
 // for): a workgroup reserves a run of ranks in each bin for its vertices.
-// Nothing is done when `go` is given and 0.
 static __global__ void __launch_bounds__(kBlock) rank_assign(const int* __restrict__ nindex, int n, int* __restrict__ bins,
                                                    int* __restrict__ rank, int* __restrict__ order,
-                                                   int* __restrict__ degree, const int* __restrict__ go)
+                                                   int* __restrict__ degree)
 {
   __shared__ int s_bin[kRankBins];
-  if (go != nullptr && *go == 0) return;
   if (degree != nullptr && blockIdx.x == 0 && threadIdx.x == 0) degree[n] = 0;  // closes a scan
   for (int i = threadIdx.x; i < kRankBins; i += kBlock) s_bin[i] = 0;
   __syncthreads();

@@ -28,10 +28,9 @@ __device__ __forceinline__ int block_excl_scan(int v, int* lds, int* total)
 
 // out[i] = sum of in[0..i) within the tile; tile_sum[b] = tile total
 static __global__ void __launch_bounds__(kBlock) scan_tiles(const int* __restrict__ in, int* __restrict__ out, int count,
-                                                      int* __restrict__ tile_sum, const int* __restrict__ go)
+                                                      int* __restrict__ tile_sum)
 {
   __shared__ int lds[kWavesPerBlock];
-  if (go != nullptr && *go == 0) return;
   const long long base = (long long)blockIdx.x * kScanTile;
   int vals[4];
   int local = 0;
@@ -53,11 +52,9 @@ static __global__ void __launch_bounds__(kBlock) scan_tiles(const int* __restric
 }
 
 // one workgroup: exclusive scan of the tile totals in place; total[0] = sum
-static __global__ void __launch_bounds__(kBlock) scan_tile_sums(int* __restrict__ tile_sum, int tiles, int* __restrict__ total,
-                                                          const int* __restrict__ go)
+static __global__ void __launch_bounds__(kBlock) scan_tile_sums(int* __restrict__ tile_sum, int tiles, int* __restrict__ total)
 {
   __shared__ int lds[kWavesPerBlock];
-  if (go != nullptr && *go == 0) return;
   int carry = 0;
   for (int base = 0; base < tiles; base += kBlock) {
     const int i = base + threadIdx.x;
@@ -70,26 +67,22 @@ static __global__ void __launch_bounds__(kBlock) scan_tile_sums(int* __restrict_
   if (threadIdx.x == 0) *total = carry;
 }
 
-static __global__ void __launch_bounds__(kBlock) scan_add(int* __restrict__ out, int count, const int* __restrict__ tile_sum,
-                                                    const int* __restrict__ go)
+static __global__ void __launch_bounds__(kBlock) scan_add(int* __restrict__ out, int count, const int* __restrict__ tile_sum)
 {
-  if (go != nullptr && *go == 0) return;
   const long long i = (long long)blockIdx.x * kBlock + threadIdx.x;
   if (i < count) out[i] += tile_sum[i / kScanTile];
 }
 
 inline int scan_tiles_for(int count) { return (count + kScanTile - 1) / kScanTile > 0 ? (count + kScanTile - 1) / kScanTile : 1; }
 
-// enqueue the three launches; tile_sum needs scan_tiles_for(count) ints.  They
-// do nothing when `go` is given and 0 on the device.
-inline void exclusive_scan(const int* in, int* out, int count, int* tile_sum, int* total, hipStream_t s,
-                           const int* go = nullptr)
+// enqueue the three launches; tile_sum needs scan_tiles_for(count) ints
+inline void exclusive_scan(const int* in, int* out, int count, int* tile_sum, int* total, hipStream_t s)
 {
   const int tiles = scan_tiles_for(count);
-  hipLaunchKernelGGL(scan_tiles, dim3(tiles), dim3(kBlock), 0, s, in, out, count, tile_sum, go);
-  hipLaunchKernelGGL(scan_tile_sums, dim3(1), dim3(kBlock), 0, s, tile_sum, tiles, total, go);
+  hipLaunchKernelGGL(scan_tiles, dim3(tiles), dim3(kBlock), 0, s, in, out, count, tile_sum);
+  hipLaunchKernelGGL(scan_tile_sums, dim3(1), dim3(kBlock), 0, s, tile_sum, tiles, total);
   hipLaunchKernelGGL(scan_add, dim3((count + kBlock - 1) / kBlock > 0 ? (count + kBlock - 1) / kBlock : 1), dim3(kBlock),
-                     0, s, out, count, tile_sum, go);
+                     0, s, out, count, tile_sum);
 }
 
 }  // namespace igx

@@ -105,17 +105,15 @@ __device__ __forceinline__ long long pr_finish(int v, Pair acc, float base, cons
 // End of an iteration (run by round_finalize): the L1 residual is the exact
 // integer sum of the per-block partials (slot 0: rows scored by the main
 // kernel, slot 1: rows merged from chunks, slot 2: rows of one chunk of a
-// renumbered graph), scaled back from 2^-50 units.  Also tells the host which
-// of the balanced style's kernels have work on this graph.
+// renumbered graph), scaled back from 2^-50 units.  Also tells the host
+// whether the balanced style's merging kernel has work on this graph.
 struct FinPr {
   double eps;
   int max_iter;
   const int* big_rows;
-  const int* relabel;
   __device__ void operator()(Ctl* ctl, const RoundTotals& t) const
   {
     ctl->aux_ll[0] = (big_rows != nullptr) ? *big_rows : 0;
-    ctl->aux_ll[1] = (relabel != nullptr) ? *relabel : 0;
     const double r = (double)(t.s[0] + t.s[1] + t.s[2]) / kResScale;
     ctl->res_last = r;
     ctl->iter += 1;
@@ -185,37 +183,95 @@ struct BigRow {
 };
 
 // Degree order.  An iteration is bound by its gathers, one contribution per
-// edge.  On a graph with hubs most of them go to few vertices, which lie all
-// over the contribution array, so each costs a cache line of its own.  Where
-// the kHotRanks vertices of highest degree (a contribution each: 64 KB of LDS)
-// take at least a quarter of the edges, the run works on a copy of the graph
-// renumbered by degree rank, whose hot contributions lie side by side.  Rows keep their edges in the order they had, and their chunks, so
-// a row of one chunk sums the same values in the same order.  R-MAT 20: the
-// iterations without the hot values in LDS 190 -> 139 us, the copy 210 us per
-// run; whole run 3.37 -> 2.21 ms with the other changes.  Chung-Lu n = 1 M,
-// average degree 16: exponent 2.3 (35% hot) 2.04 -> 1.90 ms, exponent 2.7 1.71
-// -> 1.84 ms if it were copied (under the line).
-// On other graphs (a mesh, whose ids are local) the copy would cost its build
-// and lose what locality there is.
+// edge.  On a graph with hubs most of them go to few vertices, the head (the
+// kHotRanks vertices of highest degree; a contribution each: 64 KB of LDS),
+// which may lie all over the contribution array, a cache line each.  Such a
+// graph is worked on as a copy renumbered by degree rank: the head's
+// contributions lie side by side and the chunks find them in LDS.  Rows keep
+// their edges in the order they had, and their chunks, so a row of one chunk
+// sums the same values in the same order.  R-MAT 20: the iterations without the
+// hot values in LDS 190 -> 139 us, the copy 210 us per run.
+//
+// The rule.  Copied are graphs whose head
+// * takes a quarter of the edges, and 1.5 times its share of the vertices:
+//   without the second, every graph of up to 65,536 vertices has such a head
+//   (Erdos-Renyi n = 65,536, average degree 64: 344 us as given, 459 copied);
+// * is met by long rows, which are the ones that look in LDS (kMinHits of
+//   kSamples edges): a star's are met by its leaves (300,000 vertices, 40 hubs:
+//   1576 / 2497 us), a mesh and a sparse random graph have none (200 x 200
+//   mesh 351 / 657 us);
+// * is scattered, where the contributions exceed an XCD's L2 (kNearNodes):
+//   Chung-Lu ids are in degree order already (n = 2 M, degree 16, exponent
+//   2.3: 3479 / 3853 us; R-MAT 22, edge factor 4: 7718 / 4285 us).  Below, the
+//   copy pays there too, since rows of one length side by side make long runs
+//   for pr_bal_main (n = 400 k: 1321 / 1075 us);
+// * is that of a graph with an edge a vertex, as the copy also passes over the
+//   vertices.
+// The host decides, from the degree bins and the sample, while pr_classify
+// prepares a graph that is not copied (and is empty for one that is): a graph
+// that is not copied paid 60 us for launches that found nothing to do when the
+// device decided (Erdos-Renyi n = 300 k, average degree 9: 520 -> 502 us).
 constexpr int kHotRanks = 16384;
 constexpr int kRelabelMinNodes = 2 * kHotRanks;  // below, most of the array is close by anyway
+constexpr int kNearNodes = 1 << 20;              // contributions of an XCD's L2 (4 MB)
+constexpr int kSamples = 4096;
+constexpr int kMinHits = kSamples / 50;
 
-// The graph a run works on: as given, or renumbered when *relabel says so.
-struct PrSource {
-  const int* nindex[2];
-  const int* nlist[2];
-  float* score[2];
-  const int* relabel;  // nullptr: as given
+__host__ __device__ inline bool pr_head_counts(int n, int m, long long head_edges)
+{
+  return head_edges >= m / 4 && (double)head_edges * n >= 1.5 * kHotRanks * m;
+}
+
+// what pr_sample counts; zero where the head is too small
+struct PrSample {
+  int hits;   // edges of long rows whose neighbour is in the head
+  int heads;  // edges whose neighbour is in the head
+  int mates;  // of the three vertices next to such a neighbour (ids equal but for the lowest two bits), those in it
 };
+
+__host__ __device__ inline bool pr_renumber_pays(int n, int m, const int* sample)
+{
+  const PrSample s = *(const PrSample*)sample;
+  const bool scattered = 4LL * s.mates < 3LL * 3 * s.heads;  // fewer than three quarters
+  return s.hits >= kMinHits && m >= n && (n <= kNearNodes || scattered || m < 8LL * n);
+}
+
+// The graph a run works on: as given, or the renumbered copy.
 struct PrGraph {
   const int* nindex;
   const int* nlist;
   float* score;
 };
-__device__ __forceinline__ PrGraph pr_graph(const PrSource& s)
+
+// kSamples evenly spaced edges against the head, added to *out; nothing is
+// looked at where the head is too small anyway
+__global__ void __launch_bounds__(kBlock) pr_sample(const int* __restrict__ nindex, const int* __restrict__ nlist, int n,
+                                                     int m, const int* __restrict__ tile_row,
+                                                     const RankHead* __restrict__ head, PrSample* __restrict__ out)
 {
-  const int k = (s.relabel != nullptr && *s.relabel != 0) ? 1 : 0;
-  return PrGraph{k ? s.nindex[1] : s.nindex[0], k ? s.nlist[1] : s.nlist[0], k ? s.score[1] : s.score[0]};
+  if (!pr_head_counts(n, m, head->edges)) return;
+  const int e = (int)((long long)m * (blockIdx.x * kBlock + threadIdx.x) / kSamples);
+  const int tile = e / kEdgeTile;
+  int lo = tile_row[tile], hi = ((long long)(tile + 1) * kEdgeTile < m) ? tile_row[tile + 1] + 1 : n;
+  // the last row that starts at or before e
+  while (hi - lo > 1) {
+    const int mid = lo + (hi - lo) / 2;
+    if (nindex[mid] <= e) lo = mid;
+    else hi = mid;
+  }
+  const int u = nlist[e];
+  auto in_head = [&](int v) { return v < n && nindex[v + 1] - nindex[v] >= head->degree; };
+  const bool hot = in_head(u);
+  int mates = 0;
+  for (int k = 1; k < 4; k++) mates += (hot && in_head(u ^ k)) ? 1 : 0;
+  mates = wave_sum(mates);
+  const int hits = __popcll(ballot(hot && nindex[lo + 1] - nindex[lo] > kSmallRow));
+  const int heads = __popcll(ballot(hot));
+  if (lane_id() == 0) {
+    atomicAdd(&out->hits, hits);
+    atomicAdd(&out->heads, heads);
+    atomicAdd(&out->mates, mates);
+  }
 }
 
 __global__ void __launch_bounds__(kBlock) pr_zero(int* __restrict__ p, int count)
@@ -227,12 +283,10 @@ __global__ void __launch_bounds__(kBlock) pr_zero(int* __restrict__ p, int count
 __global__ void __launch_bounds__(kBlock) pr_relabel(const int* __restrict__ nindex, const int* __restrict__ nlist, int n,
                                                       int m, const int* __restrict__ rank,
                                                       const int* __restrict__ tile_row,
-                                                      const int* __restrict__ nindex1, int* __restrict__ nlist1,
-                                                      const int* __restrict__ relabel)
+                                                      const int* __restrict__ nindex1, int* __restrict__ nlist1)
 {
   __shared__ __align__(16) int s_row[kEdgeTile];
   __shared__ int s_red[kWavesPerBlock];
-  if (*relabel == 0) return;
   const int tile = blockIdx.x;
   const int base = tile * kEdgeTile;
   const int r0 = tile_row[tile];
@@ -257,10 +311,11 @@ __global__ void __launch_bounds__(kBlock) pr_relabel(const int* __restrict__ nin
 }
 
 // scores of a renumbered graph back in the caller's order
-__global__ void __launch_bounds__(kBlock) pr_scores_out(PrSource src, int n, const int* __restrict__ order)
+__global__ void __launch_bounds__(kBlock) pr_scores_out(const float* __restrict__ score, int n, const int* __restrict__ order,
+                                                         float* __restrict__ out)
 {
   const int r = blockIdx.x * kBlock + threadIdx.x;
-  if (r < n) src.score[0][order[r]] = src.score[1][r];
+  if (r < n) out[order[r]] = score[r];
 }
 
 // counts[1]: rows of several chunks (big); counts[2]: chunks.  kClassRows
@@ -271,12 +326,13 @@ __global__ void __launch_bounds__(kBlock) pr_scores_out(PrSource src, int n, con
 // n = 1,000,000).
 constexpr int kClassPer = 2;
 constexpr int kClassRows = kClassPer * kBlock;
-__global__ void __launch_bounds__(kBlock) pr_classify(PrSource src, int n, float* __restrict__ contrib, int* __restrict__ counts,
-                                                       Entry* __restrict__ chunks, BigRow* __restrict__ big)
+__global__ void __launch_bounds__(kBlock) pr_classify(PrGraph g, int n, int m, float* __restrict__ contrib, int* __restrict__ counts,
+                                                       Entry* __restrict__ chunks, BigRow* __restrict__ big,
+                                                       const int* __restrict__ sample)
 {
   __shared__ int s_red[kWavesPerBlock];
   __shared__ int s_first, s_big;
-  const PrGraph g = pr_graph(src);
+  if (sample != nullptr && pr_renumber_pays(n, m, sample)) return;  // the copy is classified instead
   int beg[kClassPer], end[kClassPer], c[kClassPer];
   int nc = 0, nb = 0;
   #pragma unroll
@@ -358,7 +414,7 @@ __device__ __forceinline__ long long pr_chunk(const Entry& en, int k, const PrGr
 // R-MAT 20 (57% of the edges hot): 128 -> 104 us an iteration together with
 // the small rows.
 constexpr int kHotBlock = 1024;
-__global__ void __launch_bounds__(kHotBlock) pr_hot_chunks(PrSource src, int n, float base,
+__global__ void __launch_bounds__(kHotBlock) pr_hot_chunks(PrGraph g, int n, float base,
                                                             const float* __restrict__ contrib_cur,
                                                             float* __restrict__ contrib_next,
                                                             const int* __restrict__ counts,
@@ -373,22 +429,19 @@ __global__ void __launch_bounds__(kHotBlock) pr_hot_chunks(PrSource src, int n, 
     for (int i = gridDim.x + threadIdx.x; i < nparts; i += kHotBlock) ctl_parts(ctl)[(size_t)2 * kMaxParts + i] = 0;
   }
   long long err = 0;
-  if (*src.relabel != 0) {  // uniform
-    const PrGraph g = pr_graph(src);
-    for (int i = threadIdx.x; i < kHotRanks && i < n; i += kHotBlock) s_hot[i] = contrib_cur[i];
-    __syncthreads();
-    const int nch = counts[2];
-    const int waves = gridDim.x * (kHotBlock / kWave);
-    for (int k = blockIdx.x * (kHotBlock / kWave) + threadIdx.x / kWave; k < nch; k += waves) {  // uniform per wave
-      err += pr_chunk(chunks[k], k, g, base, contrib_next, partial, [&](const int* u, float* x) {
-        #pragma unroll
-        for (int j = 0; j < kChunk / kWave; j++) x[j] = (u[j] >= kHotRanks) ? contrib_cur[u[j]] : 0.0f;
-        #pragma unroll
-        for (int j = 0; j < kChunk / kWave; j++) {
-          if (u[j] >= 0 && u[j] < kHotRanks) x[j] = s_hot[u[j]];
-        }
-      });
-    }
+  for (int i = threadIdx.x; i < kHotRanks && i < n; i += kHotBlock) s_hot[i] = contrib_cur[i];
+  __syncthreads();
+  const int nch = counts[2];
+  const int waves = gridDim.x * (kHotBlock / kWave);
+  for (int k = blockIdx.x * (kHotBlock / kWave) + threadIdx.x / kWave; k < nch; k += waves) {  // uniform per wave
+    err += pr_chunk(chunks[k], k, g, base, contrib_next, partial, [&](const int* u, float* x) {
+      #pragma unroll
+      for (int j = 0; j < kChunk / kWave; j++) x[j] = (u[j] >= kHotRanks) ? contrib_cur[u[j]] : 0.0f;
+      #pragma unroll
+      for (int j = 0; j < kChunk / kWave; j++) {
+        if (u[j] >= 0 && u[j] < kHotRanks) x[j] = s_hot[u[j]];
+      }
+    });
   }
   round_partial_ll(ctl, 2, err, s_red);
 }
@@ -399,7 +452,7 @@ __global__ void __launch_bounds__(kHotBlock) pr_hot_chunks(PrSource src, int n, 
 // rows: consecutive small rows form runs whose edges are contiguous, streamed
 // kSlice at a time (independent loads, values parked in LDS); each lane then
 // adds its own row's values in edge order.
-__global__ void __launch_bounds__(kBlock) pr_bal_main(PrSource src, int n, float base,
+__global__ void __launch_bounds__(kBlock) pr_bal_main(PrGraph g, bool chunks_done, int n, float base,
                                                        const float* __restrict__ contrib_cur,
                                                        float* __restrict__ contrib_next,
                                                        const int* __restrict__ counts,
@@ -409,7 +462,6 @@ __global__ void __launch_bounds__(kBlock) pr_bal_main(PrSource src, int n, float
   __shared__ long long s_red[kWavesPerBlock];
   __shared__ float s_val[kWavesPerBlock][kSlice];
   if (round_done(ctl)) return;
-  const PrGraph g = pr_graph(src);
   const int* __restrict__ nindex = g.nindex;
   const int* __restrict__ nlist = g.nlist;
   float* __restrict__ score = g.score;
@@ -417,7 +469,7 @@ __global__ void __launch_bounds__(kBlock) pr_bal_main(PrSource src, int n, float
   const int waves = gridDim.x * kWavesPerBlock;
   const int gw = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
   const int lane = lane_id();
-  const int nch = (src.relabel != nullptr && *src.relabel != 0) ? 0 : counts[2];
+  const int nch = chunks_done ? 0 : counts[2];
   for (int k = gw; k < nch; k += waves) {  // uniform per wave
     err += pr_chunk(chunks[k], k, g, base, contrib_next, partial, [&](const int* u, float* x) {
       #pragma unroll
@@ -477,13 +529,12 @@ __global__ void __launch_bounds__(kBlock) pr_bal_main(PrSource src, int n, float
 // lane a row left the longest row's chain, 273 merges on R-MAT 20, as the
 // kernel's time: 29 us.)
 constexpr int kBigLanes = 8;
-__global__ void __launch_bounds__(kBlock) pr_bal_big(PrSource src, float base, float* __restrict__ contrib_next,
+__global__ void __launch_bounds__(kBlock) pr_bal_big(PrGraph g, float base, float* __restrict__ contrib_next,
                                                       const BigRow* __restrict__ big, const int* __restrict__ counts,
                                                       const Pair* __restrict__ partial, Ctl* ctl)
 {
   __shared__ long long s_red[kWavesPerBlock];
   if (round_done(ctl)) return;
-  const PrGraph g = pr_graph(src);
   long long err = 0;
   const int nb = counts[1];
   const int l = threadIdx.x % kBigLanes;
@@ -611,7 +662,7 @@ int style_pull(const igx_graph* g, int, void* out, const void*, igx_run_info* in
         float* nxt = (r & 1) ? c0 : c1;
         hipLaunchKernelGGL((pr_pull<G>), dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, g->nlist,
                            g->nodes, base, score, cur, nxt, R.d_ctl, P.eps, P.max_iter);
-        launch_finalize<0x1>(R.persist_blocks, FinPr{P.eps, P.max_iter, nullptr, nullptr});
+        launch_finalize<0x1>(R.persist_blocks, FinPr{P.eps, P.max_iter, nullptr});
       },
       P.max_iter, &rounds, &launches);
   IGX_TRY(timer_stop(&info->seconds));
@@ -632,88 +683,105 @@ int style_balanced(const igx_graph* g, int, void* out, const void*, igx_run_info
   // at most deg / kChunk + 1 chunks
   const size_t nrows = (size_t)m / (kSmallRow + 1) + 64;
   const size_t nchunks = (size_t)m / kChunk + nrows;
-  // counters and the degree bins; the relabel flag is kept at kFlag
-  constexpr int kFlag = 8, kSmall = 64 + kRankBins;
-  constexpr int kFirstBatch = 4;
+  constexpr int kSmall = 64 + kRankBins;  // counters and the degree bins
   const int tiles = (int)(((long long)m + kEdgeTile - 1) / kEdgeTile);
-  void *pcnt = nullptr, *pch = nullptr, *pbig = nullptr, *ppart = nullptr, *pr1 = nullptr, *pl1 = nullptr,
-       *ptile = nullptr;
+  void *pcnt = nullptr, *pch = nullptr, *pbig = nullptr, *ppart = nullptr, *ptile = nullptr;
   IGX_TRY(ws_get(WS_B, sizeof(int) * kSmall, &pcnt));
   IGX_TRY(ws_get(WS_D, sizeof(Entry) * nchunks, &pch));
   IGX_TRY(ws_get(WS_C, sizeof(BigRow) * nrows, &pbig));
   IGX_TRY(ws_get(WS_H, sizeof(Pair) * nchunks, &ppart));
-  // the renumbered copy; without the memory for it the run does without
+  // without the memory for the renumbered copy the run does without it
   const bool may = n >= kRelabelMinNodes && m > 0 &&
-                   ws_get(WS_A, sizeof(int) * 5 * ((size_t)n + 1), &pr1) == IGX_OK &&
-                   ws_get(WS_E, sizeof(int) * (size_t)m, &pl1) == IGX_OK &&
                    ws_get(WS_BLOCKS, sizeof(int) * ((size_t)tiles + scan_tiles_for(n + 1) + 64), &ptile) == IGX_OK;
   int* counts = (int*)pcnt;
   int* bins = counts + 64;
-  int* rank = (int*)pr1;
-  int* order = rank + n;
-  int* degree = order + n;             // n + 1
-  int* nindex1 = degree + n + 1;       // n + 1
-  float* score1 = (float*)(nindex1 + n + 1);
   int* tile_row = (int*)ptile;
   int* tile_sum = tile_row + tiles;
-  const PrSource src = {{g->nindex, may ? nindex1 : g->nindex},
-                        {g->nlist, may ? (int*)pl1 : g->nlist},
-                        {(float*)out, may ? score1 : (float*)out},
-                        may ? counts + kFlag : (int*)nullptr};
-  // for a graph that is known to be worked on as given: no flag to read
-  const PrSource given = {{g->nindex, g->nindex}, {g->nlist, g->nlist}, {(float*)out, (float*)out}, nullptr};
+  PrGraph from = {g->nindex, g->nlist, (float*)out};
   const PrParams P = pr_params();
   const float base = (1.0f - kDamp) / (float)n;
+  const int rank_blocks = blocks_for(n, kRankRows);
+  auto zero = [&](int count) {
+    hipLaunchKernelGGL(pr_zero, dim3(blocks_for(count, kBlock)), dim3(kBlock), 0, R.stream, counts, count);
+  };
+  auto classify = [&](const int* sample) {
+    hipLaunchKernelGGL(pr_classify, dim3(blocks_for(n, kClassRows)), dim3(kBlock), 0, R.stream, from, n, m, c0, counts,
+                       (Entry*)pch, (BigRow*)pbig, sample);
+  };
   IGX_TRY(timer_start());
   IGX_TRY(ctl_reset(n));
-  hipLaunchKernelGGL(pr_zero, dim3(blocks_for(kSmall, kBlock)), dim3(kBlock), 0, R.stream, counts, kSmall);
+  zero(kSmall);
   if (may) {
-    const int* go = counts + kFlag;
-    const int rank_blocks = blocks_for(n, kRankRows);
     hipLaunchKernelGGL(rank_hist, dim3(rank_blocks), dim3(kBlock), 0, R.stream, g->nindex, n, bins, tile_row);
-    hipLaunchKernelGGL(rank_bins, dim3(1), dim3(kBlock), 0, R.stream, bins, kSmallRow, counts + kFlag + 1,
-                       kHotRanks, m, counts + kFlag);
-    hipLaunchKernelGGL(rank_assign, dim3(rank_blocks), dim3(kBlock), 0, R.stream, g->nindex, n, bins, rank, order,
-                       degree, go);
-    exclusive_scan(degree, nindex1, n + 1, tile_sum, tile_sum + scan_tiles_for(n + 1), R.stream, go);
-    hipLaunchKernelGGL(pr_relabel, dim3(tiles), dim3(kBlock), 0, R.stream, g->nindex, g->nlist, n, m,
-                       (const int*)rank, (const int*)tile_row, (const int*)nindex1, (int*)pl1, go);
+    RankHead* head = (RankHead*)R.d_ctl->aux_ll;
+    hipLaunchKernelGGL(rank_bins, dim3(1), dim3(kBlock), 0, R.stream, bins, 0, (int*)nullptr, kHotRanks, head);
+    hipLaunchKernelGGL(pr_sample, dim3(kSamples / kBlock), dim3(kBlock), 0, R.stream, g->nindex, g->nlist, n, m,
+                       (const int*)tile_row, (const RankHead*)head, (PrSample*)R.d_ctl->sample);
+    IGX_TRY(batch_mark(0));
   }
-  hipLaunchKernelGGL(pr_classify, dim3(blocks_for(n, kClassRows)), dim3(kBlock), 0, R.stream, src, n, c0,
-                     counts, (Entry*)pch, (BigRow*)pbig);
+  classify(may ? R.d_ctl->sample : nullptr);  // under way while the host waits
+  bool hot = false;
+  int* order = nullptr;
+  if (may) {
+    IGX_TRY(batch_wait(0));
+    void *pr1 = nullptr, *pl1 = nullptr;
+    const bool pays = pr_renumber_pays(n, m, R.h_ctl->sample);
+    hot = pays && ws_get(WS_A, sizeof(int) * 5 * ((size_t)n + 1), &pr1) == IGX_OK &&
+          ws_get(WS_E, sizeof(int) * (size_t)m, &pl1) == IGX_OK;
+    if (hot) {
+      int* rank = (int*)pr1;
+      order = rank + n;
+      int* degree = order + n;        // n + 1
+      int* nindex1 = degree + n + 1;  // n + 1
+      hipLaunchKernelGGL(rank_assign, dim3(rank_blocks), dim3(kBlock), 0, R.stream, g->nindex, n, bins, rank, order,
+                         degree);
+      exclusive_scan(degree, nindex1, n + 1, tile_sum, tile_sum + scan_tiles_for(n + 1), R.stream);
+      hipLaunchKernelGGL(pr_relabel, dim3(tiles), dim3(kBlock), 0, R.stream, g->nindex, g->nlist, n, m,
+                         (const int*)rank, (const int*)tile_row, (const int*)nindex1, (int*)pl1);
+      from = PrGraph{nindex1, (const int*)pl1, (float*)(nindex1 + n + 1)};
+    }
+    if (pays) classify(nullptr);
+  }
+  // Iterations to 1e-6 fall with the degree: 14 at an average of 16, 11 at 32,
+  // 8 at 64, 5 at 300.  So a second batch goes in before the first is waited
+  // for up to a degree of 32 (Chung-Lu n = 400 k, degree 16, exponent 2.9:
+  // 1187 -> 1156 us), unless the iterations are so short that the merging
+  // kernel, which the host does not yet know to be idle, costs as much as the
+  // wait (200 x 200 mesh 350 -> 356 us).
+  const int first_batch = (m > 128LL * n) ? 5 : 4;
+  const bool behind = hot || (m <= 32LL * n && m >= (1 << 21));
+  const int unseen = first_batch + (behind ? kAheadRounds : 0);
   int rounds = 0, launches = 0;
   const int rc = run_rounds(
       [&](long long r) {
         float* cur = (r & 1) ? c1 : c0;
         float* nxt = (r & 1) ? c0 : c1;
-        // once a batch of iterations has come back, the kernels that have
-        // nothing to do on this graph are left out
-        const bool known = r >= kFirstBatch;
-        const bool hot = may && (!known || R.h_ctl->aux_ll[1] != 0);
-        const bool big = !known || R.h_ctl->aux_ll[0] != 0;
-        const PrSource& from = hot ? src : given;
+        // once a batch of iterations on the graph as given has come back, the
+        // merging kernel is left out where it has nothing to do
+        const bool big = hot || r < unseen || R.h_ctl->aux_ll[0] != 0;
         if (hot) {
-          hipLaunchKernelGGL(pr_hot_chunks, dim3(2 * R.cus), dim3(kHotBlock), 0, R.stream, src, n, base, cur, nxt,
+          ktimer_begin("pr_hot_chunks");
+          hipLaunchKernelGGL(pr_hot_chunks, dim3(2 * R.cus), dim3(kHotBlock), 0, R.stream, from, n, base, cur, nxt,
                              (const int*)counts, (const Entry*)pch, (Pair*)ppart, R.persist_blocks, R.d_ctl);
+          ktimer_end("pr_hot_chunks");
         }
         ktimer_begin("pr_bal_main");
-        hipLaunchKernelGGL(pr_bal_main, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, from, n, base, cur, nxt,
+        hipLaunchKernelGGL(pr_bal_main, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, from, hot, n, base, cur, nxt,
                            (const int*)counts, (const Entry*)pch, (Pair*)ppart, R.d_ctl);
         ktimer_end("pr_bal_main");
         if (big) {
           hipLaunchKernelGGL(pr_bal_big, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, from, base, nxt,
                              (const BigRow*)pbig, (const int*)counts, (const Pair*)ppart, R.d_ctl);
         }
-        const FinPr fin{P.eps, P.max_iter, counts + 1, from.relabel};
-        if (hot && big) launch_finalize<0x7>(R.persist_blocks, fin);
-        else if (hot) launch_finalize<0x5>(R.persist_blocks, fin);
+        const FinPr fin{P.eps, P.max_iter, counts + 1};
+        if (hot) launch_finalize<0x7>(R.persist_blocks, fin);
         else if (big) launch_finalize<0x3>(R.persist_blocks, fin);
         else launch_finalize<0x1>(R.persist_blocks, fin);
       },
-      P.max_iter, &rounds, &launches, kFirstBatch);
-  if (may && R.h_ctl->aux_ll[1] != 0) {
-    hipLaunchKernelGGL(pr_scores_out, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, R.stream, src, n,
-                       (const int*)order);
+      P.max_iter, &rounds, &launches, first_batch, behind);
+  if (hot) {
+    hipLaunchKernelGGL(pr_scores_out, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, R.stream,
+                       (const float*)from.score, n, (const int*)order, (float*)out);
   }
   IGX_TRY(timer_stop(&info->seconds));
   info->iterations = rounds;
@@ -750,7 +818,7 @@ int style_push(const igx_graph* g, int, void* out, const void*, igx_run_info* in
         ktimer_end("pr_push");
         hipLaunchKernelGGL(pr_push_compute, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, n, base,
                            score, contrib, incoming, R.d_ctl);
-        launch_finalize<0x1>(R.persist_blocks, FinPr{P.eps, P.max_iter, nullptr, nullptr});
+        launch_finalize<0x1>(R.persist_blocks, FinPr{P.eps, P.max_iter, nullptr});
       },
       P.max_iter, &rounds, &launches);
   IGX_TRY(timer_stop(&info->seconds));

@@ -764,10 +764,10 @@ int style_oriented(const igx_graph* g, int, void* out, const void*, igx_run_info
   hipLaunchKernelGGL(tc_clear, dim3(blocks_for(kSmall, kBlock)), dim3(kBlock), 0, R.stream, small, kSmall);
   if (m > 0) {
     hipLaunchKernelGGL(rank_hist, dim3(rank_blocks), dim3(kBlock), 0, R.stream, g->nindex, n, bins, tile_row);
-    hipLaunchKernelGGL(rank_bins, dim3(1), dim3(kBlock), 0, R.stream, bins, kTcShort, heavy, 0, m,
-                       (int*)nullptr);
+    hipLaunchKernelGGL(rank_bins, dim3(1), dim3(kBlock), 0, R.stream, bins, kTcShort, heavy, 0,
+                       (RankHead*)nullptr);
     hipLaunchKernelGGL(rank_assign, dim3(rank_blocks), dim3(kBlock), 0, R.stream, g->nindex, n, bins, rank, order,
-                       (int*)nullptr, (const int*)nullptr);
+                       (int*)nullptr);
     hipLaunchKernelGGL(tc_keep, dim3(tiles), dim3(kBlock), 0, R.stream, g->nindex, g->nlist, n, m, (const int*)rank,
                        (const int*)tile_row, keep, tile_count, bad);
     exclusive_scan(tile_count, tile_off, tiles, tile_sum, tile_sum + scan_tiles_for(scan_n), R.stream);
