@@ -253,11 +253,13 @@ __global__ void __launch_bounds__(kBlock) tc_clear(int* __restrict__ p, int coun
 __global__ void __launch_bounds__(kBlock) tc_keep(const int* __restrict__ nindex, const int* __restrict__ nlist, int n,
                                                    int m, const int* __restrict__ rank,
                                                    const int* __restrict__ tile_row,
-                                                   unsigned long long* __restrict__ keep, int* __restrict__ tile_count,
+                                                   unsigned long long* __restrict__ keep,
+                                                   unsigned short* __restrict__ word_pre, int* __restrict__ tile_count,
                                                    int* __restrict__ bad)
 {
   __shared__ __align__(16) int s_row[kEdgeTile];
   __shared__ int s_red[kWavesPerBlock];
+  __shared__ int s_cnt[kTcWords];
   const int tile = blockIdx.x;
   const int base = tile * kEdgeTile;
   const int r0 = tile_row[tile];
@@ -275,7 +277,6 @@ __global__ void __launch_bounds__(kBlock) tc_keep(const int* __restrict__ nindex
   for (int k = 0; k < kEdgePer; k++) ru[k] = (u[k] >= 0) ? rank[u[k]] : 0;
   edge_tile_rows(nindex, base, r0, r1, s_row, s_red);
   const int head0 = nindex[r0];  // the first row may start before the tile
-  int count = 0;
   bool wrong = false;
   #pragma unroll
   for (int k = 0; k < kEdgePer; k++) {
@@ -288,68 +289,66 @@ __global__ void __launch_bounds__(kBlock) tc_keep(const int* __restrict__ nindex
       if (same && prev[k] >= u[k]) wrong = true;
     }
     const uint64_t word = ballot(kept);
-    if (lane_id() == 0) keep[(size_t)tile * kTcWords + i / kWave] = word;
-    count += __popcll(word);
+    if (lane_id() == 0) {
+      keep[(size_t)tile * kTcWords + i / kWave] = word;
+      s_cnt[i / kWave] = __popcll(word);
+    }
   }
   if (ballot(wrong) != 0 && lane_id() == 0) store_relaxed(bad, 1);
   __syncthreads();
-  if (lane_id() == 0) s_red[threadIdx.x / kWave] = count;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int t = 0;
-    for (int k = 0; k < kWavesPerBlock; k++) t += s_red[k];
-    tile_count[tile] = t;
+  if (threadIdx.x < kWave) {
+    const int lane = lane_id();
+    const int c = (lane < kTcWords) ? s_cnt[lane] : 0;
+    const int incl = wave_incl_scan(c);
+    if (lane < kTcWords) word_pre[(size_t)tile * kTcWords + lane] = (unsigned short)(incl - c);
+    if (lane == kWave - 1) tile_count[tile] = incl;
   }
 }
 
 // The oriented lists, in the order of the rows and of each row: olist by id
 // (sorted within the row), rlist by rank, hlist by rank in 16 bits (kTcHalf for
-// all ranks from there on), and the row starts.
+// all ranks from there on); a workgroup an edge tile.  The workgroups past the
+// tiles write the rows' starts, a thread a row: between two tiles there may be
+// any number of empty rows, which would be walked by the workgroup of one tile
+// (16 million after the edges of an R-MAT 16: 20 ms).
 __global__ void __launch_bounds__(kBlock) tc_orient(const int* __restrict__ nindex, const int* __restrict__ nlist, int n,
-                                                     int m, const int* __restrict__ rank,
-                                                     const int* __restrict__ tile_row,
+                                                     int m, int tiles, const int* __restrict__ rank,
                                                      const unsigned long long* __restrict__ keep,
-                                                     const int* __restrict__ tile_off, int* __restrict__ onidx,
+                                                     const unsigned short* __restrict__ word_pre,
+                                                     const int* __restrict__ tile_off,
+                                                     const int* __restrict__ tile_count, int* __restrict__ onidx,
                                                      int* __restrict__ olist, int* __restrict__ rlist,
                                                      unsigned short* __restrict__ hlist)
 {
-  __shared__ unsigned long long s_word[kTcWords + 1];
-  __shared__ int s_pre[kTcWords + 1];
   const int tile = blockIdx.x;
-  const int base = tile * kEdgeTile;
-  const int lane = lane_id();
-  if (threadIdx.x < kWave) {
-    const unsigned long long word = (lane < kTcWords) ? keep[(size_t)tile * kTcWords + lane] : 0ull;
-    const int c = __popcll(word);
-    const int incl = wave_incl_scan(c);
-    if (lane <= kTcWords) {
-      s_word[lane] = word;
-      s_pre[lane] = incl - c;
+  if (tile >= tiles) {
+    const long long r = (long long)(tile - tiles) * kBlock + threadIdx.x;
+    if (r > n) return;
+    const int e = nindex[r];
+    if (e >= m) {
+      onidx[r] = tile_off[tiles - 1] + tile_count[tiles - 1];
+      return;
     }
+    const int t = e / kEdgeTile, i = e % kEdgeTile;
+    const size_t w = (size_t)t * kTcWords + i / kWave;
+    onidx[r] = tile_off[t] + word_pre[w] + __popcll(keep[w] & ((1ull << (i % kWave)) - 1ull));
+    return;
   }
-  __syncthreads();
+  const int base = tile * kEdgeTile;
   const int off = tile_off[tile];
   #pragma unroll
   for (int k = 0; k < kEdgePer; k++) {
     const int i = k * kBlock + (int)threadIdx.x;
-    const unsigned long long word = s_word[i / kWave];
-    if ((word >> lane) & 1ull) {
+    const size_t w = (size_t)tile * kTcWords + i / kWave;
+    const unsigned long long word = keep[w];
+    if ((word >> lane_id()) & 1ull) {
       const int u = nlist[base + i];
-      const int pos = off + s_pre[i / kWave] + mbcnt(word);
+      const int pos = off + word_pre[w] + mbcnt(word);
       olist[pos] = u;
       const int z = rank[u];
       rlist[pos] = z;
       hlist[pos] = (unsigned short)min(z, kTcHalf);
     }
-  }
-  // starts of the rows that begin in the tile (up to the next tile's first row)
-  const bool last = tile + 1 == (int)gridDim.x;
-  const int first = (tile == 0) ? 0 : tile_row[tile] + 1;
-  const int to = last ? n : tile_row[tile + 1];
-  for (int r = first + (int)threadIdx.x; r <= to; r += kBlock) {
-    const int p = nindex[r] - base;  // 0 .. kEdgeTile
-    const unsigned long long below = s_word[p >> 6] & ((1ull << (p & 63)) - 1ull);
-    onidx[r] = off + s_pre[p >> 6] + __popcll(below);
   }
 }
 
@@ -739,7 +738,8 @@ int style_oriented(const igx_graph* g, int, void* out, const void*, igx_run_info
   // per tile: first row, kept edges, their prefix, and the scan's tile sums
   const int scan_n = tiles > 0 ? tiles : 1;
   IGX_TRY(ws_get(WS_E, sizeof(int) * (3 * (size_t)scan_n + scan_tiles_for(scan_n) + 64), &ptile));
-  IGX_TRY(ws_get(WS_G, sizeof(unsigned long long) * ((size_t)scan_n * kTcWords), &pkeep));
+  // keep bits and their prefix in the tile, per word
+  IGX_TRY(ws_get(WS_G, (sizeof(unsigned long long) + sizeof(unsigned short)) * ((size_t)scan_n * kTcWords), &pkeep));
   IGX_TRY(ws_get(WS_A, sizeof(int) * 2 * (size_t)n, &prank));
   // [0,1] count, [2] sorted check, [3] heavy, then the claim counters and the bins
   constexpr int kSmall = 64 + kGroups * kTcClaimStride + kRankBins;
@@ -752,6 +752,7 @@ int style_oriented(const igx_graph* g, int, void* out, const void*, igx_run_info
   int* tile_off = tile_count + scan_n;
   int* tile_sum = tile_off + scan_n;
   unsigned long long* keep = (unsigned long long*)pkeep;
+  unsigned short* word_pre = (unsigned short*)(keep + (size_t)scan_n * kTcWords);
   int* rank = (int*)prank;
   int* order = rank + n;
   int* small = (int*)psmall;
@@ -769,10 +770,11 @@ int style_oriented(const igx_graph* g, int, void* out, const void*, igx_run_info
     hipLaunchKernelGGL(rank_assign, dim3(rank_blocks), dim3(kBlock), 0, R.stream, g->nindex, n, bins, rank, order,
                        (int*)nullptr);
     hipLaunchKernelGGL(tc_keep, dim3(tiles), dim3(kBlock), 0, R.stream, g->nindex, g->nlist, n, m, (const int*)rank,
-                       (const int*)tile_row, keep, tile_count, bad);
+                       (const int*)tile_row, keep, word_pre, tile_count, bad);
     exclusive_scan(tile_count, tile_off, tiles, tile_sum, tile_sum + scan_tiles_for(scan_n), R.stream);
-    hipLaunchKernelGGL(tc_orient, dim3(tiles), dim3(kBlock), 0, R.stream, g->nindex, g->nlist, n, m, (const int*)rank,
-                       (const int*)tile_row, (const unsigned long long*)keep, (const int*)tile_off, onidx, olist,
+    hipLaunchKernelGGL(tc_orient, dim3(tiles + blocks_for((long long)n + 1, kBlock)), dim3(kBlock), 0, R.stream,
+                       g->nindex, g->nlist, n, m, tiles, (const int*)rank, (const unsigned long long*)keep,
+                       (const unsigned short*)word_pre, (const int*)tile_off, (const int*)tile_count, onidx, olist,
                        rlist, (unsigned short*)phl);
     ktimer_begin("tc_oriented_count");
     hipLaunchKernelGGL(tc_count_long, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, g->nlist,
