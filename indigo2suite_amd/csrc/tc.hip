@@ -796,7 +796,7 @@ int style_oriented(const igx_graph* g, int, void* out, const void*, igx_run_info
   }
   memcpy(&info->count, h, sizeof(unsigned long long));
   info->iterations = 1;
-  info->launches = (m > 0) ? 11 : 2;
+  info->launches = (m > 0) ? 12 : 2;
   return IGX_OK;
 }
 
