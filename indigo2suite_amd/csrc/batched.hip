@@ -82,18 +82,20 @@ __device__ __forceinline__ int wg_excl_scan(int v, int* lds_w, int* tot)
 
 // Walk the edges of the rows given by row_of(k, v, beg, len) for k in [0,
 // count), tile by tile: the workgroup scans the tile's lengths and every
-// thread takes one edge per step.  visit(row, e) for each edge.  All threads
-// must call.
+// thread takes one edge per step.  visit(row, e) for each edge.  Returns the
+// number of edges.  All threads must call.
 template <int B, typename RowOf, typename F>
-__device__ __forceinline__ void wg_expand(int count, RowOf row_of, int* s_excl, int* s_row, int* s_beg, int* s_w,
+__device__ __forceinline__ long long wg_expand(int count, RowOf row_of, int* s_excl, int* s_row, int* s_beg, int* s_w,
                                           F visit)
 {
+  long long edges = 0;
   for (int base = 0; base < count; base += B) {
     const int k = base + (int)threadIdx.x;
     int v = 0, beg = 0, len = 0;
     if (k < count) row_of(k, v, beg, len);
     int total = 0;
     const int ex = wg_excl_scan<B>(len, s_w, &total);
+    edges += total;
     s_excl[threadIdx.x] = ex;
     s_row[threadIdx.x] = v;
     s_beg[threadIdx.x] = beg;
@@ -112,6 +114,7 @@ __device__ __forceinline__ void wg_expand(int count, RowOf row_of, int* s_excl, 
     }
     __syncthreads();
   }
+  return edges;
 }
 
 // Append the lanes with `pred` to a list through an LDS counter, one atomic
@@ -134,16 +137,21 @@ struct WgLds {
   int excl[B], row[B], beg[B];
   int w[B / kWave];
   int next;                   // entries of the list being written
-  unsigned long long edges;   // BFS: their edges
+  unsigned long long edges;   // BFS: edges of the vertices in it
   int pick;                   // CC: the largest sampled component; whether long rows are left
 };
 
 // ------------------------------------------------------------------ BFS ----
 // BFS of one graph from vertex 0 by the whole workgroup (see the file head).
-// The direction follows the single-graph style's rule (top-down -> bottom-up
-// when the frontier's edges exceed 1 / kBatchAlpha of the unvisited ones, back
-// when it has fewer than n / kBatchBeta vertices).  Both directions write the
-// next frontier's queue.
+// Bottom-up while the frontier has at least n / kBatchBeta vertices, from when
+// its edges exceed 1 / kBatchAlpha of the unvisited ones and are at least n.
+// Without the first condition on the way up too, the last levels of a mesh go
+// back and forth, each bottom-up one looking at all n vertices for a few; and
+// only a frontier that meets it has its edges counted, so that a narrow level
+// pays nothing for the choice (16 meshes of 360 x 360, 1024 threads: 4.6 -> 2.9
+// ms; 64 paths of 4096 vertices 14.0 -> 10.3 ms).  Without the last one, meshes
+// with long edges went up, where a row of four is read whole anyway (64 of
+// 100 x 100: 285 -> 217 us).  Both directions write the next frontier's queue.
 constexpr int kBatchWalk = 32;  // neighbours a lane looks at by itself; longer walks take the wave
 constexpr int kBatchAlpha = 14;
 constexpr int kBatchBeta = 24;
@@ -165,7 +173,9 @@ __device__ void bfs_graph(const Arena& A, int g, int* __restrict__ dist_all, int
   int qsize = 1;
   int level = 0;
   bool up = false;
-  long long unvisited = (long long)nidx[n] - nidx[1];
+  const long long m = nidx[n];
+  long long before = 0;    // edges of the vertices visited before the frontier
+  long long frontier = 0;  // edges of the frontier, bottom-up only
   while (qsize > 0) {
     if (threadIdx.x == 0) {
       L.next = 0;
@@ -175,26 +185,30 @@ __device__ void bfs_graph(const Arena& A, int g, int* __restrict__ dist_all, int
     const int* qin = (level & 1) ? q1 : q0;
     int* qout = (level & 1) ? q0 : q1;
     const int nd = level + 1;
-    long long edges = 0;
+    auto add_edges = [&](long long edges) {
+      edges = wave_sum_ll(edges);
+      if (lane_id() == 0 && edges != 0) atomicAdd(&L.edges, (unsigned long long)edges);
+    };
     if (!up) {
-      wg_expand<B>(qsize,
-                   [&](int i, int& v, int& beg, int& len) {
-                     v = qin[i];
-                     beg = nidx[v];
-                     len = nidx[v + 1] - beg;
-                   },
-                   L.excl, L.row, L.beg, L.w, [&](int, int e) {
-                     const int u = nl[e];
-                     bool disc = false;
-                     if (dist[u] == kInf) {
-                       int expected = kInf;
-                       disc = __hip_atomic_compare_exchange_strong(&dist[u], &expected, nd, __ATOMIC_RELAXED,
-                                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                       if (disc) edges += nidx[u + 1] - nidx[u];
-                     }
-                     wg_push(qout, &L.next, disc, u);
-                   });
+      before += wg_expand<B>(qsize,
+                             [&](int i, int& v, int& beg, int& len) {
+                               v = qin[i];
+                               beg = nidx[v];
+                               len = nidx[v + 1] - beg;
+                             },
+                             L.excl, L.row, L.beg, L.w, [&](int, int e) {
+                               const int u = nl[e];
+                               bool disc = false;
+                               if (dist[u] == kInf) {
+                                 int expected = kInf;
+                                 disc = __hip_atomic_compare_exchange_strong(&dist[u], &expected, nd, __ATOMIC_RELAXED,
+                                                                             __ATOMIC_RELAXED,
+                                                                             __HIP_MEMORY_SCOPE_WORKGROUP);
+                               }
+                               wg_push(qout, &L.next, disc, u);
+                             });
     } else {
+      long long edges = 0;
       // kSub vertices per thread and step, their loads and those of the first
       // kFirst neighbours issued together; then up to kBatchWalk neighbours by
       // the thread, the rest of a longer row by the wave, until one of the
@@ -261,15 +275,25 @@ __device__ void bfs_graph(const Arena& A, int g, int* __restrict__ dist_all, int
           wg_push(qout, &L.next, found[s], v);
         }
       }
+      before += frontier;
+      add_edges(edges);
     }
-    edges = wave_sum_ll(edges);
-    if (lane_id() == 0 && edges != 0) atomicAdd(&L.edges, (unsigned long long)edges);
     __syncthreads();
     qsize = L.next;
-    edges = (long long)L.edges;
-    unvisited -= edges;
-    if (!up) up = edges > unvisited / kBatchAlpha;
-    else up = qsize >= n / kBatchBeta;
+    const bool wide = qsize >= n / kBatchBeta;  // uniform
+    if (!up && wide) {
+      long long edges = 0;
+      for (int i = threadIdx.x; i < qsize; i += B) {
+        const int v = qout[i];
+        edges += nidx[v + 1] - nidx[v];
+      }
+      add_edges(edges);
+      __syncthreads();
+    }
+    frontier = (long long)L.edges;
+    const long long unvisited = m - before - frontier;
+    if (wide && unvisited == 0) qsize = 0;  // no vertex with an edge is left
+    up = wide && (up || (frontier > unvisited / kBatchAlpha && frontier >= n));
     level++;
     __syncthreads();
   }
