@@ -559,6 +559,9 @@ __device__ void mis_graph(const Arena& A, int g, int* __restrict__ status_all, i
           }
         }
         const bool undec = sv < 0;
+        // short lists fill few of the places (512 graphs of 200 vertices, 1024
+        // threads: 82 -> 71 us)
+        if (ballot(undec) == 0) continue;  // uniform per wave
         bool more = false;
         if (sv == -2 && result == 0) {
           const uint32_t pv = mis_priority((uint32_t)v);
