@@ -229,6 +229,9 @@ constexpr int kTcWords = kEdgeTile / kWave;      // keep-bit words per tile
 constexpr int kTcShort = 32;                     // lists up to this length: 16-byte groups against a list in LDS
 constexpr int kTcBitWords = 4096;                // bitmap of 2^17 ranks, 16 KB
 constexpr int kTcHashSlice = kTcBitWords / 4;    // list elements per pass where ranks exceed the bitmap
+constexpr int kTcWaveSlots = kTcBitWords / kWavesPerBlock;  // hash slots of a wave there
+constexpr int kTcWaveList = kTcWaveSlots / 8;    // longest list of a wave there
+constexpr int kTcMidLow = 48, kTcMidHigh = 160;  // average degrees at which waves take lists there (tc_count_mid)
 constexpr int kTcPad = 128;                      // elements that 16-byte reads may pass the end of a list array
 constexpr int kTcHalf = 65535;                   // ranks of x up to which the lists are read as 16 bits
 constexpr int kTcSingle = 32768;                 // ranks claimed one by one by the count; beyond, kTcClaim at once
@@ -352,6 +355,125 @@ __global__ void __launch_bounds__(kBlock) tc_orient(const int* __restrict__ nind
   }
 }
 
+// The x of tc_count_long whose rank exceeds the bitmap and whose list has at
+// most kTcWaveList elements, one wave each: the set is a hash table of the
+// wave's own, at most an eighth full, since x's neighbours are fewer than would
+// give the four waves of a workgroup work.  The ranks are dealt out one by one,
+// since lists grow with the rank, and a wave loads the rows of 64 of its x at
+// once.  Bound by the reads of the lists and the chains of their starts.
+// Erdos-Renyi, whole call, a workgroup for each x and now: n = 1 M, average
+// degree 64: 5437 -> 3379 us; n = 512 k, degree 100: 3996 -> 2622 us; n = 250
+// k, degree 50: 954 -> 666 us.  Below kTcMidLow few lists there are longer than
+// kTcShort and the launch costs more than it gives (n = 512 k, degree 40: 892 ->
+// 909 us); from kTcMidHigh a workgroup has work enough (n = 300 k, degree 200:
+// 4069 -> 4205 us).
+__global__ void __launch_bounds__(kBlock) tc_count_mid(const int* __restrict__ nindex, const int* __restrict__ nlist,
+                                                        const int* __restrict__ order, const int* __restrict__ heavy,
+                                                        const int* __restrict__ onidx, const int* __restrict__ rlist,
+                                                        unsigned long long* __restrict__ count)
+{
+  __shared__ unsigned s_tab[kWavesPerBlock][kTcWaveSlots];
+  __shared__ int2 s_ent[kWavesPerBlock][kWave];
+  constexpr int kFirst = kTcBitWords * 32 + 1;  // the lowest such rank
+  constexpr int kPer = kTcWaveList / kWave;
+  const int total = *heavy;
+  const int w = threadIdx.x / kWave;
+  const int lane = lane_id();
+  unsigned* tab = s_tab[w];
+  int2* ents = s_ent[w];
+  const int nwaves = gridDim.x * kWavesPerBlock;
+  const int gw = blockIdx.x * kWavesPerBlock + w;
+  for (int i = lane; i < kTcWaveSlots; i += kWave) tab[i] = 0u;
+  auto slot_of = [](unsigned z) { return (z * 0x9E3779B1u) >> (32 - __builtin_ctz(kTcWaveSlots)); };
+  unsigned long long c = 0;
+  for (long long r0 = kFirst + gw; r0 < total; r0 += (long long)nwaves * kWave) {  // uniform per wave
+    int vx = 0, vbeg = 0, vlen = 0, vnb = 0, vne = 0;
+    const long long r = r0 + (long long)lane * nwaves;
+    if (r < total) {
+      vx = order[r];
+      vbeg = onidx[vx];
+      vlen = onidx[vx + 1] - vbeg;
+      vnb = nindex[vx];
+      vne = nindex[vx + 1];
+    }
+    for (uint64_t todo = ballot(vlen > kTcShort && vlen <= kTcWaveList); todo != 0; todo &= todo - 1) {
+      const int L = __ffsll((unsigned long long)todo) - 1;
+      const int x = __shfl(vx, L, kWave), beg = __shfl(vbeg, L, kWave), len = __shfl(vlen, L, kWave);
+      const int nb = __shfl(vnb, L, kWave), ne = __shfl(vne, L, kWave);
+      const unsigned rx = (unsigned)(r0 + (long long)L * nwaves);
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      unsigned at[kPer];
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) {
+        at[k] = kTcWaveSlots;  // none
+        if (k * kWave + lane < len) {
+          const unsigned z = (unsigned)rlist[beg + k * kWave + lane];
+          unsigned h = slot_of(z);
+          while (atomicCAS(&tab[h], 0u, z + 1u) != 0u) h = (h + 1) % (unsigned)kTcWaveSlots;
+          at[k] = h;
+        }
+      }
+      unsigned found = 0;
+      for (int b0 = nb; b0 < ne; b0 += kWave) {  // uniform
+        int2 ent = make_int2(0, 0);
+        if (b0 + lane < ne) {
+          const int y = nlist[b0 + lane];
+          ent.x = onidx[y];
+          ent.y = onidx[y + 1];
+          const int ylen = ent.y - ent.x;
+          if (ylen > len || (ylen == len && y >= x)) ent.y = ent.x;
+        }
+        const uint64_t some = ballot(ent.y > ent.x);
+        __builtin_amdgcn_wave_barrier();
+        if (ent.y > ent.x) ents[mbcnt(some)] = ent;
+        const int cnt = __popcll(some);
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        int idx = lane >> 4;
+        const int off = (lane & 15) * 4;
+        int pos = 0, end = 0;
+        if (idx < cnt) {
+          pos = ents[idx].x + off;
+          end = ents[idx].y;
+        }
+        while (idx < cnt) {
+          const TcInt4 z4 = *(const TcInt4*)(rlist + pos);
+          #pragma unroll
+          for (int k = 0; k < 4; k++) {
+            // past the list, or above every rank of N+(x): not in the set
+            const unsigned z = (pos + k < end) ? (unsigned)z4[k] : ~0u;
+            if (z < rx) {
+              unsigned h = slot_of(z);
+              unsigned y = tab[h];
+              while (y != 0u && y != z + 1u) {
+                h = (h + 1) % (unsigned)kTcWaveSlots;
+                y = tab[h];
+              }
+              found += (y != 0u) ? 1u : 0u;
+            }
+          }
+          pos += 64;
+          if (pos - off >= end) {
+            idx += 4;
+            if (idx < cnt) {
+              pos = ents[idx].x + off;
+              end = ents[idx].y;
+            }
+          }
+        }
+        __builtin_amdgcn_wave_barrier();
+      }
+      c += found;
+      #pragma unroll
+      for (int k = 0; k < kPer; k++) {
+        if (at[k] < kTcWaveSlots) tab[at[k]] = 0u;
+      }
+    }
+  }
+  wave_add_count(count, c);
+}
+
 // Edges with an endpoint whose list is longer than kTcShort, at the endpoint
 // x with the longer list (ties: the larger id), one workgroup per x in rank
 // order, hubs first, claimed one at a time while they are heavy (four hubs at
@@ -380,12 +502,13 @@ __global__ void __launch_bounds__(kBlock) tc_count_long(const int* __restrict__ 
                                                          const int* __restrict__ heavy,
                                                          const int* __restrict__ onidx, const int* __restrict__ rlist,
                                                          const unsigned short* __restrict__ hlist,
-                                                         int* __restrict__ claim,
+                                                         int* __restrict__ claim, bool mid,
                                                          unsigned long long* __restrict__ count)
 {
   __shared__ unsigned s_set[kTcBitWords];
   __shared__ int2 s_ent[kWavesPerBlock][kWave];
   __shared__ int s_claim;
+  __shared__ int4 s_row[kTcClaim];  // x, the start and length of its list
   const int tid = threadIdx.x;
   const int w = tid / kWave;
   const int lane = lane_id();
@@ -402,14 +525,33 @@ __global__ void __launch_bounds__(kBlock) tc_count_long(const int* __restrict__ 
     const long long rank0 = (unit < kTcSingle) ? unit : kTcSingle + (unit - kTcSingle) * kTcClaim;
     const int ranks = (unit < kTcSingle) ? 1 : kTcClaim;
     if (rank0 >= total) break;
+    // ranks beyond the bitmap (uniform); most lists are tc_count_mid's there, so the unit's are looked at at once
+    const bool skim = mid && rank0 + ranks - 1 > kTcBitWords * 32;
+    if (skim && tid < ranks) {
+      int4 row = make_int4(0, 0, 0, 0);
+      if (rank0 + tid < total) {
+        row.x = order[rank0 + tid];
+        row.y = onidx[row.x];
+        row.z = onidx[row.x + 1] - row.y;
+      }
+      s_row[tid] = row;
+    }
+    if (skim) __syncthreads();
     for (int q = 0; q < ranks; q++) {
       const int rx = (int)rank0 + q;
-      if (rx >= total) break;
-      const int x = order[rx];
-      const int beg = onidx[x], len = onidx[x + 1] - beg;
-      if (len <= kTcShort) continue;
-      const int nb = nindex[x], ne = nindex[x + 1];
+      int x = 0, beg = 0, len = 0;
+      if (skim) {
+        x = s_row[q].x;
+        beg = s_row[q].y;
+        len = s_row[q].z;
+      } else if (rx < total) {
+        x = order[rx];
+        beg = onidx[x];
+        len = onidx[x + 1] - beg;
+      }
       const bool bits = rx <= kTcBitWords * 32;
+      if (len <= ((mid && !bits) ? kTcWaveList : kTcShort)) continue;
+      const int nb = nindex[x], ne = nindex[x + 1];
       const bool half = rx <= kTcHalf;
       const int passes = bits ? 1 : (len + kTcHashSlice - 1) / kTcHashSlice;
       for (int ps = 0; ps < passes; ps++) {
@@ -761,6 +903,7 @@ int style_oriented(const igx_graph* g, int, void* out, const void*, igx_run_info
   int* heavy = small + 3;
   int* claim = small + 64;
   int* bins = claim + kGroups * kTcClaimStride;
+  const bool mid = n > kTcBitWords * 32 + 1 && m / kTcMidLow >= n && m / kTcMidHigh < n;
   IGX_TRY(timer_start());
   hipLaunchKernelGGL(tc_clear, dim3(blocks_for(kSmall, kBlock)), dim3(kBlock), 0, R.stream, small, kSmall);
   if (m > 0) {
@@ -779,7 +922,11 @@ int style_oriented(const igx_graph* g, int, void* out, const void*, igx_run_info
     ktimer_begin("tc_oriented_count");
     hipLaunchKernelGGL(tc_count_long, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, g->nlist,
                        (const int*)order, (const int*)heavy, (const int*)onidx, (const int*)rlist,
-                       (const unsigned short*)phl, claim, count);
+                       (const unsigned short*)phl, claim, mid, count);
+    if (mid) {
+      hipLaunchKernelGGL(tc_count_mid, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, g->nlist,
+                         (const int*)order, (const int*)heavy, (const int*)onidx, (const int*)rlist, count);
+    }
     hipLaunchKernelGGL(tc_count_short, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, (const int*)onidx,
                        (const int*)olist, n, count);
     ktimer_end("tc_oriented_count");
@@ -796,7 +943,7 @@ int style_oriented(const igx_graph* g, int, void* out, const void*, igx_run_info
   }
   memcpy(&info->count, h, sizeof(unsigned long long));
   info->iterations = 1;
-  info->launches = (m > 0) ? 12 : 2;
+  info->launches = (m > 0) ? (mid ? 13 : 12) : 2;
   return IGX_OK;
 }
 
