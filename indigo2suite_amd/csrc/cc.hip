@@ -227,10 +227,13 @@ __global__ void __launch_bounds__(kBlock) cc_vdata_push(const int* __restrict__ 
 // One thread per worklist edge; when dst's label drops, all of dst's edges
 // are queued at once (NonDup per source vertex, see bfs_edata_push) and
 // written wave-cooperatively.
+constexpr int kCcOneByOne = 8;   // items per thread up to which a list is taken one by one
+constexpr int kCcOneDegree = 8;  // average degree from which it is
 __global__ void __launch_bounds__(kBlock) cc_edata_push(const int* __restrict__ nindex,
                                                          const int* __restrict__ nlist, const int* __restrict__ sp,
                                                          int* __restrict__ label, int* __restrict__ wl0,
-                                                         int* __restrict__ wl1, int* __restrict__ vstamp, Ctl* ctl)
+                                                         int* __restrict__ wl1, int* __restrict__ vstamp, bool by_one,
+                                                         Ctl* ctl)
 {
   __shared__ ListLds s_list;
   if (round_done(ctl)) return;
@@ -241,7 +244,15 @@ __global__ void __launch_bounds__(kBlock) cc_edata_push(const int* __restrict__ 
   int* wl_out = p ? wl0 : wl1;
   int* out_count = &ctl->wl_count[p ^ 1];
   const int tag = iter + 1;
-  const int per = list_items_per_thread(count);
+  // A label that an item lowers goes on in the same round, if the items after it
+  // are read then.  On a graph of many edges a vertex that saves a round or two
+  // of five, so there a list of a few items a thread is taken one by one
+  // (Erdos-Renyi, average degree 16, n = 65,536: 404 -> 319 us, n = 200 k: 660
+  // -> 460 us).  With few edges a vertex (512 x 512 mesh with long edges, one by
+  // one 1607 us, four at once 1357), or many items (R-MAT 18 457 / 449 us), the
+  // loads under way together are worth more.
+  const bool one = by_one && count <= kCcOneByOne * (int)(gridDim.x * kBlock);
+  const int per = one ? 1 : list_items_per_thread(count);
   const long long step = (long long)gridDim.x * kBlock * per;
   with_list_items(per, [&](auto items) {
     constexpr int kPer = decltype(items)::value;
@@ -690,7 +701,7 @@ int style_data_push(const igx_graph* g, int, void* out, const void* aux, igx_run
       [&](long long) {
         if (EDGE) {
           hipLaunchKernelGGL(cc_edata_push, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, g->nlist,
-                             sp, label, wl0, wl1, stamp, R.d_ctl);
+                             sp, label, wl0, wl1, stamp, g->edges / kCcOneDegree >= g->nodes, R.d_ctl);
         } else {
           hipLaunchKernelGGL(cc_vdata_push, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, g->nlist,
                              label, wl0, wl1, stamp, R.d_ctl);
