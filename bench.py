@@ -12,13 +12,14 @@ value = whole-step throughput: 2 * m / (time of one SSSP + one CC), in
 GTEPS with m the directed edge count (the reference's 1e-9 * edges / runtime
 formula, bfs_vertex_cuda.h:163, applied to the two runs of a step).
 
-roofline: the SSSP round kernel (sssp_do_round), the step's dominant kernel,
-timed with HIP events on the library stream over the timed steps.  Its
+roofline: the SSSP rounds (sssp_do_round, the step's dominant kernel, and the
+kernel that ends a round and runs the narrow rounds after it), timed with HIP
+events on the library stream over the timed steps.  Their
 algorithmic bytes are the style-independent SSSP figure, 12 bytes per
 directed edge (neighbour id, weight, neighbour distance) and 12 per vertex
 (row offsets, distance read and write): 12m + 12n + 4 per run, spread over
 the run's launches.  achieved = those bytes / the summed launch time.  The
-bytes the kernel's executed work touches (8 per edge scanned: id and weight;
+bytes their executed work touches (8 per edge scanned: id and weight;
 4 per neighbour distance gathered; 12 per row visited; counted on the device)
 are reported beside it, as is the copy-calibrated HBM traffic per launch
 from rocprofv3.
@@ -380,9 +381,9 @@ def main():
                                            "gteps": round(m / named.seconds * 1e-9, 3),
                                            "iterations": named.iterations}
 
-    # roofline of the SSSP round kernel: the style-independent algorithmic
-    # bytes of the timed runs (12m + 12n + 4 each) over the summed duration of
-    # its launches in those runs
+    # roofline of the SSSP rounds: the style-independent algorithmic bytes of
+    # the timed runs (12m + 12n + 4 each) over the summed duration of the
+    # launched rounds in those runs, each with the narrow rounds after it
     launches = max(hook_n.value, 1)
     total_s = hook_ms.value * 1e-3
     alg_total = algorithmic_bytes("sssp", n, m) * args.steps

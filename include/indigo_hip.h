@@ -117,7 +117,12 @@ int igx_last_run_info(igx_run_info* info);
  * events on the library stream; igx_profile_read() waits for the stream and
  * returns the summed duration and the number of timed launches, then resets.
  * Tags: "uf_hook", "af_link_rest", "bfs_do_level", "sssp_do_round", "sssp_bal_round", "pr_bal_main",
- * "tc_oriented_count", "mis_vdata_pull".  NULL or "" disables. */
+ * "pr_hot_chunks", "tc_oriented_count", "mis_vdata_pull", "mis_resume_pull".  NULL or "" disables.
+ * Where a step of an algorithm is shared by several kernels the tag names the
+ * step: "bfs_do_level" and "sssp_do_round" include the kernel that ends the
+ * level or round and runs the narrow ones that follow, "pr_bal_main" the sums
+ * of the longer rows of a renumbered graph ("pr_hot_chunks" times them alone),
+ * "tc_oriented_count" both counts. */
 int igx_profile_kernel(const char* tag);
 int igx_profile_read(double* total_ms, int* launches);
 

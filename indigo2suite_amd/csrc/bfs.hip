@@ -906,6 +906,9 @@ int style_do_hybrid(const igx_graph* g, int src, void* out, const void*, igx_run
     hipLaunchKernelGGL(bfs_do_finish, dim3(1), dim3(kFinBlock), 0, R.stream, g->nindex, g->nlist, dist, q0, q1,
                        (unsigned*)pb, words, R.persist_blocks, after_level, R.d_ctl);
   };
+  // the timed region of a level is the level and the narrow ones that the
+  // kernel that ends it runs; the first has those before it too
+  ktimer_begin("bfs_do_level");
   finish(false);
   int rounds = 0, launches = 0;
   const int rc = run_rounds(
@@ -914,8 +917,8 @@ int style_do_hybrid(const igx_graph* g, int src, void* out, const void*, igx_run
         hipLaunchKernelGGL(bfs_do_level, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, g->nlist,
                            g->nodes, dist, q0, q1, (const Entry*)pq, (const int*)pc, (unsigned*)pb, words,
                            g->edges / 16 < g->nodes, R.d_ctl);
-        ktimer_end("bfs_do_level");
         finish(true);
+        ktimer_end("bfs_do_level");
       },
       (long long)g->nodes + 2, &rounds, &launches, g->edges < kFewEdges ? 4 : 6);
   IGX_TRY(timer_stop(&info->seconds));

@@ -759,13 +759,13 @@ int style_balanced(const igx_graph* g, int, void* out, const void*, igx_run_info
         // once a batch of iterations on the graph as given has come back, the
         // merging kernel is left out where it has nothing to do
         const bool big = hot || r < unseen || R.h_ctl->aux_ll[0] != 0;
+        ktimer_begin("pr_bal_main");
         if (hot) {
           ktimer_begin("pr_hot_chunks");
           hipLaunchKernelGGL(pr_hot_chunks, dim3(2 * R.cus), dim3(kHotBlock), 0, R.stream, from, n, base, cur, nxt,
                              (const int*)counts, (const Entry*)pch, (Pair*)ppart, R.persist_blocks, R.d_ctl);
           ktimer_end("pr_hot_chunks");
         }
-        ktimer_begin("pr_bal_main");
         hipLaunchKernelGGL(pr_bal_main, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, from, hot, n, base, cur, nxt,
                            (const int*)counts, (const Entry*)pch, (Pair*)ppart, R.d_ctl);
         ktimer_end("pr_bal_main");
