@@ -143,22 +143,6 @@ __device__ __forceinline__ int wave_push_slot(int* counter, bool pred)
   return pred ? base + mbcnt(mask) : -1;
 }
 
-// Variable count per lane: lane reserves `cnt` consecutive slots.
-__device__ __forceinline__ int wave_reserve(int* counter, int cnt)
-{
-  const int incl = wave_incl_scan(cnt);
-  const int total = wave_bcast(incl, kWave - 1);
-  int base = 0;
-  if (total > 0) {
-    // the last lane always exists in a full wave; use the highest active lane
-    const uint64_t act = ballot(true);
-    const int last = 63 - __clzll((long long)act);
-    if (lane_id() == last) base = atomicAdd(counter, total);
-    base = wave_bcast(base, last);
-  }
-  return base + incl - cnt;
-}
-
 // --------------------------------------------------------- control ------
 // One control block per run.  `done` is checked by every round kernel at entry
 // so the host can enqueue rounds speculatively; the last block to finish a
@@ -292,10 +276,10 @@ __device__ __forceinline__ void round_partial_d(Ctl* ctl, int slot, double v, do
 }
 
 // Round kernel side of the common topology-driven rule: any lane with `again`
-// asks for another round.  A wave stores the flag only if it reads 0, and
-// plainly (the kernel boundary publishes it): agent-scope stores of thousands
-// of waves to the one address take about 11 ns each, which was 60-100 us of
-// every round in which most waves had something pending.
+// asks for another round.  A wave reads the flag first, past the caches (the
+// pointer is volatile), and stores only if it is 0: stores of thousands of
+// waves to the one address take about 11 ns each, which was 60-100 us of every
+// round in which most waves had something pending.
 __device__ __forceinline__ void raise_flag(Ctl* ctl, bool again)
 {
   const uint64_t any = ballot(again);
@@ -431,23 +415,6 @@ __global__ void __launch_bounds__(kFinBlock) round_finalize(Ctl* ctl, int nparts
   if (threadIdx.x == 0) fin(ctl, tot);
 }
 
-
-// finalizers of the two common round rules
-struct FinFlag {
-  __device__ void operator()(Ctl* ctl, const RoundTotals&) const { finalize_flag_round(ctl); }
-};
-struct FinWorklist {
-  __device__ void operator()(Ctl* ctl, const RoundTotals&) const { finalize_worklist_round(ctl); }
-};
-
-// Visiting order for one-wave-per-vertex loops: k -> (k * mult) mod n with
-// mult coprime to n is a permutation of [0, n).  R-MAT's hubs sit at ids with
-// many zero bits, so a plain round-robin (v = wave + k * waves) hands dozens of
-// them to the same wave; the multiplicative order spreads them out.
-__device__ __forceinline__ int spread_vertex(int k, int n, unsigned mult)
-{
-  return (int)(((unsigned long long)(unsigned)k * mult) % (unsigned long long)n);
-}
 
 // MIS priority: the reference's integer hash of (v + 712313887), compared as
 // unsigned (mis_vertex_omp.h:127-132 and codes/omp MIS init).

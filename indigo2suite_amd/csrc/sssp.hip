@@ -303,8 +303,8 @@ __global__ void __launch_bounds__(kBlock) sssp_edata_seed(int src, const int* __
 // when dst improves; every edge of dst is queued together, so the NonDup test
 // is kept per source vertex (vstamp[dst] == tag: dst's edges are queued this
 // round), which admits exactly the edges the per-edge stamps admit.  The
-// queueing itself is wave-cooperative (wave_push_edge_ranges): a hub's edge
-// ids are written 64 per step instead of one by one by the improving thread.
+// workgroup queues them together (block_push_edge_ranges): a hub's edge ids
+// are written 64 per step instead of one by one by the improving thread.
 // RW: the racy load/store may lose an update to a concurrent store, so the
 // edge itself is queued again (per-edge stamp estamp).
 template <bool RW>
@@ -993,6 +993,11 @@ struct FinSsspDo {
       // With many claims a wave they are left out (R-MAT 22, three pull
       // rounds 508 + 365 + 341 -> 476 + 341 + 205 us); with few, the later
       // ones fill the ends of the earlier (R-MAT 20 without them 360 -> 387).
+      // Whole runs on graphs beyond the line, with all workgroups and without
+      // the late ones: R-MAT 22 1757 and 1530 us, Chung-Lu n = 4 M, degree 32,
+      // 2640 and 2515; alike within 1% on Erdos-Renyi graphs of 2 to 8 M
+      // vertices, degree 16 and 32, R-MAT 23 of edge factor 8 and a 6000 x 6000
+      // mesh, which have few long rows.
       if (ctl->mode == 1 && claims >= kClaimsPerWave * resident * kWavesPerBlock) act = min(act, resident);
       if (act >= nblocks) act = 0;
     }
