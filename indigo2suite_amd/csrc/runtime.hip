@@ -494,7 +494,8 @@ int igx_init(int device)
   IGX_HIP(hipMalloc((void**)&g_rt.d_ctl, kCtlAllocBytes));
   IGX_HIP(hipMemset(g_rt.d_ctl, 0, kCtlAllocBytes));
   for (hipEvent_t& e : g_rt.ev_batch) IGX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  IGX_HIP(hipHostMalloc((void**)&g_rt.h_ctl, 3 * sizeof(Ctl), hipHostMallocDefault));
+  // written by ctl_publish: coherent, so that its stores are the host's when the event after them is past
+  IGX_HIP(hipHostMalloc((void**)&g_rt.h_ctl, 3 * sizeof(Ctl), hipHostMallocCoherent | hipHostMallocMapped));
   memset(g_rt.h_ctl, 0, 3 * sizeof(Ctl));
   IGX_TRY(batch_noalloc_setup(device));
   g_rt.ready = true;
