@@ -66,10 +66,10 @@ int ws_get(int slot, size_t bytes, void** ptr);
 // the stream behind the one that is waited for: at most two of them run empty,
 // where batches that doubled up to 64 cost PageRank up to 15 empty rounds of
 // three launches.  An empty round and a copy of the control block cost about
-// the same (5 us of the host's time), so with r rounds so far a batch of
-// sqrt(r / 2) balances the two empty batches of the end against the copies: a
-// run of 501 rounds enqueues 529, where batches of an eighth of the rounds, up
-// to 64, enqueued 583 (SSSP on a path of 500 vertices 4.4 -> 4.0 ms).
+// the same (5 us of the host's time), so batches of the square root of the
+// rounds so far balance the empty ones of the end against the copies: a run of
+// 501 rounds enqueues 530, where batches of an eighth of the rounds, up to 64,
+// enqueued 583 (SSSP on a path of 500 vertices 4.4 -> 4.0 ms).
 // After each batch the run also stops, with IGX_ERR_TIMEOUT, once the host
 // clock since timer_start() passes the time limit set by igx_set_time_limit;
 // what is in the stream then, two batches of at most kMaxAhead rounds, is
@@ -113,7 +113,7 @@ int run_rounds(F launch, long long max_rounds, int* rounds_done, int* launches, 
     }
     // two batches behind the first one, then one for each that came back
     while (!stop && batches - waited < 2 && launched < max_rounds) {
-      const long long b = (long long)std::sqrt((double)launched / 2.0);
+      const long long b = (long long)std::sqrt((double)launched);
       IGX_TRY(enqueue(b < kAheadRounds ? kAheadRounds : (b < kMaxAhead ? b : kMaxAhead)));
     }
   }
