@@ -80,41 +80,53 @@ __device__ __forceinline__ int wg_excl_scan(int v, int* lds_w, int* tot)
   return off + incl - v;
 }
 
-// Walk the edges of the rows given by row_of(k, v, beg, len) for k in [0,
-// count), tile by tile: the workgroup scans the tile's lengths and every
-// thread takes one edge per step.  visit(row, e) for each edge.  Returns the
-// number of edges.  All threads must call.
+// The rows given by row_of(k, v, beg, len) for k in [base, base + B) and below
+// count, as a tile in LDS: returns the number of their edges.  All threads must
+// call; the tile before has to be done with.
+template <int B, typename RowOf>
+__device__ __forceinline__ int wg_tile(int count, int base, RowOf row_of, int* s_excl, int* s_row, int* s_beg, int* s_w)
+{
+  const int k = base + (int)threadIdx.x;
+  int v = 0, beg = 0, len = 0;
+  if (k < count) row_of(k, v, beg, len);
+  int total = 0;
+  const int ex = wg_excl_scan<B>(len, s_w, &total);
+  s_excl[threadIdx.x] = ex;
+  s_row[threadIdx.x] = v;
+  s_beg[threadIdx.x] = beg;
+  __syncthreads();
+  return total;
+}
+
+// Walk the `total` edges of the tile, an edge a thread and step: visit(row, e).
+template <int B, typename F>
+__device__ __forceinline__ void wg_walk(int total, const int* s_excl, const int* s_row, const int* s_beg, F visit)
+{
+  for (int tb = 0; tb < total; tb += B) {
+    const int t = tb + (int)threadIdx.x;
+    if (t < total) {
+      int lo = 0, hi = B;
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (s_excl[mid] <= t) lo = mid;
+        else hi = mid;
+      }
+      visit(s_row[lo], s_beg[lo] + (t - s_excl[lo]));
+    }
+  }
+}
+
+// Walk the edges of all rows k in [0, count), tile by tile.  All threads must
+// call.
 template <int B, typename RowOf, typename F>
-__device__ __forceinline__ long long wg_expand(int count, RowOf row_of, int* s_excl, int* s_row, int* s_beg, int* s_w,
+__device__ __forceinline__ void wg_expand(int count, RowOf row_of, int* s_excl, int* s_row, int* s_beg, int* s_w,
                                           F visit)
 {
-  long long edges = 0;
   for (int base = 0; base < count; base += B) {
-    const int k = base + (int)threadIdx.x;
-    int v = 0, beg = 0, len = 0;
-    if (k < count) row_of(k, v, beg, len);
-    int total = 0;
-    const int ex = wg_excl_scan<B>(len, s_w, &total);
-    edges += total;
-    s_excl[threadIdx.x] = ex;
-    s_row[threadIdx.x] = v;
-    s_beg[threadIdx.x] = beg;
-    __syncthreads();
-    for (int tb = 0; tb < total; tb += B) {
-      const int t = tb + (int)threadIdx.x;
-      if (t < total) {
-        int lo = 0, hi = B;
-        while (hi - lo > 1) {
-          const int mid = (lo + hi) >> 1;
-          if (s_excl[mid] <= t) lo = mid;
-          else hi = mid;
-        }
-        visit(s_row[lo], s_beg[lo] + (t - s_excl[lo]));
-      }
-    }
+    const int total = wg_tile<B>(count, base, row_of, s_excl, s_row, s_beg, s_w);
+    wg_walk<B>(total, s_excl, s_row, s_beg, visit);
     __syncthreads();
   }
-  return edges;
 }
 
 // Append the lanes with `pred` to a list through an LDS counter, one atomic
@@ -143,18 +155,21 @@ struct WgLds {
 
 // ------------------------------------------------------------------ BFS ----
 // BFS of one graph from vertex 0 by the whole workgroup (see the file head).
-// Bottom-up while the frontier has at least n / kBatchBeta vertices, from when
-// its edges exceed 1 / kBatchAlpha of the unvisited ones and are at least n.
-// Without the first condition on the way up too, the last levels of a mesh go
-// back and forth, each bottom-up one looking at all n vertices for a few; and
-// only a frontier that meets it has its edges counted, so that a narrow level
-// pays nothing for the choice (16 meshes of 360 x 360, 1024 threads: 4.6 -> 2.9
-// ms; 64 paths of 4096 vertices 14.0 -> 10.3 ms).  Without the last one, meshes
-// with long edges went up, where a row of four is read whole anyway (64 of
-// 100 x 100: 285 -> 217 us).  Both directions write the next frontier's queue.
+// Bottom-up from when the frontier's edges exceed 1 / kBatchAlpha of the
+// unvisited ones and are at least n, while it has at least n / kBatchBeta
+// vertices.  Without the bound by n, the last levels of a mesh went back and
+// forth, each bottom-up one looking at all n vertices for a few, and meshes
+// with long edges went up where a row of four is read whole anyway.  The edges
+// are counted by the scan that a top-down level begins with, beyond its first
+// tile only for frontiers of n / kBatchLook vertices, so a narrow level pays
+// nothing for the choice.  1024 threads, by the first condition alone and now:
+// 16 meshes of 360 x 360 4.6 -> 2.9 ms, 64 of 100 x 100 with long edges 286 ->
+// 210 us, 64 paths of 4096 vertices 14.1 -> 10.5 ms.  Both directions write the
+// next frontier's queue.
 constexpr int kBatchWalk = 32;  // neighbours a lane looks at by itself; longer walks take the wave
 constexpr int kBatchAlpha = 14;
 constexpr int kBatchBeta = 24;
+constexpr int kBatchLook = 64;
 
 template <int B>
 __device__ void bfs_graph(const Arena& A, int g, int* __restrict__ dist_all, int* __restrict__ queue_all, WgLds<B>& L)
@@ -175,7 +190,7 @@ __device__ void bfs_graph(const Arena& A, int g, int* __restrict__ dist_all, int
   bool up = false;
   const long long m = nidx[n];
   long long before = 0;    // edges of the vertices visited before the frontier
-  long long frontier = 0;  // edges of the frontier, bottom-up only
+  long long frontier = 0;  // edges of the frontier, if bottom-up
   while (qsize > 0) {
     if (threadIdx.x == 0) {
       L.next = 0;
@@ -190,24 +205,53 @@ __device__ void bfs_graph(const Arena& A, int g, int* __restrict__ dist_all, int
       if (lane_id() == 0 && edges != 0) atomicAdd(&L.edges, (unsigned long long)edges);
     };
     if (!up) {
-      before += wg_expand<B>(qsize,
-                             [&](int i, int& v, int& beg, int& len) {
-                               v = qin[i];
-                               beg = nidx[v];
-                               len = nidx[v + 1] - beg;
-                             },
-                             L.excl, L.row, L.beg, L.w, [&](int, int e) {
-                               const int u = nl[e];
-                               bool disc = false;
-                               if (dist[u] == kInf) {
-                                 int expected = kInf;
-                                 disc = __hip_atomic_compare_exchange_strong(&dist[u], &expected, nd, __ATOMIC_RELAXED,
-                                                                             __ATOMIC_RELAXED,
-                                                                             __HIP_MEMORY_SCOPE_WORKGROUP);
-                               }
-                               wg_push(qout, &L.next, disc, u);
-                             });
-    } else {
+      auto row_of = [&](int i, int& v, int& beg, int& len) {
+        v = qin[i];
+        beg = nidx[v];
+        len = nidx[v + 1] - beg;
+      };
+      int total = wg_tile<B>(qsize, 0, row_of, L.excl, L.row, L.beg, L.w);
+      bool more = true;  // uniform
+      if (qsize >= n / kBatchLook) {
+        frontier = total;
+        if (qsize > B) {
+          long long edges = 0;
+          for (int i = B + (int)threadIdx.x; i < qsize; i += B) {
+            const int v = qin[i];
+            edges += nidx[v + 1] - nidx[v];
+          }
+          add_edges(edges);
+          __syncthreads();
+          frontier += (long long)L.edges;
+          __syncthreads();
+          if (threadIdx.x == 0) L.edges = 0;
+          __syncthreads();
+        }
+        const long long unvisited = m - before - frontier;
+        more = unvisited > 0;  // else no vertex with an edge is left
+        up = more && frontier > unvisited / kBatchAlpha && frontier >= n;
+      }
+      if (!up && more) {
+        for (int base = 0;;) {
+          before += total;
+          wg_walk<B>(total, L.excl, L.row, L.beg, [&](int, int e) {
+            const int u = nl[e];
+            bool disc = false;
+            if (dist[u] == kInf) {
+              int expected = kInf;
+              disc = __hip_atomic_compare_exchange_strong(&dist[u], &expected, nd, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                          __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+            wg_push(qout, &L.next, disc, u);
+          });
+          base += B;
+          if (base >= qsize) break;
+          __syncthreads();
+          total = wg_tile<B>(qsize, base, row_of, L.excl, L.row, L.beg, L.w);
+        }
+      }
+    }
+    if (up) {
       long long edges = 0;
       // kSub vertices per thread and step, their loads and those of the first
       // kFirst neighbours issued together; then up to kBatchWalk neighbours by
@@ -280,20 +324,10 @@ __device__ void bfs_graph(const Arena& A, int g, int* __restrict__ dist_all, int
     }
     __syncthreads();
     qsize = L.next;
-    const bool wide = qsize >= n / kBatchBeta;  // uniform
-    if (!up && wide) {
-      long long edges = 0;
-      for (int i = threadIdx.x; i < qsize; i += B) {
-        const int v = qout[i];
-        edges += nidx[v + 1] - nidx[v];
-      }
-      add_edges(edges);
-      __syncthreads();
+    if (up) {
+      frontier = (long long)L.edges;
+      up = qsize >= n / kBatchBeta;
     }
-    frontier = (long long)L.edges;
-    const long long unvisited = m - before - frontier;
-    if (wide && unvisited == 0) qsize = 0;  // no vertex with an edge is left
-    up = wide && (up || (frontier > unvisited / kBatchAlpha && frontier >= n));
     level++;
     __syncthreads();
   }
