@@ -70,6 +70,11 @@ int ws_get(int slot, size_t bytes, void** ptr);
 // rounds so far balance the empty ones of the end against the copies: a run of
 // 501 rounds enqueues 530, where batches of an eighth of the rounds, up to 64,
 // enqueued 583 (SSSP on a path of 500 vertices 4.4 -> 4.0 ms).
+// While it enqueues, the host also looks at the pinned copies and stops once
+// one says that the run is over: where rounds are shorter than their
+// submission, the batch ahead was most of the time after the last round
+// (Erdos-Renyi n = 16384, average degree 8, BFS entry on a slow host: 194 ->
+// 162 us, 12 rounds enqueued for 8 -> 9).
 // After each batch the run also stops, with IGX_ERR_TIMEOUT, once the host
 // clock since timer_start() passes the time limit set by igx_set_time_limit;
 // what is in the stream then, two batches of at most kMaxAhead rounds, is
@@ -84,6 +89,8 @@ constexpr int kMaxAhead = 32;
 bool past_time_limit();
 int batch_mark(int slot);    // copy the control block to slot's pinned mirror, behind the work so far
 int batch_wait(int slot);    // wait for it and make it *R.h_ctl
+void batch_forget();         // before the first batch of a run
+bool batch_saw_end();        // a copy already reads "done" (a hint: the copy may not be whole)
 template <typename F>
 int run_rounds(F launch, long long max_rounds, int* rounds_done, int* launches, int first_batch = 2,
                bool behind_first = false)
@@ -91,14 +98,19 @@ int run_rounds(F launch, long long max_rounds, int* rounds_done, int* launches, 
   Runtime& R = rt();
   long long launched = 0, batches = 0;
   auto enqueue = [&](long long batch) -> int {
-    const long long k = (launched + batch > max_rounds) ? (max_rounds - launched) : batch;
+    long long k = (launched + batch > max_rounds) ? (max_rounds - launched) : batch;
     for (long long i = 0; i < k; i++) {
+      if (batch_saw_end()) {
+        k = i;  // the run is over: what is left of the batch would run empty
+        break;
+      }
       launch(launched + i);
     }
     IGX_HIP(hipGetLastError());
     launched += k;
     return batch_mark((int)(batches++ & 1));
   };
+  batch_forget();
   IGX_TRY(enqueue(first_batch));
   if (behind_first && launched < max_rounds) IGX_TRY(enqueue(kAheadRounds));
   long long waited = 0;
@@ -112,7 +124,7 @@ int run_rounds(F launch, long long max_rounds, int* rounds_done, int* launches, 
       break;
     }
     // two batches behind the first one, then one for each that came back
-    while (!stop && batches - waited < 2 && launched < max_rounds) {
+    while (!stop && batches - waited < 2 && launched < max_rounds && (batches == waited || !batch_saw_end())) {
       const long long b = (long long)std::sqrt((double)launched);
       IGX_TRY(enqueue(b < kAheadRounds ? kAheadRounds : (b < kMaxAhead ? b : kMaxAhead)));
     }

@@ -384,6 +384,7 @@ void ktimer_end(const char* tag)
 
 int batch_mark(int slot)
 {
+  ((volatile Ctl*)g_rt.h_ctl)[1 + slot].done = 0;
   hipLaunchKernelGGL(ctl_publish, dim3(1), dim3(64), 0, g_rt.stream, (const int*)g_rt.d_ctl,
                      (int*)(g_rt.h_ctl + 1 + slot));
   IGX_HIP(hipGetLastError());
@@ -396,6 +397,19 @@ int batch_wait(int slot)
   IGX_HIP(hipEventSynchronize(g_rt.ev_batch[slot]));
   *g_rt.h_ctl = g_rt.h_ctl[1 + slot];
   return IGX_OK;
+}
+
+void batch_forget()
+{
+  volatile Ctl* h = g_rt.h_ctl;
+  h[1].done = 0;
+  h[2].done = 0;
+}
+
+bool batch_saw_end()
+{
+  const volatile Ctl* h = g_rt.h_ctl;
+  return h[1].done != 0 || h[2].done != 0;
 }
 
 int timer_start()
