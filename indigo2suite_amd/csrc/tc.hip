@@ -231,7 +231,7 @@ constexpr int kTcBitWords = 4096;                // bitmap of 2^17 ranks, 16 KB
 constexpr int kTcHashSlice = kTcBitWords / 4;    // list elements per pass where ranks exceed the bitmap
 constexpr int kTcWaveSlots = kTcBitWords / kWavesPerBlock;  // hash slots of a wave there
 constexpr int kTcWaveList = kTcWaveSlots / 8;    // longest list of a wave there
-constexpr int kTcMidLow = 48, kTcMidHigh = 160;  // average degrees at which waves take lists there (tc_count_mid)
+constexpr int kTcMidLow = 42, kTcMidHigh = 160;  // average degrees at which waves take lists there (tc_count_mid)
 constexpr int kTcPad = 128;                      // elements that 16-byte reads may pass the end of a list array
 constexpr int kTcHalf = 65535;                   // ranks of x up to which the lists are read as 16 bits
 constexpr int kTcSingle = 32768;                 // ranks claimed one by one by the count; beyond, kTcClaim at once
@@ -363,9 +363,10 @@ __global__ void __launch_bounds__(kBlock) tc_orient(const int* __restrict__ nind
 // once.  Bound by the reads of the lists and the chains of their starts.
 // Erdos-Renyi, whole call, a workgroup for each x and now: n = 1 M, average
 // degree 64: 5437 -> 3379 us; n = 512 k, degree 100: 3996 -> 2622 us; n = 250
-// k, degree 50: 954 -> 666 us.  Below kTcMidLow few lists there are longer than
-// kTcShort and the launch costs more than it gives (n = 512 k, degree 40: 892 ->
-// 909 us); from kTcMidHigh a workgroup has work enough (n = 300 k, degree 200:
+// k, degree 50: 954 -> 666 us; n = 500 k, degree 42: 990 -> 951 us.  Below
+// kTcMidLow few lists there are longer than kTcShort and the launch costs more
+// than it gives (n = 1 M, degree 38: 1705 -> 1755 us, R-MAT 20 of edge factor
+// 20: 1764 -> 1827 us); from kTcMidHigh a workgroup has work enough (n = 300 k, degree 200:
 // 4069 -> 4205 us).
 __global__ void __launch_bounds__(kBlock) tc_count_mid(const int* __restrict__ nindex, const int* __restrict__ nlist,
                                                         const int* __restrict__ order, const int* __restrict__ heavy,

@@ -1,7 +1,7 @@
 """Triangle counting where ranks exceed the bitmap's 2^17: disjoint cliques,
 whose vertices all have one degree, so that any of them may be ranked there.
 The lists of a clique of k vertices have 0 to k - 1 elements: up to 32 they are
-counted row by row; longer ones by a workgroup, or, at average degrees from 48
+counted row by row; longer ones by a workgroup, or, at average degrees from 42
 to 160, one wave each up to 128.  Closed form: copies * C(k, 3)."""
 import math
 
@@ -22,7 +22,7 @@ def _cliques(k, copies, extra=0):
     return G.Graph(np.r_[nindex, np.full(extra, nindex[-1])].astype(np.int32), nlist, None, f"cliques{k}x{copies}")
 
 
-@pytest.mark.parametrize("k,copies", [(34, 4000), (35, 3745), (35, 3746), (49, 2700), (50, 2650), (66, 2100), (97, 1500),
+@pytest.mark.parametrize("k,copies", [(34, 4000), (35, 3745), (35, 3746), (42, 3200), (43, 3150), (44, 3100), (50, 2650), (66, 2100), (97, 1500),
                                       (129, 1020), (130, 1010), (160, 830), (161, 830), (162, 830), (290, 470)])
 def test_cliques(gpu, k, copies):
     with gpu.DeviceGraph(_cliques(k, copies, extra=77)) as dg:
