@@ -498,18 +498,20 @@ __global__ void __launch_bounds__(kBlock) tc_count_mid(const int* __restrict__ n
 // quarter full.  On R-MAT 20 99.9% of the probes meet the bitmap.  Between
 // two x the LDS words are all zero (both forms clear what they set).
 // R-MAT 20: 36.8 -> 1.0 ms for the count.
+// kMid: the shorter lists beyond the bitmap are tc_count_mid's.
+template <bool kMid>
 __global__ void __launch_bounds__(kBlock) tc_count_long(const int* __restrict__ nindex, const int* __restrict__ nlist,
                                                          const int* __restrict__ order,
                                                          const int* __restrict__ heavy,
                                                          const int* __restrict__ onidx, const int* __restrict__ rlist,
                                                          const unsigned short* __restrict__ hlist,
-                                                         int* __restrict__ claim, bool mid,
+                                                         int* __restrict__ claim,
                                                          unsigned long long* __restrict__ count)
 {
   __shared__ unsigned s_set[kTcBitWords];
   __shared__ int2 s_ent[kWavesPerBlock][kWave];
   __shared__ int s_claim;
-  __shared__ int4 s_row[kTcClaim];  // x, the start and length of its list
+  __shared__ int4 s_row[kMid ? kTcClaim : 1];  // x, the start and length of its list
   const int tid = threadIdx.x;
   const int w = tid / kWave;
   const int lane = lane_id();
@@ -526,8 +528,8 @@ __global__ void __launch_bounds__(kBlock) tc_count_long(const int* __restrict__ 
     const long long rank0 = (unit < kTcSingle) ? unit : kTcSingle + (unit - kTcSingle) * kTcClaim;
     const int ranks = (unit < kTcSingle) ? 1 : kTcClaim;
     if (rank0 >= total) break;
-    // ranks beyond the bitmap (uniform); most lists are tc_count_mid's there, so the unit's are looked at at once
-    const bool skim = mid && rank0 + ranks - 1 > kTcBitWords * 32;
+    // ranks beyond the bitmap (uniform): few lists are left there, so the unit's are looked at at once
+    const bool skim = kMid && rank0 + ranks - 1 > kTcBitWords * 32;
     if (skim && tid < ranks) {
       int4 row = make_int4(0, 0, 0, 0);
       if (rank0 + tid < total) {
@@ -540,18 +542,19 @@ __global__ void __launch_bounds__(kBlock) tc_count_long(const int* __restrict__ 
     if (skim) __syncthreads();
     for (int q = 0; q < ranks; q++) {
       const int rx = (int)rank0 + q;
-      int x = 0, beg = 0, len = 0;
+      if (rx >= total) break;
+      int x, beg, len;
       if (skim) {
         x = s_row[q].x;
         beg = s_row[q].y;
         len = s_row[q].z;
-      } else if (rx < total) {
+      } else {
         x = order[rx];
         beg = onidx[x];
         len = onidx[x + 1] - beg;
       }
       const bool bits = rx <= kTcBitWords * 32;
-      if (len <= ((mid && !bits) ? kTcWaveList : kTcShort)) continue;
+      if (len <= ((kMid && !bits) ? kTcWaveList : kTcShort)) continue;
       const int nb = nindex[x], ne = nindex[x + 1];
       const bool half = rx <= kTcHalf;
       const int passes = bits ? 1 : (len + kTcHashSlice - 1) / kTcHashSlice;
@@ -921,9 +924,10 @@ int style_oriented(const igx_graph* g, int, void* out, const void*, igx_run_info
                        (const unsigned short*)word_pre, (const int*)tile_off, (const int*)tile_count, onidx, olist,
                        rlist, (unsigned short*)phl);
     ktimer_begin("tc_oriented_count");
-    hipLaunchKernelGGL(tc_count_long, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, g->nlist,
+    auto count_long = mid ? tc_count_long<true> : tc_count_long<false>;
+    hipLaunchKernelGGL(count_long, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, g->nlist,
                        (const int*)order, (const int*)heavy, (const int*)onidx, (const int*)rlist,
-                       (const unsigned short*)phl, claim, mid, count);
+                       (const unsigned short*)phl, claim, count);
     if (mid) {
       hipLaunchKernelGGL(tc_count_mid, dim3(R.persist_blocks), dim3(kBlock), 0, R.stream, g->nindex, g->nlist,
                          (const int*)order, (const int*)heavy, (const int*)onidx, (const int*)rlist, count);
